@@ -5,6 +5,7 @@
 #include "tmoe_kernels.hpp"
 #include "tmoe_small.hpp"
 #include "tmoe_latent.hpp"
+#include "tmoe_latent_grouped.hpp"
 #include "tmoe_outproj_wide.hpp"
 #include "tmoe_outproj_mid.hpp"
 #include "tmoe_front_ks.hpp"
@@ -762,9 +763,32 @@ struct LatentLayout {
   size_t w, gt, zero, h, xt, dt, wt, parts, total;
   int64_t bp;
   int slices;
+  // grouped by expert (tmoe_latent_grouped.hpp; bf16 only, over the same bytes)
+  size_t meta, pair_hist, exp_hist, order, tiles, etok, ew, chunks, exp_chunks, zrow, dpp, xs, planes;
+  int64_t max_tiles, max_chunks;
+  int chunk_target;
 };
 
 constexpr int kDgBM = 128, kDgBN = 128;
+
+// Shapes of the grouped kernels: 128-wide tiles of both ranks, at most 64 experts.
+bool latent_grouped_shape(int64_t E, int64_t r3, int64_t r2) {
+  return r3 % 128 == 0 && r2 % 128 == 0 && E <= dev::kLatMaxE;
+}
+// Forward and dx / dp by pairs of experts: k <= 2, and the row tiles' products (each of
+// the E (E + 1) / 2 pairs pads half a tile on average) well below the dense form's E per
+// token. The grouped kernels reach about 0.45 of the dense ones' rate (420 against 970
+// TFLOP/s forward at 16384 tokens) but skip dx / dp's pass over H, so the line is drawn at
+// 1.3 products of the grouped form against one of the dense.
+bool latent_pairs(const LatentArgs& l) {
+  if (l.dtype != kDtypeBF16 || l.k > 2 || !latent_grouped_shape(l.E, l.r3, l.r2)) return false;
+  const int64_t keys = l.k == 2 ? l.E * (l.E + 1) / 2 : l.E;
+  return 13 * (l.B + keys * (dev::kLatBM / 2)) * l.k <= 10 * l.B * l.E;
+}
+// dG over each expert's own entries: below the dense form's B E rows.
+bool latent_dg_grouped(const LatentArgs& l) {
+  return l.dtype == kDtypeBF16 && latent_grouped_shape(l.E, l.r3, l.r2) && 5 * l.k <= 4 * l.E;
+}
 
 LatentLayout latent_layout(int64_t B, int64_t E, int64_t r3, int64_t r2, int es, bool bwd) {
   LatentLayout L{};
@@ -789,6 +813,34 @@ LatentLayout latent_layout(int64_t B, int64_t E, int64_t r3, int64_t r2, int es,
     L.parts = o; o = al256(o + (size_t)L.slices * M * r2 * 4);
   }
   L.total = o;
+  if (es == 2 && latent_grouped_shape(E, r3, r2)) {
+    // the pair order and row tiles beside what the dense forward or H use; the entries,
+    // xs (over H) and the planes for dG, which starts once H has been read
+    o = bwd ? L.xt : o;
+    const int64_t kmax = E < kMaxTopK ? E : kMaxTopK;
+    L.max_tiles = B / dev::kLatBM + E * (E + 1) / 2;
+    L.meta = o; o = al256(o + 256);
+    L.pair_hist = o; o = al256(o + (size_t)dev::kSortBlocks * (E * (E + 1) / 2) * 4);
+    L.exp_hist = o; o = al256(o + (size_t)dev::kSortBlocks * (E + 1) * 4);
+    L.order = o; o = al256(o + (size_t)B * 4);
+    L.tiles = o; o = al256(o + (size_t)L.max_tiles * 16);
+    if (bwd) {
+      // chunks of entries (chunk_target full ones, and a rest per expert): at most two
+      // work-groups a compute unit over all their tiles, one round of the chip
+      const int64_t per = (r3 / 128) * (r2 / 128);
+      L.chunk_target = (int)(512 / per > E ? 512 / per - E : 1);
+      L.max_chunks = L.chunk_target + E;
+      L.xs = L.h;   // (B k, r3) with k <= E: no larger than H
+      L.etok = o; o = al256(o + (size_t)B * kmax * 4);
+      L.ew = o; o = al256(o + (size_t)B * kmax * 4);
+      L.chunks = o; o = al256(o + (size_t)L.max_chunks * 16);
+      L.exp_chunks = o; o = al256(o + (size_t)E * 8);
+      L.zrow = o; o = al256(o + 256);
+      L.dpp = o; o = al256(o + (size_t)(r3 / 32) * B * 2 * 4);
+      L.planes = o; o = al256(o + (size_t)L.max_chunks * r3 * r2 * 4);
+    }
+    if (o > L.total) L.total = o;
+  }
   return L;
 }
 
@@ -809,6 +861,111 @@ hipError_t latent_weights(const LatentArgs& l, float* w, hipStream_t st) {
   return hipGetLastError();
 }
 
+// The sort of the tokens by pair and (exp) of the entries by expert, in two launches.
+hipError_t launch_latent_sort(const LatentArgs& l, const LatentLayout& L, bool pairs, bool exp,
+                              hipStream_t st) {
+  char* ws = static_cast<char*>(l.ws);
+  dev::LatentSort q{};
+  q.idx = l.idx;
+  q.p = l.p;
+  q.p_f32 = l.p_f32;
+  q.B = l.B;
+  q.E = (int)l.E;
+  q.k = (int)l.k;
+  // ranges of at least 256 items
+  auto blocks = [](int64_t n) {
+    return (int)(n < dev::kSortBlocks * 256 ? cdiv(n, 256) : dev::kSortBlocks);
+  };
+  q.pair_blocks = pairs ? blocks(l.B) : 0;
+  q.exp_blocks = exp ? blocks(l.B * l.k) : 0;
+  if (exp) {
+    const int64_t c = cdiv(l.B * l.k, L.chunk_target);
+    q.chunk = (int)(c < 256 ? 256 : c);
+    q.max_chunks = (int)L.max_chunks;
+    q.chunks = reinterpret_cast<int4*>(ws + L.chunks);
+    q.exp_chunks = reinterpret_cast<int2*>(ws + L.exp_chunks);
+    q.etok = reinterpret_cast<int*>(ws + L.etok);
+    q.ew = reinterpret_cast<float*>(ws + L.ew);
+  }
+  q.meta = reinterpret_cast<int*>(ws + L.meta);
+  q.tiles = reinterpret_cast<int4*>(ws + L.tiles);
+  q.order = reinterpret_cast<int*>(ws + L.order);
+  q.pair_hist = reinterpret_cast<int*>(ws + L.pair_hist);
+  q.exp_hist = reinterpret_cast<int*>(ws + L.exp_hist);
+  const dim3 grid(q.pair_blocks + q.exp_blocks), block(256);
+  hipLaunchKernelGGL(dev::k_latent_count, grid, block, 0, st, q);
+  if (hipError_t e = hipGetLastError(); e != hipSuccess) return e;
+  hipLaunchKernelGGL(dev::k_latent_sort, grid, block, 0, st, q);
+  return hipGetLastError();
+}
+
+template <int NSLOT, bool BWD>
+hipError_t launch_latent_pair(const LatentArgs& l, const LatentLayout& L, hipStream_t st) {
+  char* ws = static_cast<char*>(l.ws);
+  dev::LatentPair q{};
+  q.N = (int)(BWD ? l.r3 : l.r2);
+  const int64_t K = BWD ? l.r2 : l.r3;
+  q.A = static_cast<const char*>(BWD ? l.dout : l.x);
+  q.a_row = K * 2;
+  q.Bt = BWD ? static_cast<const char*>(l.G) : ws + L.gt;
+  q.b_row = BWD ? l.r2 * 2 : l.E * l.r3 * 2;
+  q.b_exp = BWD ? l.r3 * l.r2 * 2 : l.r3 * 2;
+  q.nkt = (int)(K / 64);
+  q.meta = reinterpret_cast<const int*>(ws + L.meta);
+  q.tiles = reinterpret_cast<const int4*>(ws + L.tiles);
+  q.order = reinterpret_cast<const int*>(ws + L.order);
+  q.idx = l.idx;
+  q.p = l.p;
+  q.p_f32 = l.p_f32 || l.dtype != kDtypeBF16;
+  q.E = (int)l.E;
+  q.out = static_cast<uint16_t*>(BWD ? l.dx : l.out);
+  q.x = static_cast<const uint16_t*>(l.x);
+  q.dpp = reinterpret_cast<float*>(ws + L.dpp);
+  q.dp_plane = l.B * l.k;
+  const int64_t ncol = q.N / (128 / NSLOT);
+  hipLaunchKernelGGL((dev::k_latent_pair<NSLOT, BWD>), dim3((unsigned)(cdiv(L.max_tiles, 8) * 8 * ncol)),
+                     dim3(256), 0, st, q);
+  return hipGetLastError();
+}
+
+// dG over each expert's entries (after the sort) and, with dp_parts, dp from the pair
+// kernel's parts.
+hipError_t latent_dg_by_expert(const LatentArgs& l, const LatentLayout& L, bool dp_parts,
+                               hipStream_t st) {
+  char* ws = static_cast<char*>(l.ws);
+  const int64_t n = l.B * l.k;
+  const int* etok = reinterpret_cast<const int*>(ws + L.etok);
+  hipLaunchKernelGGL(dev::k_latent_scale, dim3(cdiv(n * (l.r3 / 8), 256)), dim3(256), 0, st,
+                     static_cast<const uint16_t*>(l.x), etok,
+                     reinterpret_cast<const float*>(ws + L.ew), n, (int)l.r3,
+                     reinterpret_cast<uint16_t*>(ws + L.xs),
+                     reinterpret_cast<dev::u32x4*>(ws + L.zrow), 16);
+  hipError_t e = hipGetLastError();
+  if (e != hipSuccess) return e;
+  dev::LatentDg q{};
+  q.xs = ws + L.xs;
+  q.dout = static_cast<const char*>(l.dout);
+  q.etok = etok;
+  q.meta = reinterpret_cast<const int*>(ws + L.meta);
+  q.chunks = reinterpret_cast<const int4*>(ws + L.chunks);
+  q.zero = ws + L.zrow;
+  q.planes = reinterpret_cast<float*>(ws + L.planes);
+  q.r3 = (int)l.r3;
+  q.r2 = (int)l.r2;
+  const int64_t per = (l.r3 / 128) * (l.r2 / 128);
+  hipLaunchKernelGGL(dev::k_latent_dge, dim3((unsigned)(cdiv(L.max_chunks, 8) * 8 * per)), dim3(256),
+                     0, st, q);
+  if ((e = hipGetLastError()) != hipSuccess) return e;
+  const int64_t total = l.E * l.r3 * l.r2;
+  const int blk = cdiv(total, 1024), dp_blk = dp_parts ? cdiv(n, 256) : 0;
+  hipLaunchKernelGGL(dev::k_latent_finish, dim3(blk + dp_blk), dim3(256), 0, st,
+                     (const float*)q.planes, reinterpret_cast<const int2*>(ws + L.exp_chunks),
+                     l.r3 * l.r2, total, static_cast<uint16_t*>(l.dG), blk,
+                     reinterpret_cast<const float*>(ws + L.dpp), (int)(l.r3 / 32), n, l.idx,
+                     (int)l.E, l.dp, l.p_f32);
+  return hipGetLastError();
+}
+
 }  // namespace
 
 size_t latent_workspace_bytes(int64_t B, int64_t E, int64_t r3, int64_t r2, int es, bool bwd) {
@@ -821,7 +978,13 @@ hipError_t latent_forward(const LatentArgs& l, hipStream_t st) {
   const LatentLayout L = latent_layout(l.B, l.E, l.r3, l.r2, es, false);
   char* ws = static_cast<char*>(l.ws);
   float* w = reinterpret_cast<float*>(ws + L.w);
-  hipError_t e = bf && !l.p_f32 ? latent_weights<uint16_t>(l, w, st) : latent_weights<float>(l, w, st);
+  hipError_t e;
+  if (latent_pairs(l)) {
+    if ((e = launch_transpose(l.G, ws + L.gt, l.E * l.r3, l.r2, es, st)) != hipSuccess) return e;
+    if ((e = launch_latent_sort(l, L, true, false, st)) != hipSuccess) return e;
+    return l.k == 2 ? launch_latent_pair<2, false>(l, L, st) : launch_latent_pair<1, false>(l, L, st);
+  }
+  e = bf && !l.p_f32 ? latent_weights<uint16_t>(l, w, st) : latent_weights<float>(l, w, st);
   if (e != hipSuccess) return e;
   // G as (E r3, r2), transposed: the B^T operand (r2, E r3) of the Khatri-Rao GEMM
   if ((e = launch_transpose(l.G, ws + L.gt, l.E * l.r3, l.r2, es, st)) != hipSuccess) return e;
@@ -842,7 +1005,15 @@ hipError_t latent_backward(const LatentArgs& l, hipStream_t st) {
   const int64_t M = l.E * l.r3;
   char* ws = static_cast<char*>(l.ws);
   float* w = reinterpret_cast<float*>(ws + L.w);
-  hipError_t e = bf && !l.p_f32 ? latent_weights<uint16_t>(l, w, st) : latent_weights<float>(l, w, st);
+  const bool pairs = latent_pairs(l), dg_grouped = latent_dg_grouped(l);
+  hipError_t e;
+  if (pairs) {   // then dG is grouped too
+    if ((e = launch_latent_sort(l, L, true, true, st)) != hipSuccess) return e;
+    e = l.k == 2 ? launch_latent_pair<2, true>(l, L, st) : launch_latent_pair<1, true>(l, L, st);
+    if (e != hipSuccess) return e;
+    return latent_dg_by_expert(l, L, true, st);
+  }
+  e = bf && !l.p_f32 ? latent_weights<uint16_t>(l, w, st) : latent_weights<float>(l, w, st);
   if (e != hipSuccess) return e;
   // H = dout G_flat^T (B, E r3): the out-projection GEMM with U_out^T := G as (E r3, r2)
   if ((e = launch_copy_pad(nullptr, ws + L.zero, 0, M, 4, st)) != hipSuccess) return e;
@@ -871,6 +1042,10 @@ hipError_t latent_backward(const LatentArgs& l, hipStream_t st) {
                        l.idx, l.B, (int)l.E, (int)l.k, (int)l.r3, static_cast<float*>(l.dx),
                        static_cast<float*>(l.dp));
   if ((e = hipGetLastError()) != hipSuccess) return e;
+  if (dg_grouped) {
+    if ((e = launch_latent_sort(l, L, false, true, st)) != hipSuccess) return e;
+    return latent_dg_by_expert(l, L, false, st);
+  }
   // dG: token-major transposes (zero-padded to Bp tokens), then the weighted GEMM
   // in K slices and the sum of the slices
   if (bf) {

@@ -12,7 +12,9 @@
 //   dx[b, s] = sum_e w[b,e] H[b,(e,s)],  dp[b,j] = sum_s x[b,s] H[b,(idx[b,j], s)]
 //   dG_flat[(e,s), q] = sum_b w[b,e] x[b,s] dout[b,q]: a GEMM over the tokens whose
 //                   A rows are products of two token-major rows (WeightedRowLoader)
-// so every product runs on the MFMA GEMMs of the layer forward.
+// so every product runs on the MFMA GEMMs of the layer forward, dense over the E experts.
+// Taken for fp32, for ranks that are not multiples of 128 and where a token selects most of
+// the experts; otherwise tmoe_latent_grouped.hpp contracts the selected ones only.
 #pragma once
 
 #include "tmoe_kernels.hpp"

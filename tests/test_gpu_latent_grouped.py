@@ -1,0 +1,84 @@
+"""FusedLatentMoE grouped by expert (bf16, r3 and r2 multiples of 128, few of the experts
+selected per token) against the float64 formulation, at the edges of its row tiles (128
+tokens of one pair), chunks and dispatch rule, with experts nobody selects, one that
+everybody does, repeated experts and indices outside [0, E). bf16 bar as in
+test_gpu_latent.py: rel-L2 1e-2 (16-bit operands and outputs give about 2.3e-3)."""
+import numpy as np
+import pytest
+import torch
+
+from oracle import latent_np as ln
+from oracle import tucker_moe_np as onp
+
+pytestmark = pytest.mark.gpu
+
+
+def _check(pkg, dev, x, G, idx, p, dout):
+    xs, Gs, ps = (t.to(dev).requires_grad_(True) for t in (x, G, p))
+    out = pkg.FusedLatentMoE.apply(xs, Gs, idx.to(dev), ps)
+    out.backward(dout.to(dev))
+    torch.cuda.synchronize()
+    valid = (idx >= 0) & (idx < G.shape[0])
+    i0, p0 = torch.where(valid, idx, 0), torch.where(valid, p, torch.zeros_like(p))
+    dx, dG, dp = ln.backward(x, G, i0, p0, dout)
+    dp = np.where(valid.numpy(), dp, 0.0)
+    ref = {"out": ln.forward(x, G, i0, p0), "dx": dx, "dG": dG, "dp": dp}
+    got = {"out": out.detach(), "dx": xs.grad, "dG": Gs.grad, "dp": ps.grad}
+    for n, v in got.items():
+        v = v.float().cpu().numpy()
+        assert np.isfinite(v).all(), n
+        if not np.any(ref[n]):
+            assert not np.any(v), n
+            continue
+        err = onp.rel_l2(v, ref[n])
+        print(f"{n}={err:.2e}", end=" ", flush=True)
+        assert err <= 1e-2, (n, err)
+    return got
+
+
+def _inputs(B, E, k, r3, r2, seed, p32):
+    g = torch.Generator().manual_seed(seed)
+    x = torch.randn(B, r3, generator=g).bfloat16()
+    G = (torch.randn(E, r3, r2, generator=g) * r3 ** -0.5).bfloat16()
+    v, idx = torch.topk(torch.randn(B, E, generator=g), k, dim=-1)
+    p = torch.softmax(v, -1).to(torch.float32 if p32 else torch.bfloat16)
+    return x, G, idx, p, torch.randn(B, r2, generator=g).bfloat16()
+
+
+# (E, k, r3, r2, B): k = 2 pairs from B = 1110 on at E = 8 (the rule's first size and one
+# below it), k = 1 from 91 at E = 16, 4 of 16 experts (dG alone grouped), one token,
+# entries that do not fill a K tile, the widest router, one tile of r2
+@pytest.mark.parametrize("E,k,r3,r2,B", [
+    (8, 2, 256, 1024, 1109), (8, 2, 256, 1024, 1110), (8, 2, 128, 128, 2049),
+    (16, 1, 256, 512, 90), (16, 1, 256, 512, 91), (16, 1, 128, 384, 129),
+    (16, 4, 256, 256, 1), (16, 4, 256, 256, 65), (64, 2, 128, 128, 4300), (8, 6, 128, 128, 333),
+])
+@pytest.mark.parametrize("p32", [False, True], ids=["pbf16", "pf32"])
+def test_grouped(pkg, dev, E, k, r3, r2, B, p32):
+    _check(pkg, dev, *_inputs(B, E, k, r3, r2, B + E, p32))
+
+
+@pytest.mark.parametrize("kind", ["one", "repeat", "outside", "none"])
+@pytest.mark.parametrize("k", [1, 2, 4])
+def test_grouped_odd_routing(pkg, dev, kind, k):
+    B, E = 1500, 16
+    x, G, idx, p, dout = _inputs(B, E, k, 128, 256, 5, True)
+    if kind == "one":              # every token the same expert first: one group of all
+        idx = torch.where(idx == 3, idx[:, :1], idx)
+        idx[:, 0] = 3
+    elif kind == "repeat":         # a token that selects one expert k times
+        idx[::3] = idx[::3, :1]
+    elif kind == "outside":
+        idx[::4, 0] = -1
+        idx[1::4, k - 1] = E
+        idx[2::8] = 1 << 40
+    else:
+        idx[:] = -5
+    _check(pkg, dev, x, G, idx, p, dout)
+
+
+def test_grouped_is_deterministic(pkg, dev):
+    args = _inputs(3000, 8, 2, 256, 512, 9, True)
+    a, b = _check(pkg, dev, *args), _check(pkg, dev, *args)
+    for n in a:
+        assert torch.equal(a[n], b[n]), n
