@@ -9,6 +9,7 @@ from __future__ import annotations
 import os
 import shutil
 import subprocess
+import sysconfig
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 ROOT = os.path.dirname(HERE)
@@ -21,6 +22,9 @@ SOURCES = ["tmoe_kernels.hip", "tmoe_static.hip", "tmoe_api.cpp"]
 # their own so that libtmoe.so holds only the layer
 PROBE_SOURCES = ["tmoe_probe.hip"]
 PROBE_LIB = os.path.join(HERE, "libtmoe_probe.so")
+# the Python modules' host work (CPython extension over libtorch; no device code)
+NATIVE_SOURCE = "tmoe_torch.cpp"
+NATIVE_LIB = os.path.join(HERE, "_tmoe_native.so")
 ARCH = "gfx950"
 
 # Packed FP32 vector instructions are disabled for all device code: hipcc -O3
@@ -45,9 +49,22 @@ def hipcc() -> str:
     raise RuntimeError("hipcc not found: the gfx950 library cannot be built")
 
 
+def native_cmd(out: str) -> list:
+    """The host compiler's line for _tmoe_native.so, against the torch that runs it."""
+    import torch
+    inc = os.path.join(os.path.dirname(torch.__file__), "include")
+    lib = os.path.join(os.path.dirname(torch.__file__), "lib")
+    return [os.environ.get("CXX") or "g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall",
+            "-Wno-unknown-pragmas",
+            f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", "-I", INCLUDE,
+            "-isystem", inc, "-isystem", os.path.join(inc, "torch", "csrc", "api", "include"),
+            "-isystem", sysconfig.get_paths()["include"], os.path.join(CSRC, NATIVE_SOURCE),
+            "-o", out, "-L", lib, "-ltorch_python", "-ltorch_cpu", "-lc10"]
+
+
 def build(verbose: bool = False) -> str:
-    """Compiles every source (concurrently) and links libtmoe.so and
-    libtmoe_probe.so; returns libtmoe.so's path."""
+    """Compiles every source (concurrently) and links libtmoe.so, libtmoe_probe.so and
+    _tmoe_native.so; returns libtmoe.so's path."""
     objdir = os.path.join(HERE, "_build")
     os.makedirs(objdir, exist_ok=True)
     cmds, groups = [], []
@@ -60,7 +77,10 @@ def build(verbose: bool = False) -> str:
                          os.path.join(CSRC, src), "-o", obj])
             objs.append(obj)
         groups.append((lib, objs))
+    native_tmp = NATIVE_LIB + ".tmp"
+    cmds.append(native_cmd(native_tmp))
     _run_all(cmds, verbose)
+    os.replace(native_tmp, NATIVE_LIB)
     for lib, objs in groups:
         tmp = lib + ".tmp"
         cmd = [hipcc(), f"--offload-arch={ARCH}", "-shared", "-fPIC", *objs, "-o", tmp,

@@ -11,6 +11,7 @@ There is no fallback: if the library is missing, lib() raises.
 from __future__ import annotations
 
 import ctypes
+import importlib.util
 import os
 import threading
 
@@ -18,6 +19,7 @@ import torch  # noqa: F401  (loads torch's HIP runtime before libtmoe.so)
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(HERE, "libtmoe.so")
+NATIVE_PATH = os.path.join(HERE, "_tmoe_native.so")
 
 ABI_VERSION = 12
 TMOE_OK, TMOE_EINVAL, TMOE_EUNSUPPORTED, TMOE_EHIP, TMOE_ESIGNAL = 0, -1, -2, -3, -4
@@ -75,6 +77,7 @@ class TmoeError(RuntimeError):
 
 _lock = threading.Lock()
 _lib = None
+_native = None
 
 
 def lib() -> ctypes.CDLL:
@@ -152,6 +155,28 @@ def lib() -> ctypes.CDLL:
     return _lib
 
 
+def native():
+    """The CPython extension that makes a forward's allocations and C ABI call
+    (csrc/tmoe_torch.cpp), loaded once and bound to lib(); raises if it is not built."""
+    global _native
+    if _native is not None:
+        return _native
+    L = lib()
+    with _lock:
+        if _native is None:
+            if not os.path.exists(NATIVE_PATH):
+                raise RuntimeError(f"{NATIVE_PATH} is not built; build it with "
+                                   "__graft_entry__.build(). There is no fallback path.")
+            spec = importlib.util.spec_from_file_location("_tmoe_native", NATIVE_PATH)
+            mod = importlib.util.module_from_spec(spec)
+            spec.loader.exec_module(mod)
+            mod.bind(*(ctypes.cast(getattr(L, f), ctypes.c_void_p).value for f in (
+                "tmoe_workspace_bytes", "tmoe_signal_status", "tmoe_forward_epi",
+                "tmoe_forward_glu", "tmoe_rmsnorm_rows")))
+            _native = mod
+    return _native
+
+
 def check(rc: int) -> int:
     """Raises TmoeError for a negative return code."""
     if rc < 0:
@@ -188,6 +213,8 @@ class Plan:
                             f"parameter dtype {dtype}: supported are bfloat16 and float32")
         self.shape = TmoeShape(d_in, d_out, E, k, r1, r2, r3, code, eps, int(router[0]),
                                float(router[1]), float(router[2]), int(flags))
+        # the shape's fields, to compare plans by
+        self.fields = tuple(getattr(self.shape, f) for f, _ in TmoeShape._fields_)
         self.flags = int(flags)
         self.router = tuple(router)
         self.dtype = dtype
@@ -195,6 +222,7 @@ class Plan:
         self._ptr = ctypes.c_void_p()
         L = lib()
         check(L.tmoe_plan_create(ctypes.byref(self.shape), ctypes.byref(self._ptr)))
+        self.address = self._ptr.value     # for native()
         self._destroy = L.tmoe_plan_destroy
 
     @property

@@ -28,7 +28,7 @@ import torch
 import torch.nn as nn
 
 from . import _lib
-from .module import RMSNorm, TuckerMoE
+from .module import RMSNorm, TuckerMoE, launch_stream
 
 
 class LayerScale(nn.Module):
@@ -53,7 +53,7 @@ def _check_input(x: torch.Tensor, d: int, dtype: torch.dtype, who: str) -> None:
 
 
 def _same_plan(a: _lib.Plan, b: _lib.Plan) -> bool:
-    return all(getattr(a.shape, f) == getattr(b.shape, f) for f, _ in _lib.TmoeShape._fields_)
+    return a.fields == b.fields
 
 
 def glu_pair(gate: TuckerMoE, up: TuckerMoE, x: torch.Tensor) -> torch.Tensor:
@@ -64,17 +64,11 @@ def glu_pair(gate: TuckerMoE, up: TuckerMoE, x: torch.Tensor) -> torch.Tensor:
     if not _same_plan(pg, pu):
         g = gate(x)
         return up.forward_raw(x, epi=_lib.TMOE_EPI_GLU, epi_a=g, out=g)[0]
-    T = x.shape[0]
-    d_out = gate.U_out.shape[1]
     packed_g, packed_u = gate.packed(), up.packed()
-    out = torch.empty(T, d_out, dtype=x.dtype, device=x.device)
-    nws = pg.workspace_bytes(T)
-    wsg = torch.empty(max(nws, 1), dtype=torch.uint8, device=x.device)
-    wsu = torch.empty(max(nws, 1), dtype=torch.uint8, device=x.device)
-    with torch.cuda.device(x.device):
-        _lib.check(_lib.lib().tmoe_forward_glu(
-            pg.ptr, x.data_ptr(), T, packed_g.data_ptr(), packed_u.data_ptr(), out.data_ptr(),
-            wsg.data_ptr(), wsu.data_ptr(), nws, torch.cuda.current_stream(x.device).cuda_stream))
+    out = _lib.native().glu(pg.address, x, packed_g, packed_u, gate.U_out.shape[1],
+                            launch_stream(x.device))
+    if type(out) is int:
+        _lib.check(out)
     return out
 
 

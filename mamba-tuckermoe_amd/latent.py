@@ -22,6 +22,7 @@ from __future__ import annotations
 import torch
 
 from . import _lib
+from .module import device_guard, launch_stream
 
 
 def _ws(nbytes: int, dev) -> torch.Tensor:
@@ -63,11 +64,10 @@ class FusedLatentMoE(torch.autograd.Function):
         out = torch.empty(B, r2, dtype=x.dtype, device=x.device)
         nws = L.tmoe_latent_workspace_bytes(B, E, r3, r2, dt, 0)
         ws = _ws(nws, x.device)
-        with torch.cuda.device(x.device):
+        with device_guard(x.device):
             _lib.check(L.tmoe_latent_forward(
                 x.data_ptr(), G.data_ptr(), idx.data_ptr(), p.data_ptr(), B, E, k, r3, r2, dt,
-                out.data_ptr(), ws.data_ptr(), nws,
-                torch.cuda.current_stream(x.device).cuda_stream))
+                out.data_ptr(), ws.data_ptr(), nws, launch_stream(x.device)))
         ctx.save_for_backward(x, G, idx, p)
         ctx.p_dtype = top_k_probs.dtype
         return out
@@ -87,11 +87,11 @@ class FusedLatentMoE(torch.autograd.Function):
         dp = torch.empty(B, k, dtype=p.dtype, device=x.device)
         nws = L.tmoe_latent_workspace_bytes(B, E, r3, r2, dt, 1)
         ws = _ws(nws, x.device)
-        with torch.cuda.device(x.device):
+        with device_guard(x.device):
             _lib.check(L.tmoe_latent_backward(
                 x.data_ptr(), G.data_ptr(), idx.data_ptr(), p.data_ptr(), d.data_ptr(), B, E, k,
                 r3, r2, dt, dx.data_ptr(), dG.data_ptr(), dp.data_ptr(), ws.data_ptr(), nws,
-                torch.cuda.current_stream(x.device).cuda_stream))
+                launch_stream(x.device)))
         return dx, dG, None, dp.to(ctx.p_dtype)
 
 

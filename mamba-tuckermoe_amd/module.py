@@ -90,6 +90,30 @@ def _tracked(p: nn.Parameter) -> TrackedParameter:
     return p if isinstance(p, TrackedParameter) else TrackedParameter(p.detach(), p.requires_grad)
 
 
+def launch_stream(dev: torch.device) -> int:
+    """The hipStream_t of torch's current stream on `dev` (a call made for every
+    forward: torch.cuda.current_stream builds a Stream object around it, 1.8 us)."""
+    return torch._C._cuda_getCurrentRawStream(dev.index)
+
+
+class _SameDevice:
+    """Stands in for torch.cuda.device(dev) where dev is current already."""
+
+    def __enter__(self):
+        return None
+
+    def __exit__(self, *exc):
+        return False
+
+
+_SAME_DEVICE = _SameDevice()
+
+
+def device_guard(dev: torch.device):
+    """torch.cuda.device(dev), or nothing to enter when dev is the current device."""
+    return _SAME_DEVICE if torch.cuda.current_device() == dev.index else torch.cuda.device(dev)
+
+
 # state_dict keys of TuckerMoE's parameters, in the order of TuckerMoE._params()
 PARAM_KEYS = ("router.weight", "U_in", "inner_norm.weight", "U_expert", "core", "U_out", "bias")
 
@@ -108,19 +132,19 @@ class RMSNorm(nn.Module):
         self.eps = eps
 
     def forward(self, x: torch.Tensor, out: Optional[torch.Tensor] = None) -> torch.Tensor:
-        d = self.weight.shape[0]
-        if x.device.type != "cuda":
+        weight = self.weight
+        d = weight.shape[0]
+        dev = x.device
+        if dev.type != "cuda":
             raise RuntimeError(f"RMSNorm runs on HIP devices only; input is on {x.device}")
-        if x.shape[-1] != d or x.dtype != self.weight.dtype:
+        if x.shape[-1] != d or x.dtype != weight.dtype:
             raise RuntimeError(f"RMSNorm: input (..., {x.shape[-1]}) {x.dtype}, weight ({d}) "
-                               f"{self.weight.dtype}")
+                               f"{weight.dtype}")
         dt = _lib.dtype_code(x.dtype)
         X = x.reshape(-1, d).contiguous()
-        y = torch.empty_like(X) if out is None else out
-        with torch.cuda.device(X.device):
-            _lib.check(_lib.lib().tmoe_rmsnorm_rows(
-                X.data_ptr(), X.shape[0], d, self.weight.data_ptr(), float(self.eps), dt,
-                y.data_ptr(), torch.cuda.current_stream(X.device).cuda_stream))
+        y = _lib.native().rmsnorm(X, weight, float(self.eps), dt, out, launch_stream(dev))
+        if type(y) is int:
+            _lib.check(y)
         return y.reshape(x.shape)
 
 
@@ -150,6 +174,15 @@ class TuckerMoE(nn.Module):
 
     # -- packed-weight cache -------------------------------------------------
     def _params(self):
+        # straight from the modules' tables: nn.Module's attribute lookup takes 0.3 us a
+        # parameter, in every forward. A parametrised or replaced one is not there.
+        own, sub = self._parameters, self._modules
+        try:
+            return (sub["router"]._parameters["weight"], own["U_in"],
+                    sub["inner_norm"]._parameters["weight"], own["U_expert"], own["core"],
+                    own["U_out"], own["bias"])
+        except (KeyError, AttributeError):
+            pass
         return (self.router.weight, self.U_in, self.inner_norm.weight, self.U_expert,
                 self.core, self.U_out, self.bias)
 
@@ -159,8 +192,10 @@ class TuckerMoE(nn.Module):
                 f["U_out_scale"])
 
     def _key(self):
-        ts = self._params() + (self._fp8_tensors() if self._fp8 is not None else ())
-        return tuple((p.data_ptr(), p._version, tracked_gen(p), p.dtype, p.device) for p in ts)
+        ts = self._params()
+        if self._fp8 is not None:
+            ts = ts + self._fp8_tensors()
+        return _lib.native().param_key(ts)
 
     def _load_from_state_dict(self, *args, **kwargs):
         # load_state_dict copies in place (moving the version counters); forget the
@@ -169,10 +204,11 @@ class TuckerMoE(nn.Module):
         return super()._load_from_state_dict(*args, **kwargs)
 
     def plan(self) -> _lib.Plan:
-        dtype = self.U_in.dtype
+        dtype = self._params()[1].dtype
         fp8 = self._fp8 is not None
-        if (self._plan is None or self._plan.dtype != dtype or self._plan.fp8_weights != fp8
-                or self._plan.router != self._router or self._plan.flags != self._plan_flags):
+        p = self._plan
+        if (p is None or p.dtype != dtype or p.fp8_weights != fp8 or p.router != self._router
+                or p.flags != self._plan_flags):
             d_in, r3 = self.U_in.shape
             r2, d_out = self.U_out.shape
             E, r1 = self.U_expert.shape
@@ -379,35 +415,39 @@ class TuckerMoE(nn.Module):
         (out = epi_a + epi_b * y), y = this layer's output; epi_a (..., d_out) and
         epi_b (d_out) in the parameter dtype. `out` (T, d_out), which may be
         epi_a itself, receives the result."""
-        *batch, d_in = x.shape
-        dtype = self.U_in.dtype
-        if x.device.type != "cuda":
+        batch = None
+        if x.dim() == 2:
+            d_in = x.shape[1]
+        else:
+            *batch, d_in = x.shape
+        params = self._params()
+        U_in, U_expert, U_out = params[1], params[3], params[5]
+        dtype, dev = U_in.dtype, x.device
+        if dev.type != "cuda":
             raise RuntimeError(f"TuckerMoE runs on HIP devices only; input is on {x.device}")
         if x.dtype != dtype:
             raise RuntimeError(f"TuckerMoE: input dtype {x.dtype} != parameter dtype {dtype}")
-        if d_in != self.U_in.shape[0]:
-            raise RuntimeError(f"TuckerMoE: input feature size {d_in} != d_in {self.U_in.shape[0]}")
-        if torch.is_grad_enabled() and (x.requires_grad or self.U_in.requires_grad) \
-                and not self._warned_grad:
+        if d_in != U_in.shape[0]:
+            raise RuntimeError(f"TuckerMoE: input feature size {d_in} != d_in {U_in.shape[0]}")
+        if not self._warned_grad and torch.is_grad_enabled() and (x.requires_grad
+                                                                  or U_in.requires_grad):
             warnings.warn("TuckerMoE (gfx950) is forward-only; its output carries no gradient")
             self._warned_grad = True
-        X = x.reshape(-1, d_in).contiguous()
-        T = X.shape[0]
-        d_out = self.U_out.shape[1]
-        E = self.U_expert.shape[0]
+        X = x if batch is None and x.is_contiguous() else x.reshape(-1, d_in).contiguous()
+        d_out = U_out.shape[1]
         plan = self.plan()
         # an earlier forward's kernel that lost an in-launch signal (host memory the
         # kernels write: no synchronisation) is reported before any new work
-        plan.signal_status(clear=True)
+        native = _lib.native()
+        _lib.check(native.signal(plan.address))
         packed = self.packed()
-        dev = X.device
-        if out is None:
-            out = torch.empty(T, d_out, dtype=dtype, device=dev)
-        elif (out.shape != (T, d_out) or out.dtype != dtype or out.device != dev
-              or not out.is_contiguous()):
-            raise RuntimeError(f"TuckerMoE: out must be a contiguous ({T}, {d_out}) {dtype} tensor")
+        if out is not None and (out.shape != (X.shape[0], d_out) or out.dtype != dtype
+                                or out.device != dev or not out.is_contiguous()):
+            raise RuntimeError(f"TuckerMoE: out must be a contiguous ({X.shape[0]}, {d_out}) "
+                               f"{dtype} tensor")
         ea = eb = None
         if epi != _lib.TMOE_EPI_NONE:
+            T = X.shape[0]
             ea = epi_a.reshape(T, d_out) if epi_a is not None else None
             if ea is None or ea.dtype != dtype or ea.device != dev or not ea.is_contiguous():
                 raise RuntimeError(f"TuckerMoE: epi_a must be a contiguous ({T}, {d_out}) "
@@ -418,21 +458,13 @@ class TuckerMoE(nn.Module):
                     or not eb.is_contiguous()):
                 raise RuntimeError(f"TuckerMoE: epi_b must be a contiguous ({d_out},) {dtype} "
                                    f"tensor on {dev}")
-        idx = torch.empty(T, self.top_k, dtype=torch.int32, device=dev) if routing else None
-        w = torch.empty(T, self.top_k, dtype=torch.float32, device=dev) if routing else None
-        lg = torch.empty(T, E, dtype=torch.float32, device=dev) if logits else None
-        ws_bytes = plan.workspace_bytes(T)
-        ws = torch.empty(max(ws_bytes, 1), dtype=torch.uint8, device=dev)
-        with torch.cuda.device(dev):
-            stream = torch.cuda.current_stream(dev).cuda_stream
-            _lib.check(_lib.lib().tmoe_forward_epi(
-                plan.ptr, X.data_ptr(), T, packed.data_ptr(), out.data_ptr(),
-                idx.data_ptr() if idx is not None else None,
-                w.data_ptr() if w is not None else None,
-                lg.data_ptr() if lg is not None else None,
-                ws.data_ptr(), ws_bytes, epi, ea.data_ptr() if ea is not None else None,
-                eb.data_ptr() if eb is not None else None, stream))
-        out = out.reshape(*batch, d_out)
+        got = native.forward(plan.address, X, packed, out, d_out, self.top_k if routing else 0,
+                             U_expert.shape[0] if logits else 0, epi, ea, eb, launch_stream(dev))
+        if type(got) is int:
+            _lib.check(got)
+        out, idx, w, lg = got
+        if batch is not None:
+            out = out.reshape(*batch, d_out)
         return out, (idx.long() if idx is not None else None), w, lg
 
 
