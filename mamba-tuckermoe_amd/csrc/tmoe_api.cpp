@@ -128,8 +128,11 @@ struct Layout {
   int split, fsplit;
 };
 
-Layout workspace_layout(const tmoe_plan* p, int64_t T) {
+// lean: without the fp32 plans' K slices (their planes), for a caller whose scratch
+// does not hold them.
+Layout workspace_layout(const tmoe_plan* p, int64_t T, bool lean = false) {
   Layout L{};
+  lean = lean && p->kdtype == TMOE_F32;
   size_t o = 0;
   // k_core_pp reads c and stores mid in whole 256-token tiles; a folded plan's
   // out-projection reads its A operand (c (x) z in mid) in whole 256-row tiles
@@ -146,7 +149,7 @@ Layout workspace_layout(const tmoe_plan* p, int64_t T) {
       p->fold && T > tmoe::kSmallT && p->rk * p->s.r3 > p->s.r2 ? p->rk * p->s.r3 : p->s.r2;
   L.mid = o; o = align256(o + (size_t)tile_rows * mid_cols * p->es);
   L.raw = o;
-  L.fsplit = tmoe::front_split(T, p->s.d_in, p->E_pad, p->kdtype == TMOE_BF16);
+  L.fsplit = lean ? 1 : tmoe::front_split(T, p->s.d_in, p->E_pad, p->es);
   if (T <= tmoe::kSmallT || L.fsplit > 1) {
     int64_t raw_floats = L.fsplit * T * tmoe::raw_stride(p->s.r3, p->s.E);
     // the one-launch decode's scratch (z columns, sums of squares, c)
@@ -161,6 +164,12 @@ Layout workspace_layout(const tmoe_plan* p, int64_t T) {
     L.split = tmoe::core_p_split(T, p->rk, p->s.r2);
     L.mpart = o;
     o = align256(o + (size_t)L.split * tile_rows * p->s.r2 * sizeof(float));
+  } else if (p->kdtype == TMOE_F32 && T > tmoe::kSmallT && !lean) {
+    L.split = tmoe::core_f32_split(T, p->rk, p->s.r3, p->s.r2);
+    if (L.split > 1) {
+      L.mpart = o;
+      o = align256(o + (size_t)L.split * T * p->s.r2 * sizeof(float));
+    }
   }
   // error word and flags of the kernels that signal between work-groups
   L.sync = o;
@@ -560,7 +569,7 @@ namespace {
 int forward_impl(const tmoe_plan* p, const void* x, int64_t T, const void* packed, void* out,
                  int32_t* topk_idx, float* topk_w, float* logits, void* workspace,
                  size_t workspace_bytes, int epi_mode, const void* epi_a, const void* epi_b,
-                 void* stream, bool prof_ok) {
+                 void* stream, bool prof_ok, bool lean = false) {
   if (!p) return fail(TMOE_EINVAL, "tmoe_forward: null plan");
   if (epi_mode != TMOE_EPI_NONE && epi_mode != TMOE_EPI_GLU && epi_mode != TMOE_EPI_RESIDUAL_SCALE)
     return fail(TMOE_EINVAL, "tmoe_forward_epi: epi_mode %d is not a TMOE_EPI_* value", epi_mode);
@@ -576,7 +585,7 @@ int forward_impl(const tmoe_plan* p, const void* x, int64_t T, const void* packe
     return fail(TMOE_EINVAL, "tmoe_forward: null x/packed/out/workspace");
   if (!aligned16(x) || !aligned16(packed) || !aligned16(workspace) || !aligned16(out))
     return fail(TMOE_EINVAL, "tmoe_forward: x/packed/out/workspace must be 16-byte aligned");
-  const Layout L = workspace_layout(p, T);
+  const Layout L = workspace_layout(p, T, lean);
   if (workspace_bytes < L.total)
     return fail(TMOE_EINVAL, "tmoe_forward: workspace of %zu bytes, %zu needed for T=%lld",
                 workspace_bytes, L.total, (long long)T);
@@ -666,7 +675,9 @@ int tmoe_forward_static(const tmoe_plan* p, const void* x, int64_t T, const void
     return fail(TMOE_EUNSUPPORTED, "tmoe_forward_static: T=%lld too large", (long long)T);
   if (T == 0) return TMOE_OK;
   // every check that needs no GPU comes before the scratch lookup
-  const size_t need = workspace_layout(p, T).total;
+  size_t need = workspace_layout(p, T).total;
+  const bool lean = need > tmoe::kStaticScratchBytes;
+  if (lean) need = workspace_layout(p, T, true).total;
   if (need > tmoe::kStaticScratchBytes)
     return fail(TMOE_EUNSUPPORTED,
                 "tmoe_forward_static: T=%lld needs %zu bytes of scratch, more than the static "
@@ -679,7 +690,8 @@ int tmoe_forward_static(const tmoe_plan* p, const void* x, int64_t T, const void
   if (hipError_t e = tmoe::static_scratch(static_cast<hipStream_t>(stream), &ws); e != hipSuccess)
     return hip_fail(e, "tmoe_forward_static: static scratch address");
   return forward_impl(p, x, T, packed, out, topk_idx, topk_w, logits, ws,
-                      tmoe::kStaticScratchBytes, TMOE_EPI_NONE, nullptr, nullptr, stream, false);
+                      tmoe::kStaticScratchBytes, TMOE_EPI_NONE, nullptr, nullptr, stream, false,
+                      lean);
 }
 
 int tmoe_forward_glu(const tmoe_plan* p, const void* x, int64_t T, const void* packed_gate,

@@ -150,14 +150,20 @@ constexpr int64_t kFrontMinKTiles = 16;
 constexpr int64_t kFrontSliceKTiles = 3;
 constexpr int kMaxFrontPlanes = 8;
 constexpr int64_t kFrontXcds = 8, kFrontGroupsPerXcd = 32;
-inline int front_split(int64_t T, int64_t d_in, int64_t E_pad, bool bf16) {
+// Tokens of a K-sliced front tile: 64 in bf16; 32 in fp32, whose MFMAs bound the slice
+// (a K tile of 32 takes 64 rows 2.2 us), so that twice the work-groups share it. d_in
+// 1536 at T = 1021: 119 us unsliced (16 work-groups of 64 tokens), 25.5 sliced over 64-token
+// tiles, 19.8 over 32.
+constexpr int64_t front_slice_rows(int64_t es) { return es == 2 ? 64 : 32; }
+inline int front_split(int64_t T, int64_t d_in, int64_t E_pad, int64_t es) {
   // E_pad = 256 measured slower sliced (C4: front 44.6 us against 34.8 us for the
   // split z / router front plus 7.7 us of k_expand_cz)
-  if (!bf16 || T <= 256 || E_pad > 128) return 1;
-  const int64_t tiles = (T + 63) / 64, nkt = d_in * 2 / 128;
-  // measured at d_in = 1536: slices win up to 64 tiles (T = 4096); at 128 tiles
+  if (T <= 256 || E_pad > 128) return 1;
+  const int64_t rows = front_slice_rows(es);
+  const int64_t tiles = (T + rows - 1) / rows, nkt = d_in * es / 128;
+  // measured at d_in = 1536, bf16: slices win up to T = 4096 (64 tiles); at 128 tiles
   // the 32-token front is faster
-  if (4 * tiles > 256 || nkt < kFrontMinKTiles) return 1;
+  if (T > 4096 || nkt < kFrontMinKTiles) return 1;
   int64_t s = kFrontGroupsPerXcd / ((tiles + kFrontXcds - 1) / kFrontXcds);
   if (s > nkt / kFrontSliceKTiles) s = nkt / kFrontSliceKTiles;
   if (s > kMaxFrontPlanes) s = kMaxFrontPlanes;
@@ -181,6 +187,17 @@ inline int core_p_split(int64_t T, int64_t r1, int64_t r2) {
   for (int64_t s = 1; s < G; ++s)
     if (G % s == 0 && n * s >= kCoreUnits) return (int)s;
   return (int)G;
+}
+// K slices of the fp32 core (k_core, 64 x 64 tiles): about two work-groups a compute
+// unit, slices of at least 8 K tiles of 32, at most kMaxCoreSlices.
+constexpr int64_t kMaxCoreSlices = 8;
+inline int64_t core_f32_tiles(int64_t T, int64_t r2) { return (T + 63) / 64 * ((r2 + 63) / 64); }
+inline int core_f32_split(int64_t T, int64_t r1, int64_t r3, int64_t r2) {
+  int64_t s = 2 * kCoreUnits / core_f32_tiles(T, r2);
+  const int64_t nkt = r1 * r3 * 4 / 128;
+  if (s > nkt / 8) s = nkt / 8;
+  if (s > kMaxCoreSlices) s = kMaxCoreSlices;
+  return s > 1 ? (int)s : 1;
 }
 inline bool core_p_supported(int64_t r1, int64_t r2, bool bf16, bool fp8w) {
   if (!bf16) return false;

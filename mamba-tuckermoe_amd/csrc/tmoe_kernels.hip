@@ -32,7 +32,10 @@ inline unsigned cdiv(int64_t a, int64_t b) { return (unsigned)((a + b - 1) / b);
 struct CoreCfgBF16 { static constexpr int BM = 256, BN = 256, WM = 2, WN = 4, P = 1; };
 struct OutCfgBF16 { static constexpr int BM = 256, BN = 192, WM = 4, WN = 2, P = 2; };
 struct CoreCfgF32 { static constexpr int BM = 128, BN = 128, WM = 2, WN = 2, P = 2; };
+struct CoreCfgF32S { static constexpr int BM = 64, BN = 64, WM = 2, WN = 2, P = 2; };
 struct OutCfgF32 { static constexpr int BM = 128, BN = 128, WM = 2, WN = 2, P = 2; };
+struct OutCfgF32XS { static constexpr int BM = 64, BN = 64, WM = 2, WN = 2, P = 2; };
+struct OutCfgF32S { static constexpr int BM = 64, BN = 128, WM = 2, WN = 2, P = 2; };
 
 // Front tiles: kFrontBM tokens in kFrontWM row groups; with the widest router
 // (E > 128) one group of 32 tokens, whose smaller LDS footprint measured faster,
@@ -44,25 +47,27 @@ int cu_count();
 template <class Elt, int R3, int NR>
 hipError_t launch_front_nr(const FwdArgs& a, hipStream_t st) {
   constexpr int NW = R3 / 32 < 4 ? R3 / 32 : 4;
-  if constexpr (std::is_same<Elt, EltBF16>::value) {
+  if constexpr (NR < 8) {
     if (a.front_split > 1) {
-      // K slices of 64-token tiles (k_front_part), then the per-token epilogue over
-      // their planes: in one launch (k_front_sliced, a fresh epoch for its signals)
-      // or two
-      constexpr int kStageBytes = (kFrontBM + R3 + 32 * NR) * 128;
+      // K slices of 64-token (fp32: 32-token) tiles (k_front_part), then the per-token
+      // epilogue over their planes: in one launch (k_front_sliced, a fresh epoch for
+      // its signals) or two
+      constexpr int BMS = (int)front_slice_rows(sizeof(typename Elt::T)), WMS = BMS / 32;
+      static_assert(kFrontBM == 64 && kFrontWM == 2, "bf16: the plain front's tile");
+      constexpr int kStageBytes = (BMS + R3 + 32 * NR) * 128;
       constexpr int NS = 3 * kStageBytes <= 160 * 1024 ? 3 : 2;
       if (a.front_one) {
         FwdArgs b = a;
         b.epoch = next_epoch();
-        hipLaunchKernelGGL(
-            (dev::k_front_sliced<Elt, R3, NR, kFrontPFA, kFrontBM, NS, kFrontWM>),
-            dim3(dev::sliced::kGrid), dim3(64 * NW * kFrontWM), 0, st, b, b.raw, b.front_split);
+        hipLaunchKernelGGL((dev::k_front_sliced<Elt, R3, NR, kFrontPFA, BMS, NS, WMS>),
+                           dim3(dev::sliced::kGrid), dim3(64 * NW * WMS), 0, st, b, b.raw,
+                           b.front_split);
         return hipGetLastError();
       }
       const int64_t stride = a.T * raw_stride(a.r3, a.E);
-      hipLaunchKernelGGL((dev::k_front_part<Elt, R3, NR, kFrontPFA, kFrontBM, NS, kFrontWM>),
-                         dim3(cdiv(a.T, kFrontBM), a.front_split), dim3(64 * NW * kFrontWM), 0,
-                         st, a, a.raw, a.front_split);
+      hipLaunchKernelGGL((dev::k_front_part<Elt, R3, NR, kFrontPFA, BMS, NS, WMS>),
+                         dim3(cdiv(a.T, BMS), a.front_split), dim3(64 * NW * WMS), 0, st, a, a.raw,
+                         a.front_split);
       if (hipError_t e = hipGetLastError(); e != hipSuccess) return e;
       hipLaunchKernelGGL((dev::k_front_epi<Elt, R3 / 64, kMaxFrontPlanes, 2>),
                          dim3(cdiv(a.T, 4)), dim3(256), (size_t)(a.E * a.r1) * sizeof(float), st,
@@ -177,8 +182,16 @@ hipError_t launch_core_pp_r(const FwdArgs& a, hipStream_t st);
 
 template <class Elt, class C>
 hipError_t launch_core_t(const FwdArgs& a, hipStream_t st) {
-  const dim3 grid(cdiv(a.T, C::BM) * cdiv(a.r2, C::BN)), block(64 * C::WM * C::WN);
+  // K slices (fp32: core_f32_split) leave one plane each in mpart
+  const int S = a.dtype != kDtypeBF16 && a.mpart ? a.core_split : 1;
+  const dim3 grid(cdiv(a.T, C::BM) * cdiv(a.r2, C::BN), S), block(64 * C::WM * C::WN);
   hipLaunchKernelGGL((dev::k_core<Elt, C::BM, C::BN, C::WM, C::WN, C::P>), grid, block, 0, st, a);
+  if (S > 1) {
+    if (hipError_t e = hipGetLastError(); e != hipSuccess) return e;
+    const int64_t n = a.T * a.r2;
+    hipLaunchKernelGGL(dev::k_sum_planes_f4, dim3(cdiv(n, 1024)), dim3(256), 0, st, a.mpart, S, n,
+                       static_cast<float*>(a.mid));
+  }
   return hipGetLastError();
 }
 
@@ -485,8 +498,12 @@ hipError_t launch_core(const FwdArgs& a, hipStream_t st) {
         return hipErrorInvalidValue;
     }
   }
-  return a.dtype == kDtypeBF16 ? launch_core_t<EltBF16, CoreCfgBF16>(a, st)
-                               : launch_core_t<EltF32, CoreCfgF32>(a, st);
+  if (a.dtype == kDtypeBF16) return launch_core_t<EltBF16, CoreCfgBF16>(a, st);
+  // fp32, 64 x 64 tiles in core_f32_split slices while 128 x 128 ones would number at most
+  // one a compute unit (1021 x 512, K 2048: 25 + 5 us of adding the slices against 140 for
+  // 32 work-groups of 128 x 128)
+  if (core_f32_tiles(a.T, a.r2) > 4 * cu_count()) return launch_core_t<EltF32, CoreCfgF32>(a, st);
+  return launch_core_t<EltF32, CoreCfgF32S>(a, st);
 }
 
 hipError_t launch_pack_frag(const void* wfront, void* dst, int64_t rows, int64_t d_in,
@@ -587,10 +604,10 @@ bool front_fuses_cz(const FwdArgs& a, hipStream_t st) {
 }
 
 bool front_sliced_ok(const FwdArgs& a, hipStream_t st) {
-  if (a.dtype != kDtypeBF16 || a.front_split <= 1 || !a.sync || a.E_pad > 128) return false;
+  if (a.front_split <= 1 || !a.sync || a.E_pad > 128) return false;
   // every (XCD, slot) pair of the grid holds at most one slice
-  const int64_t per_xcd = ((int64_t)cdiv(a.T, kFrontBM) + dev::sliced::kXcds - 1) /
-                          dev::sliced::kXcds;
+  const int64_t rows = front_slice_rows(a.dtype == kDtypeBF16 ? 2 : 4);
+  const int64_t per_xcd = ((int64_t)cdiv(a.T, rows) + dev::sliced::kXcds - 1) / dev::sliced::kXcds;
   return per_xcd * a.front_split <= dev::sliced::kGroupsPerXcd &&
          cu_count() == dev::sliced::kGrid && !stream_capturing(st);
 }
@@ -663,8 +680,18 @@ hipError_t launch_eye(float* dst, int64_t n, hipStream_t st) {
 }
 
 hipError_t launch_outproj(const FwdArgs& a, hipStream_t st) {
-  return a.dtype == kDtypeBF16 ? launch_outproj_bf16(a, st)
-                               : launch_outproj_t<EltF32, OutCfgF32>(a, st);
+  if (a.dtype == kDtypeBF16) return launch_outproj_bf16(a, st);
+  // fp32: the tile whose rounds of the compute units take least, in 64 x 64 units (the
+  // fp32 MFMAs bound every tile alike; 1021 x 6144 x 512: 64 x 128 tiles, three rounds,
+  // 60.5 us against 73.5 for 128 x 128, one and a half; T = 257, d_out 2304, K 1024: the
+  // layer 64 us with 64 x 64 tiles, 81 with 64 x 128)
+  const int64_t ncu = cu_count(), m64 = cdiv(a.T, 64);
+  const int64_t r1 = cdiv(m64 * cdiv(a.d_out, 64), ncu);
+  const int64_t r2 = 2 * (int64_t)cdiv(m64 * cdiv(a.d_out, 128), ncu);
+  const int64_t r4 = 4 * (int64_t)cdiv((int64_t)cdiv(a.T, 128) * cdiv(a.d_out, 128), ncu);
+  if (r1 < r2 && r1 < r4) return launch_outproj_t<EltF32, OutCfgF32XS>(a, st);
+  return r2 < r4 ? launch_outproj_t<EltF32, OutCfgF32S>(a, st)
+                 : launch_outproj_t<EltF32, OutCfgF32>(a, st);
 }
 
 hipError_t launch_transpose(const void* src, void* dst, int64_t rows, int64_t cols, int es,
@@ -995,7 +1022,7 @@ hipError_t latent_forward(const LatentArgs& l, hipStream_t st) {
   a.c = w;
   a.coreT = ws + L.gt;
   a.mid = l.out;
-  return bf ? launch_core_t<EltBF16, CoreCfgBF16>(a, st) : launch_core_t<EltF32, CoreCfgF32>(a, st);
+  return launch_core(a, st);
 }
 
 hipError_t latent_backward(const LatentArgs& l, hipStream_t st) {

@@ -129,10 +129,11 @@ struct KhatriRaoLoader {
   const float* c;           // first row of the tile, (., r1)
   int r1, r3;
   int rows_valid;
+  int kt0;                  // the K tile that the loop calls 0 (K slices)
   __device__ __forceinline__ Raw fetch(int row, int ch, int kt) const {
     constexpr int kTileK = kTileKBytes / (int)sizeof(typename Elt::T);
     const int r = row < rows_valid ? row : rows_valid - 1;
-    const int k0 = kt * kTileK;
+    const int k0 = (kt0 + kt) * kTileK;
     const int rr = k0 / r3;
     const int s0 = k0 - rr * r3;
     Raw o;
@@ -1696,17 +1697,23 @@ __global__ __launch_bounds__(64 * WM * WN) void k_core(FwdArgs a) {
   const int rows_valid = (int)(a.T - m0 < BM ? a.T - m0 : BM);
   const int64_t K = a.r1 * a.r3;
   const int64_t b_row_bytes = K * (int64_t)sizeof(T);
+  // K slice sl of S = gridDim.y (fp32 plans, whose scales CoreRescale does not need): its
+  // plane of mpart takes the place of mid
+  const int S = (int)gridDim.y, sl = (int)blockIdx.y;
+  const int nkt = (int)(b_row_bytes / kTileKBytes);
+  const int kt0 = sl * nkt / S, kt1 = (sl + 1) * nkt / S;
   KhatriRaoLoader<Elt> al{reinterpret_cast<const char*>(a.z) + m0 * a.r3 * (int64_t)sizeof(T),
-                          a.c + m0 * a.r1, (int)a.r1, (int)a.r3, rows_valid};
-  RowLoader bl{reinterpret_cast<const char*>(a.coreT) + n0 * b_row_bytes, b_row_bytes,
-               (int)(a.r2 - n0)};
+                          a.c + m0 * a.r1, (int)a.r1, (int)a.r3, rows_valid, kt0};
+  RowLoader bl{reinterpret_cast<const char*>(a.coreT) + n0 * b_row_bytes +
+                   (int64_t)kt0 * kTileKBytes,
+               b_row_bytes, (int)(a.r2 - n0)};
   f32x16 acc[TL::FM][TL::FN];
   const int wn = (threadIdx.x >> 6) % WN, lane = threadIdx.x & 63;
   const int col0 = wn * TL::kWaveN + (lane & 31);   // column of block j: col0 + 32 j
   CoreRescale<TL::FM, TL::FN> rs;
   rs.init(a.core_scale, (int)(a.r3 * (int64_t)sizeof(T) / kTileKBytes), (int)a.r1, (int)a.r2,
           (int)n0 + col0);
-  gemm_mainloop<TL, Elt>(acc, al, bl, (int)(b_row_bytes / kTileKBytes), smem, rs);
+  gemm_mainloop<TL, Elt>(acc, al, bl, kt1 - kt0, smem, rs);
 
   char* stage = reinterpret_cast<char*>(smem);
   float zero[TL::FN], last[TL::FN];
@@ -1719,8 +1726,21 @@ __global__ __launch_bounds__(64 * WM * WN) void k_core(FwdArgs a) {
   }
   stage_tile<TL, T>(acc, stage, zero, last);
   __syncthreads();
-  flush_tile<TL, T>(stage, reinterpret_cast<T*>(a.mid) + m0 * a.r2 + n0, a.r2, rows_valid,
-                    (int)(a.r2 - n0));
+  T* dst = S > 1 ? reinterpret_cast<T*>(a.mpart) + sl * a.T * a.r2 : reinterpret_cast<T*>(a.mid);
+  flush_tile<TL, T>(stage, dst + m0 * a.r2 + n0, a.r2, rows_valid, (int)(a.r2 - n0));
+}
+
+// dst (n, a multiple of 4) = the sum of S planes of n floats, in plane order.
+__global__ __launch_bounds__(256) void k_sum_planes_f4(const float* __restrict__ parts, int S,
+                                                       int64_t n, float* __restrict__ dst) {
+  const int64_t i = ((int64_t)blockIdx.x * 256 + threadIdx.x) * 4;
+  if (i >= n) return;
+  float4 v = *reinterpret_cast<const float4*>(parts + i);
+  for (int p = 1; p < S; ++p) {
+    const float4 u = *reinterpret_cast<const float4*>(parts + p * n + i);
+    v.x += u.x; v.y += u.y; v.z += u.z; v.w += u.w;
+  }
+  *reinterpret_cast<float4*>(dst + i) = v;
 }
 
 // ---- k_core_pp: mid = sum_r c_r (z P_r), persistent ping-pong  (model.py:87-98)
