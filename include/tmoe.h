@@ -250,7 +250,7 @@ int tmoe_forward_static(const tmoe_plan* plan, const void* x, int64_t T, const v
  * No counterpart in the reference; for measurement tools, which attribute time
  * per kernel. Returns one of TMOE_PATH_* (0 for T == 0) or a negative error. */
 #define TMOE_PATH_SMALL  1  /* T <= 256: skinny kernels, two or three launches        */
-#define TMOE_PATH_DECODE 2  /* T <= 64, bf16, folded: the whole layer in one launch   */
+#define TMOE_PATH_DECODE 2  /* T <= 64, bf16: the whole layer in one folded launch      */
 #define TMOE_PATH_LARGE  3  /* front, (core or c (x) z), out-projection launches      */
 #define TMOE_PATH_FUSED  4  /* large T, folded: the whole layer in one launch         */
 #define TMOE_PATH_LARGE_KR 5 /* large T, folded, E > 128: front (stores z and c) and an

@@ -39,6 +39,9 @@ struct tmoe_plan {
   int64_t rk;
   // folded form (large T): W^T (d_out, rk*r3) at off_fold, one GEMM of c (x) z against W
   bool fold;
+  // W^T also packed for a plan that is not folded, for its decode-size batches
+  // (tmoe::decode_fold_ok)
+  bool decode_fold;
   size_t off_fold;
   // status block (tmoe::kStatusWords words of pinned host memory mapped for the
   // device, set by kernels; null on a machine without a GPU): host and device address
@@ -259,15 +262,33 @@ tmoe::FwdArgs folded_args(const tmoe_plan* p, const tmoe::FwdArgs& a, const void
   return f;
 }
 
+// The arguments of the folded one-launch forward of a plan that is not folded
+// otherwise (decode_fold); the caller checks T and small_decode_ok.
+tmoe::FwdArgs decode_fold_args(const tmoe_plan* p, const tmoe::FwdArgs& a, const void* packed) {
+  tmoe::FwdArgs f = a;
+  f.r2 = p->rk * p->s.r3;
+  f.uoutT = static_cast<const char*>(packed) + p->off_fold;
+  f.out_scale = nullptr;   // in W^T
+  return f;
+}
+
 hipError_t launch_nothing(const tmoe::FwdArgs&, hipStream_t) { return hipSuccess; }
 
 using Launch = hipError_t (*)(const tmoe::FwdArgs&, hipStream_t);
 
-// The small-T stages (front, core, out-projection) of a forward with args a: the
+// The small-T stages (front, core, out-projection) of a forward with args a (which become
+// the folded ones where a decode-size batch of an unfolded plan runs folded): the
 // front epilogue runs inside the core (or, folded, the out-projection) when that
 // kernel's LDS holds it, else as its own kernel after the front's GEMM.
-void small_stages(const tmoe::FwdArgs& a, bool fold, hipStream_t stream, Launch (&st)[kStages]) {
-  if (fold && tmoe::small_decode_ok(a, stream)) {   // one launch
+void small_stages(const tmoe_plan* p, const void* packed, tmoe::FwdArgs& a, hipStream_t stream,
+                  Launch (&st)[kStages]) {
+  const bool fold = p->fold;
+  bool decode = fold && tmoe::small_decode_ok(a, stream);
+  if (p->decode_fold && a.T <= tmoe::kDecodeMaxT) {
+    const tmoe::FwdArgs f = decode_fold_args(p, a, packed);
+    if ((decode = tmoe::small_decode_ok(f, stream))) a = f;
+  }
+  if (decode) {   // one launch
     st[0] = tmoe::launch_small_decode;
     st[1] = launch_nothing;
     st[2] = launch_nothing;
@@ -382,7 +403,12 @@ int tmoe_plan_create(const tmoe_shape* shape, tmoe_plan** plan_out) {
   p->off_core_p = 0;
   if (p->core_p) { p->off_core_p = o; o = align256(o + (size_t)p->rk * s.r2 * s.r3 * p->es); }
   p->off_fold = 0;
-  if (p->fold) { p->off_fold = o; o = align256(o + (size_t)s.d_out * K * p->es); }
+  p->decode_fold = !p->fold && bf && !(s.flags & TMOE_FLAG_NO_FOLD) &&
+                   tmoe::decode_fold_ok(s.E, p->rk, s.r3, s.d_out);
+  if (p->fold || p->decode_fold) {
+    p->off_fold = o;
+    o = align256(o + (size_t)s.d_out * K * p->es);
+  }
   // the register-weight front (k_front_ks): bf16 kernels, r3 = 256, one router block
   p->wfrag = bf && s.r3 == 256 && p->E_pad == 32;
   p->off_wfrag = 0;
@@ -412,8 +438,9 @@ int tmoe_plan_folded(const tmoe_plan* plan) { return plan && plan->fold ? 1 : 0;
 // r1 in {1, 2, 4}; 3: P^T also for r1 = 4G in rank-group order; 4: plans with fewer
 // experts than ranks packed in the expert form (identity U_expert, core G); 5: folded
 // plans add W^T = (core U_out)^T; 7: bf16 plans with r3 = 256 and E_pad = 32 add the
-// front operand in fragment order (k_front_ks).
-int tmoe_packed_layout_version(void) { return 7; }
+// front operand in fragment order (k_front_ks); 8: W^T also for unfolded plans whose
+// decode-size batches run folded.
+int tmoe_packed_layout_version(void) { return 8; }
 
 size_t tmoe_workspace_bytes(const tmoe_plan* plan, int64_t T) {
   if (!plan || T < 0) return 0;
@@ -484,7 +511,7 @@ int tmoe_pack_weights(const tmoe_plan* p, const void* router_w, const void* U_in
   if ((e = tmoe::launch_to_f32(bias, reinterpret_cast<float*>(base + p->off_bias), s.d_out,
                                s.dtype, st)) != hipSuccess)
     return hip_fail(e, "pack bias");
-  if (p->fold && (e = pack_fold(p, base, st)) != hipSuccess) return hip_fail(e, "pack W (fold)");
+  if ((p->fold || p->decode_fold) && (e = pack_fold(p, base, st)) != hipSuccess) return hip_fail(e, "pack W (fold)");
   return TMOE_OK;
 }
 
@@ -552,7 +579,7 @@ int tmoe_pack_weights_fp8(const tmoe_plan* p, const void* router_w, const uint8_
   if ((e = tmoe::launch_to_f32(core_scale, f32at(p->off_craw), s.r1 * s.r2, TMOE_F32, st)) !=
       hipSuccess)
     return hip_fail(e, "pack core scales");
-  if (p->fold && (e = pack_fold(p, base, st)) != hipSuccess) return hip_fail(e, "pack W (fold)");
+  if ((p->fold || p->decode_fold) && (e = pack_fold(p, base, st)) != hipSuccess) return hip_fail(e, "pack W (fold)");
   return TMOE_OK;
 }
 
@@ -611,7 +638,7 @@ int forward_impl(const tmoe_plan* p, const void* x, int64_t T, const void* packe
       fused || fused_mid ? launch_nothing : tmoe::launch_outproj};
   // folded: the out-projection builds c (x) z from z and c itself (no core stage)
   Launch small_path[kStages];
-  small_stages(a, fold, st, small_path);
+  if (small) small_stages(p, packed, a, st, small_path);
   const Launch* stages = small ? small_path : big_path;
   const char* stage_names[kStages] = {"front (router + in-projection)", "core",
                                       "out-projection"};
@@ -724,9 +751,9 @@ int tmoe_forward_glu(const tmoe_plan* p, const void* x, int64_t T, const void* p
     u = folded_args(p, u, packed_up, st);
   }
   if (T <= tmoe::kSmallT) {
-    for (const tmoe::FwdArgs* a : {&g, &u}) {
+    for (tmoe::FwdArgs* a : {&g, &u}) {
       Launch small[kStages];
-      small_stages(*a, p->fold, st, small);
+      small_stages(p, a == &g ? packed_gate : packed_up, *a, st, small);
       for (int i = 0; i < kStages; ++i)
         if ((e = small[i](*a, st)) != hipSuccess) return hip_fail(e, "tmoe_forward_glu");
     }
@@ -847,6 +874,9 @@ int tmoe_forward_path(const tmoe_plan* p, int64_t T) {
       tmoe::FwdArgs f = folded_args(p, a, fake, nullptr);
       if (tmoe::small_decode_shape_ok(f)) return TMOE_PATH_DECODE;
     }
+    if (p->decode_fold && T <= tmoe::kDecodeMaxT &&
+        tmoe::small_decode_shape_ok(decode_fold_args(p, a, fake)))
+      return TMOE_PATH_DECODE;
     return TMOE_PATH_SMALL;
   }
   if (p->fold) {

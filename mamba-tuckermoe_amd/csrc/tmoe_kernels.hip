@@ -462,8 +462,11 @@ hipError_t launch_small_decode_t(const FwdArgs& a, hipStream_t st) {
   b.epoch = next_epoch();
   const dim3 grid((unsigned)((a.r3 / 16 + 1) * dev::kDecodeRowGroups + cdiv(a.d_out, 16))),
       block(64 * kSkW);
-  hipLaunchKernelGGL((dev::k_sk_decode<MF, kSkW>), grid, block, dev::sk_decode_dyn_bytes(MF, a),
-                     st, b);
+  const size_t dyn = dev::sk_decode_dyn_bytes(MF, a);
+  if (a.r1 * a.r3 > 1024)
+    hipLaunchKernelGGL((dev::k_sk_decode<MF, kSkW, 2>), grid, block, dyn, st, b);
+  else
+    hipLaunchKernelGGL((dev::k_sk_decode<MF, kSkW, 1>), grid, block, dyn, st, b);
   return hipGetLastError();
 }
 
@@ -551,6 +554,11 @@ hipError_t launch_fold_out_t(const uint16_t* coreT, const uint16_t* uoutT, const
                              int64_t d_out, hipStream_t st) {
   if (K == 0 || d_out == 0) return hipSuccess;
   if (K % 32 || r2 % 32 || r3 % 32) return hipErrorInvalidValue;
+  if (!cs && !os && K % 64 == 0 && r2 % 64 == 0) {
+    hipLaunchKernelGGL(dev::k_fold_out_mfma, dim3(cdiv(K, 128), cdiv(d_out, 128)), dim3(256), 0, st,
+                       coreT, uoutT, dst, K, r2, d_out);
+    return hipGetLastError();
+  }
   hipLaunchKernelGGL(dev::k_fold_out_t, dim3(cdiv(K, 32), cdiv(d_out, 32)), dim3(256), 0, st,
                      coreT, uoutT, cs, os, dst, K, r3, r2, d_out);
   return hipGetLastError();

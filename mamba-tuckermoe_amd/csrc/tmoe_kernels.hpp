@@ -609,6 +609,37 @@ __device__ __forceinline__ void tile_coords(int n_tiles_n, int n_tiles, int& tm,
   tile_coords_of(blockIdx.x, n_tiles_n, n_tiles, tm, tn);
 }
 
+// ---- K-major operands: transposed reads ---------------------------------------
+// An operand whose rows are K steps (64 of them in an LDS tile, 128 columns, 256 bytes a
+// row) gives an MFMA fragment, 8 K steps of one column a lane, as two transposed 64-bit
+// reads (ds_read_b64_tr_b16: 16 lanes read 4 rows x 16 columns and get a column each).
+// The 32-byte units of row k lie at unit ^ tr_swz(k): the four rows that 16 lanes touch,
+// and the two column blocks of 32 lanes, then fall on eight distinct units (256 bytes).
+// A DMA instruction fills four rows: lane l of block blk fetches 16-byte chunk
+// tr_dma_chunk(l) of row 4 blk + (l >> 4). The compiler waits for every DMA in flight
+// before a transposed read (it takes them for aliases): issue none ahead of the reads.
+typedef short s16x4 __attribute__((ext_vector_type(4)));
+typedef __attribute__((address_space(3))) s16x4* lds_s16x4;
+__device__ __forceinline__ int tr_swz(int k) { return ((k & 3) << 1) | ((k >> 1) & 1); }
+__device__ __forceinline__ int tr_dma_chunk(int lane) {
+  const int c = lane & 15;
+  return (((c >> 1) ^ tr_swz(lane >> 4)) << 1) | (c & 1);
+}
+// the fragment of K rows 16 ks .. + 15 and column block u (32 columns) of the tile at LDS
+// address base
+__device__ __forceinline__ u32x4 tr_frag(uint32_t base, int ks, int u, int lane) {
+  const int l = lane & 15, g = lane >> 4;
+  const int unit = (u * 2 + (g & 1)) ^ tr_swz(l >> 2);
+  const uint32_t a = base + (16 * ks + 8 * (g >> 1) + (l >> 2)) * 256 + unit * 32 + (l & 3) * 8;
+  const uint2 w0 = __builtin_bit_cast(
+      uint2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4)(size_t)a));
+  const uint2 w1 = __builtin_bit_cast(
+      uint2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4)(size_t)(a + 4 * 256)));
+  u32x4 o;
+  o[0] = w0.x; o[1] = w0.y; o[2] = w1.x; o[3] = w1.y;
+  return o;
+}
+
 // ---- C tile store through LDS ----------------------------------------------
 // The MFMA result layout gives each lane one column of sixteen rows, so direct
 // stores would be 2- or 4-byte scatters. The tile is instead converted into LDS
@@ -2156,10 +2187,93 @@ __global__ __launch_bounds__(64 * WM * WN) void k_outproj_pp(FwdArgs a) {
 }
 
 // ---- packing kernels -----------------------------------------------------
+// k_fold_out_t without scales, on the MFMAs: a 128 (rows n) x 128 (kk) tile of W^T a
+// work-group of 4 waves, K tiles of 64 q; uoutT's rows are q-contiguous, coreT's are K steps
+// (tr_frag). fp32 sums, one rounding. Packing a layer of K 1024, d_out 2304, r2 1024: 254 us
+// with k_fold_out_t, 46 with this kernel.
+__global__ __launch_bounds__(256, 2) void k_fold_out_mfma(const uint16_t* __restrict__ coreT,
+                                                          const uint16_t* __restrict__ uoutT,
+                                                          uint16_t* __restrict__ dst, int64_t K,
+                                                          int64_t r2, int64_t d_out) {
+  typedef Tile<128, 128, 0, 2, 2, 1, 1, 2, true, true> TL;   // for the store
+  constexpr int kStage = 2 * 1024;   // u32x4 slots: A 128 rows x 8 chunks, B 64 rows x 16
+  __shared__ u32x4 smem[cmax(2 * kStage * 16, TileStage<TL, uint16_t>::kBytes) / 16];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int wm = wave >> 1, wn = wave & 1;
+  const int64_t k0 = (int64_t)blockIdx.x * 128, n0 = (int64_t)blockIdx.y * 128;
+  const int rows = (int)(d_out - n0 < 128 ? d_out - n0 : 128);
+  const int cols = (int)(K - k0 < 128 ? K - k0 : 128);
+  const char *ap[4], *bp[4];
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    const int blk = wave * 4 + j, r = blk * 8 + (lane >> 3);
+    ap[j] = reinterpret_cast<const char*>(uoutT + (n0 + (r < rows ? r : rows - 1)) * r2) +
+            dma_chunk(lane, blk) * 16;
+    const int ch = tr_dma_chunk(lane);
+    bp[j] = reinterpret_cast<const char*>(coreT + (int64_t)(blk * 4 + (lane >> 4)) * K + k0) +
+            (ch * 8 < cols ? ch * 16 : 0);   // columns past K: any, never stored
+  }
+  const uint32_t lds0 = (uint32_t)(size_t)(__attribute__((address_space(3))) u32x4*)smem;
+  auto dma = [&](int stage) __attribute__((always_inline)) {
+    const uint32_t s = lds0 + stage * (kStage * 16);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      __builtin_amdgcn_global_load_lds((gbl_cvptr)ap[j], (lds_vptr)(size_t)(s + (wave * 4 + j) * 1024),
+                                       16, 0, 0);
+      __builtin_amdgcn_global_load_lds(
+          (gbl_cvptr)bp[j], (lds_vptr)(size_t)(s + 16384 + (wave * 4 + j) * 1024), 16, 0, 0);
+      ap[j] += kTileKBytes;
+      bp[j] += 64 * K * 2;
+    }
+  };
+  f32x16 acc[TL::FM][TL::FN];
+#pragma unroll
+  for (int i = 0; i < 2; ++i)
+#pragma unroll
+    for (int j = 0; j < 2; ++j) acc[i][j] = zero16();
+  const int nkt = (int)(r2 / 64);
+  dma(0);
+  for (int kt = 0; kt < nkt; ++kt) {
+    wait_vm_lds<0>();
+    lds_barrier();
+    const u32x4* s = smem + (kt & 1) * kStage;
+    const uint32_t sb = lds0 + (kt & 1) * (kStage * 16) + 16384;
+    u32x4 af[4][2], bf[4][2];
+#pragma unroll
+    for (int ks = 0; ks < 4; ++ks)
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {
+        af[ks][i] = s[lds_slot(wm * 64 + i * 32 + (lane & 31), ks * 2 + (lane >> 5))];
+        bf[ks][i] = tr_frag(sb, ks, wn * 2 + i, lane);
+      }
+    __builtin_amdgcn_sched_barrier(0);
+    if (kt + 1 < nkt) dma((kt + 1) & 1);
+#pragma unroll
+    for (int ks = 0; ks < 4; ++ks)
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int j = 0; j < 2; ++j) mma(acc[i][j], af[ks][i], bf[ks][j], EltBF16{});
+  }
+  mfma_drain();
+  __syncthreads();
+  char* stage = reinterpret_cast<char*>(smem);
+  float zero[TL::FN], one[TL::FN];
+#pragma unroll
+  for (int j = 0; j < TL::FN; ++j) {
+    zero[j] = 0.f;
+    one[j] = 1.f;
+  }
+  stage_tile<TL, uint16_t>(acc, stage, zero, one);
+  __syncthreads();
+  flush_tile<TL, uint16_t>(stage, dst + n0 * K + k0, K, rows, cols);
+}
+
 // W^T of a folded plan: dst[n][kk] = os[n] * sum_q uoutT[n][q] * coreT[q][kk] * cs[kk / r3][q]
 // (bf16 bits in and out, fp32 sums in q order, one rounding), i.e. W = core (K x r2)
 // times U_out (r2 x d_out) stored transposed (d_out rows of K). 32 x 32 output tiles,
-// 256 threads each holding 4 rows n; K and r2 are multiples of 32, d_out of 16.
+// 256 threads each holding 4 rows n; K and r2 are multiples of 32, d_out of 16. For fp8
+// plans (cs, os set); the others take k_fold_out_mfma.
 __global__ void k_fold_out_t(const uint16_t* __restrict__ coreT, const uint16_t* __restrict__ uoutT,
                              const float* __restrict__ cs, const float* __restrict__ os,
                              uint16_t* __restrict__ dst, int64_t K, int64_t r3, int64_t r2,

@@ -465,14 +465,6 @@ __global__ __launch_bounds__(256) void k_latent_scale(const uint16_t* __restrict
   *reinterpret_cast<u32x4*>(xs + i * r3 + ch * 8) = o;
 }
 
-typedef short s16x4 __attribute__((ext_vector_type(4)));
-typedef __attribute__((address_space(3))) s16x4* lds_s16x4;
-
-// 32-byte units of row k of a 256-byte-row LDS tile sit at unit ^ tr_swz(k): the four
-// rows that 16 lanes of a transposed read touch, and the two column blocks of its 32
-// lanes, then fall on eight distinct units (256 bytes).
-__device__ __forceinline__ int tr_swz(int k) { return ((k & 3) << 1) | ((k >> 1) & 1); }
-
 struct LatentDg {
   const char* xs;         // (B k, r3) by expert
   const char* dout;       // (B, r2)
@@ -503,8 +495,7 @@ __global__ __launch_bounds__(256, 2) void k_latent_dge(LatentDg q) {
   const int tm = t / ntn, tn = t - tm * ntn;
   const int4 d = q.chunks[c];
   const int sub = lane >> 4;
-  const int cp = lane & 15;
-  const int chunk = (((cp >> 1) ^ tr_swz(sub)) << 1) | (cp & 1);   // logical 16-byte chunk
+  const int chunk = tr_dma_chunk(lane);
   const int64_t a_row = (int64_t)q.r3 * 2, b_row = (int64_t)q.r2 * 2;
   const char* abase = q.xs + d.x * a_row + tm * 256 + chunk * 16;
   const char* bbase = q.dout + tn * 256 + chunk * 16;
@@ -538,20 +529,6 @@ __global__ __launch_bounds__(256, 2) void k_latent_dge(LatentDg q) {
   for (int i = 0; i < 2; ++i)
 #pragma unroll
     for (int j = 0; j < 2; ++j) acc[i][j] = zero16();
-  // byte offset of this lane's transposed read of column block 0, entry rows 0 .. 3 (+ 8
-  // for the upper lanes); block u and row group r add to it
-  const int l = lane & 15, g = lane >> 4;
-  const int rrow = 8 * (g >> 1) + (l >> 2);
-  auto frag = [&](uint32_t base, int ks, int u) __attribute__((always_inline)) {
-    u32x4 o;
-    const int unit = (u * 2 + (g & 1)) ^ tr_swz(l >> 2);
-    const uint32_t a = base + (16 * ks + rrow) * 256 + unit * 32 + (l & 3) * 8;
-    const s16x4 v0 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4)(size_t)a);
-    const s16x4 v1 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4)(size_t)(a + 4 * 256));
-    const uint2 w0 = __builtin_bit_cast(uint2, v0), w1 = __builtin_bit_cast(uint2, v1);
-    o[0] = w0.x; o[1] = w0.y; o[2] = w1.x; o[3] = w1.y;
-    return o;
-  };
   load_tok(0);
   dma(0, 0);
   load_tok(1);
@@ -568,8 +545,8 @@ __global__ __launch_bounds__(256, 2) void k_latent_dge(LatentDg q) {
     for (int ks = 0; ks < 4; ++ks)
 #pragma unroll
       for (int i = 0; i < 2; ++i) {
-        af[ks][i] = frag(sa, ks, wm * 2 + i);
-        bf[ks][i] = frag(sb, ks, wn * 2 + i);
+        af[ks][i] = tr_frag(sa, ks, wm * 2 + i, lane);
+        bf[ks][i] = tr_frag(sb, ks, wn * 2 + i, lane);
       }
     __builtin_amdgcn_sched_barrier(0);
     if (kt + 1 < nkt) {

@@ -590,7 +590,7 @@ __global__ __launch_bounds__(64 * W) void k_sk_epi_gemm(FwdArgs a) {
 // the GEMM of k_sk_epi_gemm against W^T with A = c (x) z from LDS. Producer data
 // crosses the work-groups through the scratch at a.raw, 16 bytes per device-scope
 // access: zr (T, r3) fp32, cs (T, r1) fp32. T <= MF * 16: one token block; the z a
-// thread loads is held in registers (kDecodeGroups 4-column groups per thread).
+// thread loads is held in registers (MF 4-column groups per thread).
 constexpr int kDecodeRowGroups = 4;   // T <= 64: at most 16 tokens a producer
 struct SkDecodeScratch {
   float *zr, *cs;
@@ -599,7 +599,6 @@ struct SkDecodeScratch {
     cs = zr + a.T * a.r3;
   }
 };
-constexpr int kDecodeGroups = 4;
 // Dynamic LDS bytes of k_sk_decode: a router work-group's U_expert and c rows; a
 // consumer's z rows (bf16) and c rows.
 inline size_t sk_decode_dyn_bytes(int mf, const FwdArgs& a) {
@@ -705,9 +704,13 @@ __device__ __forceinline__ void route_row16(const FwdArgs& a, int64_t t, int sl,
   }
 }
 
-template <int MF, int W>
+// GB: K groups a consumer wave's weight loads hold at once, issued before the wait: 2 where
+// K = 2048 gives each of the 16 waves two (K <= 1024: one). One token block (MF = 1) stays
+// within 64 registers, so that two work-groups fit a compute unit (d_out 4608: 356 of them).
+template <int MF, int W, int GB>
 __global__ __launch_bounds__(64 * W) void k_sk_decode(FwdArgs a) {
   static_assert(W == 16, "one 16-lane row per token of a 64-token block");
+  constexpr int kGroups = MF;   // 4-column groups of z a thread holds: 16 MF tokens, r3 <= 256
   typedef EltBF16 Elt;
   typedef typename Elt::T T;
   __shared__ float red[SkLds<MF, W>::kFloats];
@@ -773,15 +776,15 @@ __global__ __launch_bounds__(64 * W) void k_sk_decode(FwdArgs a) {
   // under the wait: the GEMM's first weight chunks, the column's bias and scale,
   // and the gain of the z groups g = thread + 64 W j (4 columns each) this thread
   // normalises
-  u32x4 bpre[1][2];
-  skinny_b_first<Elt, W, 1>(bsrc, rb, cols_valid, K, bpre);
+  u32x4 bpre[GB][2];
+  skinny_b_first<Elt, W, GB>(bsrc, rb, cols_valid, K, bpre);
   const int c = threadIdx.x & 15;
   const float bias = c < cols_valid ? a.bias[n0 + c] : 0.f;
   const float osc = a.out_scale && c < cols_valid ? a.out_scale[n0 + c] : 1.f;
   const int G = R3 / 4, NG = Tn * G;
-  float gv[kDecodeGroups][4];
+  float gv[kGroups][4];
 #pragma unroll
-  for (int j = 0; j < kDecodeGroups; ++j) {
+  for (int j = 0; j < kGroups; ++j) {
     const int g = threadIdx.x + 64 * W * j;
     const int col = (g - (g / G) * G) * 4;
 #pragma unroll
@@ -791,9 +794,9 @@ __global__ __launch_bounds__(64 * W) void k_sk_decode(FwdArgs a) {
                              reinterpret_cast<int*>(red), false, a.wait_polls, a.status);
   // every load first: the z groups and c
   const __amdgpu_buffer_rsrc_t rz = coherent_rsrc(sc.zr, (int64_t)Tn * R3);
-  f32x4 zv[kDecodeGroups];
+  f32x4 zv[kGroups];
 #pragma unroll
-  for (int j = 0; j < kDecodeGroups; ++j) {
+  for (int j = 0; j < kGroups; ++j) {
     const int g = threadIdx.x + 64 * W * j;
     zv[j] = load_coherent4(rz, g < NG ? g * 16 : Tn * R3 * 4);   // past the end: 0
   }
@@ -802,7 +805,7 @@ __global__ __launch_bounds__(64 * W) void k_sk_decode(FwdArgs a) {
   // each row's sum of squares: its G groups sit in G consecutive lanes of one wave
   // (G = r3 / 4 in {16, 32, 64}), added by the lanes' cross-lane sum
 #pragma unroll
-  for (int j = 0; j < kDecodeGroups; ++j) {
+  for (int j = 0; j < kGroups; ++j) {
     const int g = threadIdx.x + 64 * W * j;
     if ((g & ~63) >= NG) break;   // wave-uniform: no group of this wave left
     const float ss = lane_group_sum(((zv[j][0] * zv[j][0] + zv[j][1] * zv[j][1]) +
@@ -817,8 +820,8 @@ __global__ __launch_bounds__(64 * W) void k_sk_decode(FwdArgs a) {
   }
   __syncthreads();
   SkKhatriRaoLds<Elt> as{zl, cl, R1, R3, Tn};
-  skinny_tile<Elt, MF, W, 1, SkKhatriRaoLds<Elt>, true>(as, bsrc, rb, cols_valid, K, red, 0,
-                                                        nullptr, 0, bpre);
+  skinny_tile<Elt, MF, W, GB, SkKhatriRaoLds<Elt>, true>(as, bsrc, rb, cols_valid, K, red, 0,
+                                                         nullptr, 0, bpre);
   for (int e = threadIdx.x; e < MF * 256; e += 64 * W) {
     const int row = e >> 4;
     if (row < Tn && c < cols_valid) {
