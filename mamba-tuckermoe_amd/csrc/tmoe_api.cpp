@@ -129,30 +129,42 @@ hipEvent_t prof_event() {
 struct Layout {
   size_t z, c, idx, w, mid, raw, mpart, sync, total;
   int split, fsplit;
+  int osplit;   // FwdArgs::out_split
 };
 
-// lean: without the fp32 plans' K slices (their planes), for a caller whose scratch
-// does not hold them.
+// Whether a forward of T tokens is a folded batch (tmoe::batch_out_split).
+bool batch_folded(const tmoe_plan* p, int64_t T) {
+  if (T <= tmoe::kDecodeMaxT || T > tmoe::kSmallT) return false;
+  return p->fold || (p->decode_fold && tmoe::batch_out_tiles(T, p->s.d_out) <= tmoe::kBatchFoldTiles);
+}
+
+// lean: without the fp32 plans' K slices (their planes) and without folded batches, for a
+// caller whose scratch does not hold them.
 Layout workspace_layout(const tmoe_plan* p, int64_t T, bool lean = false) {
   Layout L{};
+  const bool batch = !lean && batch_folded(p, T);
+  const bool fold = p->fold || batch;
   lean = lean && p->kdtype == TMOE_F32;
   size_t o = 0;
   // k_core_pp reads c and stores mid in whole 256-token tiles; a folded plan's
   // out-projection reads its A operand (c (x) z in mid) in whole 256-row tiles
-  const int64_t tile_rows = p->core_p || p->fold
+  const int64_t tile_rows = p->core_p || fold
                                 ? (T + tmoe::kCorePRows - 1) / tmoe::kCorePRows * tmoe::kCorePRows
                                 : T;
   // z in whole tiles too: a folded plan's out-projection may read it as its A operand
-  L.z = o;   o = align256(o + (size_t)(p->fold ? tile_rows : T) * p->s.r3 * p->es);
+  L.z = o;   o = align256(o + (size_t)(fold ? tile_rows : T) * p->s.r3 * p->es);
   L.c = o;   o = align256(o + (size_t)tile_rows * p->rk * sizeof(float));
   L.idx = o; o = align256(o + (size_t)T * p->s.k * sizeof(int32_t));
   L.w = o;   o = align256(o + (size_t)T * p->s.k * sizeof(float));
-  // mid: (T, r2), or c (x) z (T, rk*r3) in a folded plan's large-T forward
+  // mid: (T, r2), or c (x) z (T, rk*r3) in a folded large-T forward or batch
   const int64_t mid_cols =
-      p->fold && T > tmoe::kSmallT && p->rk * p->s.r3 > p->s.r2 ? p->rk * p->s.r3 : p->s.r2;
+      (batch || (p->fold && T > tmoe::kSmallT)) && p->rk * p->s.r3 > p->s.r2 ? p->rk * p->s.r3
+                                                                             : p->s.r2;
   L.mid = o; o = align256(o + (size_t)tile_rows * mid_cols * p->es);
   L.raw = o;
-  L.fsplit = lean ? 1 : tmoe::front_split(T, p->s.d_in, p->E_pad, p->es);
+  // the small-T kernels read one plane; a folded batch's front may be the sliced one
+  L.fsplit = lean || (T <= tmoe::kSmallT && !batch)
+                 ? 1 : tmoe::front_split(T, p->s.d_in, p->E_pad, p->es);
   if (T <= tmoe::kSmallT || L.fsplit > 1) {
     int64_t raw_floats = L.fsplit * T * tmoe::raw_stride(p->s.r3, p->s.E);
     // the one-launch decode's scratch (z columns, sums of squares, c)
@@ -163,7 +175,14 @@ Layout workspace_layout(const tmoe_plan* p, int64_t T, bool lean = false) {
   // k_core_pp in rank groups: fp32 partial sums of mid
   L.mpart = 0;
   L.split = 1;
-  if (p->core_p && tmoe::core_p_grouped(p->rk) && T > tmoe::kSmallT) {
+  L.osplit = 0;
+  if (batch) {
+    L.osplit = tmoe::batch_out_split(T, p->s.d_out, p->rk * p->s.r3);
+    if (L.osplit > 1) {
+      L.mpart = o;
+      o = align256(o + (size_t)L.osplit * T * p->s.d_out * sizeof(float));
+    }
+  } else if (p->core_p && tmoe::core_p_grouped(p->rk) && T > tmoe::kSmallT) {
     L.split = tmoe::core_p_split(T, p->rk, p->s.r2);
     L.mpart = o;
     o = align256(o + (size_t)L.split * tile_rows * p->s.r2 * sizeof(float));
@@ -222,10 +241,11 @@ tmoe::FwdArgs make_args(const tmoe_plan* p, const void* x, int64_t T, const void
   a.c = reinterpret_cast<float*>(ws + L.c);
   a.z = ws + L.z;
   a.mid = ws + L.mid;
-  a.mid_rows_256 = p->core_p || p->fold;   // workspace_layout's tile_rows
+  a.mid_rows_256 = p->core_p || p->fold || L.osplit > 0;   // workspace_layout's tile_rows
   a.raw = reinterpret_cast<float*>(ws + L.raw);
   a.mpart = L.mpart ? reinterpret_cast<float*>(ws + L.mpart) : nullptr;
   a.core_split = L.split;
+  a.out_split = L.osplit;
   a.front_split = L.fsplit;
   a.sync = reinterpret_cast<uint32_t*>(ws + L.sync);
   a.wait_polls = g_wait_polls.load(std::memory_order_relaxed);
@@ -283,6 +303,13 @@ using Launch = hipError_t (*)(const tmoe::FwdArgs&, hipStream_t);
 void small_stages(const tmoe_plan* p, const void* packed, tmoe::FwdArgs& a, hipStream_t stream,
                   Launch (&st)[kStages]) {
   const bool fold = p->fold;
+  if (a.out_split > 0) {   // a folded batch (a: the folded arguments)
+    a.cz = a.mid;
+    st[0] = a.front_split > 1 ? tmoe::launch_front : tmoe::launch_small_front;
+    st[1] = launch_nothing;
+    st[2] = tmoe::launch_outproj;
+    return;
+  }
   bool decode = fold && tmoe::small_decode_ok(a, stream);
   if (p->decode_fold && a.T <= tmoe::kDecodeMaxT) {
     const tmoe::FwdArgs f = decode_fold_args(p, a, packed);
@@ -623,7 +650,7 @@ int forward_impl(const tmoe_plan* p, const void* x, int64_t T, const void* packe
 
   hipStream_t st = static_cast<hipStream_t>(stream);
   const bool small = T <= tmoe::kSmallT;
-  const bool fold = p->fold;
+  const bool fold = p->fold || a.out_split > 0;
   // the K-sliced front in one launch where the device and the stream allow
   a.front_one = !(p->s.flags & TMOE_FLAG_NO_FUSE) && tmoe::front_sliced_ok(a, st);
   if (fold) a = folded_args(p, a, packed, st);
@@ -746,7 +773,8 @@ int tmoe_forward_glu(const tmoe_plan* p, const void* x, int64_t T, const void* p
   u.epi_a = out;
   hipStream_t st = static_cast<hipStream_t>(stream);
   hipError_t e;
-  if (p->fold) {
+  const bool fold = p->fold || L.osplit > 0;
+  if (fold) {
     g = folded_args(p, g, packed_gate, st);
     u = folded_args(p, u, packed_up, st);
   }
@@ -759,7 +787,7 @@ int tmoe_forward_glu(const tmoe_plan* p, const void* x, int64_t T, const void* p
     }
     return TMOE_OK;
   }
-  const Launch mid = p->fold ? launch_cz : tmoe::launch_core;
+  const Launch mid = fold ? launch_cz : tmoe::launch_core;
   if ((e = tmoe::launch_front_pair(g, u, st)) != hipSuccess ||
       (e = mid(g, st)) != hipSuccess || (e = mid(u, st)) != hipSuccess ||
       (e = tmoe::launch_outproj(g, st)) != hipSuccess ||
@@ -879,7 +907,7 @@ int tmoe_forward_path(const tmoe_plan* p, int64_t T) {
       return TMOE_PATH_DECODE;
     return TMOE_PATH_SMALL;
   }
-  if (p->fold) {
+  if (p->fold || L.osplit > 0) {
     const tmoe::FwdArgs f = folded_args(p, a, fake, nullptr);
     if (!(p->s.flags & TMOE_FLAG_NO_FUSE) && tmoe::fused_large_shape_ok(f)) return TMOE_PATH_FUSED;
     if (!(p->s.flags & TMOE_FLAG_NO_FUSE) && tmoe::fused_mid_shape_ok(f))

@@ -72,6 +72,9 @@ struct FwdArgs {
   float* mpart;                 // (S, T_pad, r2) fp32  k_core_pp with r1 > 4: partial sums
                                 //                      over rank groups (null otherwise)
   int core_split;               // S: parts an output tile's rank groups are split into
+  int out_split;                // folded batches (batch_out_split): K slices of the
+                                //                      out-projection, their planes in mpart;
+                                //                      0: not such a batch
   int front_split;              // K slices of the large-T front (raw holds that many
                                 //                      (T, r3 + E) fp32 planes), 1: none
   bool front_one;               // front_split > 1: slices and epilogue in one launch
@@ -158,7 +161,7 @@ constexpr int64_t front_slice_rows(int64_t es) { return es == 2 ? 64 : 32; }
 inline int front_split(int64_t T, int64_t d_in, int64_t E_pad, int64_t es) {
   // E_pad = 256 measured slower sliced (C4: front 44.6 us against 34.8 us for the
   // split z / router front plus 7.7 us of k_expand_cz)
-  if (T <= 256 || E_pad > 128) return 1;
+  if (T <= 64 || E_pad > 128) return 1;
   const int64_t rows = front_slice_rows(es);
   const int64_t tiles = (T + rows - 1) / rows, nkt = d_in * es / 128;
   // measured at d_in = 1536, bf16: slices win up to T = 4096 (64 tiles); at 128 tiles
@@ -204,6 +207,28 @@ inline bool core_p_supported(int64_t r1, int64_t r2, bool bf16, bool fp8w) {
   if (core_p_grouped(r1)) return r1 % 4 == 0 && r2 % 64 == 0 && !fp8w;
   return (r1 == 1 || r1 == 2 || r1 == 4) && (r1 * r2) % 256 == 0 &&
          (!fp8w || r1 * r2 <= kCorePScales);
+}
+
+// Folded batches between the decode launch and the large-tile kernels (kDecodeMaxT < T <=
+// kSmallT): folded plans, and plans with decode_fold's W^T whose 64 x 128 out-projection tiles
+// number at most kBatchFoldTiles (one a compute unit; past it the fold's extra multiply-adds,
+// 3 times as many at the reference's 1536 -> 6144, outweigh the core's launches). The front's
+// per-token epilogue writes c (x) z; the out-projection is a plain GEMM of it against W^T, K
+// in slices of at least 4 K tiles of 64 while the tiles leave compute units idle. Per layer,
+// before and now: 1536 -> 6144 at T = 65 43.3 -> 27.3 us, 256 53.3 -> 30.5; the output
+// sub-block 50-54 -> 34; the folded 1536 -> 2304 layer at T = 128 31.8 -> 22.5, 256 39.2 ->
+// 24.9. Not past kSmallT for unfolded plans, though faster up to T = 2000 there: their core
+// then reduces over the ranks in fp32, and the fold would add the rounding of c z.
+constexpr int64_t kBatchFoldTiles = 256;
+inline int64_t batch_out_tiles(int64_t T, int64_t d_out) {
+  return (T + 63) / 64 * ((d_out + 127) / 128);
+}
+constexpr int64_t kMaxOutSlices = 8;
+inline int batch_out_split(int64_t T, int64_t d_out, int64_t K) {
+  int64_t s = kCoreUnits / batch_out_tiles(T, d_out);
+  if (s > K / 256) s = K / 256;
+  if (s > kMaxOutSlices) s = kMaxOutSlices;
+  return s > 1 ? (int)s : 1;
 }
 
 // The latent expert contraction of the training module (tmoe_latent.hpp) and its

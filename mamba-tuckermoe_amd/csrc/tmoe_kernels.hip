@@ -237,6 +237,16 @@ bool outproj_mid_tiles(const FwdArgs& a) {
 hipError_t launch_outproj_bf16(const FwdArgs& a, hipStream_t st) {
   typedef OutCfgBF16 C;
   const int64_t ncu = cu_count();
+  if (a.out_split > 0) {   // a folded batch
+    const dim3 grid(cdiv(a.T, 64) * cdiv(a.d_out, 128), a.out_split);
+    hipLaunchKernelGGL((dev::k_outproj<EltBF16, 64, 128, 2, 2, 3>), grid, dim3(256), 0, st, a);
+    if (a.out_split > 1) {
+      if (hipError_t e = hipGetLastError(); e != hipSuccess) return e;
+      hipLaunchKernelGGL(dev::k_out_combine<EltBF16>, dim3(cdiv(a.T * a.d_out, 1024)), dim3(256),
+                         0, st, a, a.out_split);
+    }
+    return hipGetLastError();
+  }
   if (outproj_tiled_ok(a)) {
     // measured at d_out = 2304, K = 1024 (plain GEMM, us): T = 2048: 128 x 144 tiles
     // 19.3, 128 x 288 23.8, 256 x 288 32.8; T = 4096: 36.2, 26.4, 34.0; T = 6144:

@@ -2090,12 +2090,13 @@ __global__ __launch_bounds__(256) void k_core_combine(FwdArgs a) {
 }
 
 // ---- k_outproj: out = mid U_out + bias  (model.py:101) --------------------
-// Both operands arrive by DMA through NS LDS stages.
+// Both operands arrive by DMA through NS LDS stages. With gridDim.y = S > 1 slices of K,
+// slice sl leaves its plane (T, d_out) of fp32 sums in mpart (k_out_combine adds them).
 template <class Elt, int BM, int BN, int WM, int WN, int NS>
 __global__ __launch_bounds__(64 * WM * WN) void k_outproj(FwdArgs a) {
   typedef typename Elt::T T;
   typedef Tile<BM, BN, 0, WM, WN, 1, 1, NS, true, true> TL;
-  __shared__ u32x4 smem[cmax(TL::kLdsBytes, TileStage<TL, T>::kBytes) / 16];
+  __shared__ u32x4 smem[cmax(TL::kLdsBytes, TileStage<TL, float>::kBytes) / 16];
 
   const int ntn = (int)((a.d_out + BN - 1) / BN);
   const int ntm = (int)((a.T + BM - 1) / BM);
@@ -2105,15 +2106,32 @@ __global__ __launch_bounds__(64 * WM * WN) void k_outproj(FwdArgs a) {
   const int64_t n0 = (int64_t)tn * BN;
   const int rows_valid = (int)(a.T - m0 < BM ? a.T - m0 : BM);
   const int64_t row_bytes = a.r2 * (int64_t)sizeof(T);
-  RowLoader al{reinterpret_cast<const char*>(a.mid) + m0 * row_bytes, row_bytes, rows_valid};
-  RowLoader bl{reinterpret_cast<const char*>(a.uoutT) + n0 * row_bytes, row_bytes,
+  const int S = (int)gridDim.y, sl = (int)blockIdx.y;
+  const int nkt = (int)(row_bytes / kTileKBytes);
+  const int kt0 = sl * nkt / S, kt1 = (sl + 1) * nkt / S;
+  const int64_t koff = (int64_t)kt0 * kTileKBytes;
+  RowLoader al{reinterpret_cast<const char*>(a.mid) + m0 * row_bytes + koff, row_bytes, rows_valid};
+  RowLoader bl{reinterpret_cast<const char*>(a.uoutT) + n0 * row_bytes + koff, row_bytes,
                (int)(a.d_out - n0)};
   f32x16 acc[TL::FM][TL::FN];
   NoExtra nx;
-  gemm_mainloop<TL, Elt>(acc, al, bl, (int)(row_bytes / kTileKBytes), smem, nx);
+  gemm_mainloop<TL, Elt>(acc, al, bl, kt1 - kt0, smem, nx);
 
   char* stage = reinterpret_cast<char*>(smem);
   const int cols_valid = (int)(a.d_out - n0);
+  if (S > 1) {
+    float zero[TL::FN], one[TL::FN];
+#pragma unroll
+    for (int j = 0; j < TL::FN; ++j) {
+      zero[j] = 0.f;
+      one[j] = 1.f;
+    }
+    stage_tile<TL, float>(acc, stage, zero, one);
+    __syncthreads();
+    flush_tile<TL, float>(stage, a.mpart + (sl * a.T + m0) * a.d_out + n0, a.d_out, rows_valid,
+                          cols_valid);
+    return;
+  }
   float bcol[TL::FN], scol[TL::FN];
   {
     const int wn = (threadIdx.x >> 6) % WN, lane = threadIdx.x & 63;
@@ -2127,6 +2145,44 @@ __global__ __launch_bounds__(64 * WM * WN) void k_outproj(FwdArgs a) {
   stage_tile<TL, T>(acc, stage, bcol, scol);
   __syncthreads();
   flush_tile_by<TL, T, TL::kThreads>(stage, a, m0, n0, rows_valid, cols_valid, (int)threadIdx.x);
+}
+
+// out from the S planes of k_outproj's K slices, in plane order, with its bias, scale and
+// fused epilogue: four columns a thread.
+template <class Elt>
+__global__ __launch_bounds__(256) void k_out_combine(FwdArgs a, int S) {
+  typedef typename Elt::T T;
+  const int64_t n = a.T * a.d_out, i = ((int64_t)blockIdx.x * 256 + threadIdx.x) * 4;
+  if (i >= n) return;
+  // every plane's load at once (past S: plane 0 again, not added)
+  float4 u[kMaxOutSlices];
+#pragma unroll
+  for (int p = 0; p < kMaxOutSlices; ++p)
+    u[p] = *reinterpret_cast<const float4*>(a.mpart + (p < S ? p : 0) * n + i);
+  float4 v = u[0];
+#pragma unroll
+  for (int p = 1; p < kMaxOutSlices; ++p)
+    if (p < S) {
+      v.x += u[p].x; v.y += u[p].y; v.z += u[p].z; v.w += u[p].w;
+    }
+  const int64_t col = i % a.d_out;
+  const float4 b = *reinterpret_cast<const float4*>(a.bias + col);
+  float y[4] = {v.x, v.y, v.z, v.w};
+  const float bb[4] = {b.x, b.y, b.z, b.w};
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    y[j] = a.out_scale ? y[j] * a.out_scale[col + j] + bb[j] : y[j] + bb[j];
+    if (a.epi_mode != kEpiNone)
+      y[j] = epi_value<Elt>(a.epi_mode, round_as(y[j], Elt{}),
+                            load_as_f32(static_cast<const T*>(a.epi_a) + i + j),
+                            a.epi_mode == kEpiResScale
+                                ? load_as_f32(static_cast<const T*>(a.epi_b) + col + j) : 0.f);
+  }
+  T* o = static_cast<T*>(a.out) + i;
+  if constexpr (sizeof(T) == 2)
+    *reinterpret_cast<uint2*>(o) = make_uint2(pack_bf16x2(y[0], y[1]), pack_bf16x2(y[2], y[3]));
+  else
+    *reinterpret_cast<float4*>(o) = make_float4(y[0], y[1], y[2], y[3]);
 }
 
 // Persistent bf16 out-projection (8 waves, ping-pong main loop): work-group b
