@@ -182,7 +182,7 @@ int tmoe_pack_weights_fp8(const tmoe_plan* plan, const void* router_w,
  *   logits   (T, E) f32, nullable: router scores x @ router_w^T (model.py:75)
  *   workspace of at least tmoe_workspace_bytes(plan, T) bytes. Its contents need
  *            no initialisation: kernels whose work-groups hand data to each other
- *            inside one launch (the T <= 64 bf16 decode launch, the E = 256 front,
+ *            inside one launch (the T <= 64 decode launch, the E = 256 front,
  *            the one-launch large-T forward) tag their signal words with a value
  *            drawn per launch, and wait for one at most a budget of polls
  *            (tmoe_set_wait_polls; about a second by default). Past it the affected
@@ -250,7 +250,7 @@ int tmoe_forward_static(const tmoe_plan* plan, const void* x, int64_t T, const v
  * No counterpart in the reference; for measurement tools, which attribute time
  * per kernel. Returns one of TMOE_PATH_* (0 for T == 0) or a negative error. */
 #define TMOE_PATH_SMALL  1  /* T <= 256: skinny kernels, two or three launches        */
-#define TMOE_PATH_DECODE 2  /* T <= 64, bf16: the whole layer in one folded launch      */
+#define TMOE_PATH_DECODE 2  /* T <= 64: the whole layer in one folded launch            */
 #define TMOE_PATH_LARGE  3  /* front, (core or c (x) z), out-projection launches      */
 #define TMOE_PATH_FUSED  4  /* large T, folded: the whole layer in one launch         */
 #define TMOE_PATH_LARGE_KR 5 /* large T, folded, E > 128: front (stores z and c) and an

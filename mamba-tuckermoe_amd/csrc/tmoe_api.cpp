@@ -134,7 +134,7 @@ struct Layout {
 
 // Whether a forward of T tokens is a folded batch (tmoe::batch_out_split).
 bool batch_folded(const tmoe_plan* p, int64_t T) {
-  if (T <= tmoe::kDecodeMaxT || T > tmoe::kSmallT) return false;
+  if (p->kdtype != TMOE_BF16 || T <= tmoe::kDecodeMaxT || T > tmoe::kSmallT) return false;
   return p->fold || (p->decode_fold && tmoe::batch_out_tiles(T, p->s.d_out) <= tmoe::kBatchFoldTiles);
 }
 
@@ -258,6 +258,10 @@ tmoe::FwdArgs make_args(const tmoe_plan* p, const void* x, int64_t T, const void
 hipError_t pack_fold(const tmoe_plan* p, char* base, hipStream_t st) {
   const tmoe_shape& s = p->s;
   auto f32at = [&](size_t off) { return reinterpret_cast<const float*>(base + off); };
+  if (p->kdtype == TMOE_F32)
+    return tmoe::launch_fold_out_f32(f32at(p->off_core), f32at(p->off_uout),
+                                     reinterpret_cast<float*>(base + p->off_fold), p->rk * s.r3,
+                                     s.r2, s.d_out, st);
   return tmoe::launch_fold_out_t(reinterpret_cast<const uint16_t*>(base + p->off_core),
                                  reinterpret_cast<const uint16_t*>(base + p->off_uout),
                                  p->fp8w ? f32at(p->off_craw) : nullptr,
@@ -430,8 +434,8 @@ int tmoe_plan_create(const tmoe_shape* shape, tmoe_plan** plan_out) {
   p->off_core_p = 0;
   if (p->core_p) { p->off_core_p = o; o = align256(o + (size_t)p->rk * s.r2 * s.r3 * p->es); }
   p->off_fold = 0;
-  p->decode_fold = !p->fold && bf && !(s.flags & TMOE_FLAG_NO_FOLD) &&
-                   tmoe::decode_fold_ok(s.E, p->rk, s.r3, s.d_out);
+  p->decode_fold = !p->fold && !(s.flags & TMOE_FLAG_NO_FOLD) &&
+                   tmoe::decode_fold_ok(s.E, p->rk, s.r3, s.d_out, (int64_t)p->es);
   if (p->fold || p->decode_fold) {
     p->off_fold = o;
     o = align256(o + (size_t)s.d_out * K * p->es);

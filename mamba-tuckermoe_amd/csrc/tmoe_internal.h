@@ -276,16 +276,17 @@ bool small_epi_fused_ok(const FwdArgs& a);
 bool small_decode_ok(const FwdArgs& a, hipStream_t stream);
 hipError_t launch_small_decode(const FwdArgs& a, hipStream_t stream);
 constexpr int64_t kDecodeMaxT = 64;
-// Unfolded bf16 plans whose decode-size batches (T <= kDecodeMaxT) still run folded, in
+// Unfolded plans whose decode-size batches (T <= kDecodeMaxT) still run folded, in
 // that one launch, against a W^T packed beside the two-GEMM weights: K = rk r3 of at most
 // 2048 (two K groups a consumer wave) and W^T of at most 32 MB (read whole by every
 // forward, about 6 us). The two-GEMM form takes three launches there: the reference
 // model's FFN (three layers and a norm) 61 us at T = 1 and 135 at T = 64, folded 41 and 80;
-// its 1536 -> 6144 layer 31 and 43, folded 14 and 29.
+// its 1536 -> 6144 layer 31 and 43, folded 14 and 29; in fp32 the 1536 -> 2304 layer 31 and 50,
+// folded 12 and 20, the 512 -> 1024 layer at T = 64 28, folded 18 (with its routing).
 constexpr int64_t kDecodeFoldK = 2048, kDecodeFoldBytes = 32 << 20;
-inline bool decode_fold_ok(int64_t E, int64_t rk, int64_t r3, int64_t d_out) {
+inline bool decode_fold_ok(int64_t E, int64_t rk, int64_t r3, int64_t d_out, int64_t es) {
   return E <= 16 && rk <= 32 && rk * r3 <= kDecodeFoldK &&
-         rk * r3 * d_out * 2 <= kDecodeFoldBytes;
+         rk * r3 * d_out * es <= kDecodeFoldBytes;
 }
 // floats of its scratch at FwdArgs::raw: z columns (T, r3), c (T, r1)
 constexpr int64_t sk_decode_scratch_floats(int64_t T, int64_t r3, int64_t r1) {
@@ -356,6 +357,8 @@ hipError_t launch_mix_core_t(const void* uexp, const void* core, void* dst, int6
 // from the packed core^T (r2, K) and U_out^T (d_out, r2) (bf16 bits); with fp8
 // weights each core entry takes its channel scale cs[(kk / r3) * r2 + q] and each
 // output column the U_out scale os[n] (both null otherwise). fp32 sums, one rounding.
+hipError_t launch_fold_out_f32(const float* coreT, const float* uoutT, float* dst, int64_t K,
+                               int64_t r2, int64_t d_out, hipStream_t stream);   // fp32 plans
 hipError_t launch_fold_out_t(const uint16_t* coreT, const uint16_t* uoutT, const float* cs,
                              const float* os, uint16_t* dst, int64_t K, int64_t r3, int64_t r2,
                              int64_t d_out, hipStream_t stream);

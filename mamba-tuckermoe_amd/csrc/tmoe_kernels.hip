@@ -452,7 +452,7 @@ bool stream_capturing(hipStream_t st) {
 }
 
 bool small_decode_shape_ok(const FwdArgs& a) {
-  if (a.dtype != kDtypeBF16 || a.T > kDecodeMaxT || a.T * a.r3 > 16384 || a.E > 16 ||
+  if (a.T > kDecodeMaxT || a.T * a.r3 > 16384 || a.E > 16 ||
       (a.r3 != 64 && a.r3 != 128 && a.r3 != 256) || !a.sync || a.r1 > 32)
     return false;
   const int mf = small_mf(a.T);
@@ -466,26 +466,32 @@ bool small_decode_ok(const FwdArgs& a, hipStream_t st) {
   return small_decode_shape_ok(a) && !stream_capturing(st);
 }
 
-template <int MF>
+template <class Elt, int MF>
 hipError_t launch_small_decode_t(const FwdArgs& a, hipStream_t st) {
   FwdArgs b = a;
   b.epoch = next_epoch();
   const dim3 grid((unsigned)((a.r3 / 16 + 1) * dev::kDecodeRowGroups + cdiv(a.d_out, 16))),
       block(64 * kSkW);
   const size_t dyn = dev::sk_decode_dyn_bytes(MF, a);
-  if (a.r1 * a.r3 > 1024)
-    hipLaunchKernelGGL((dev::k_sk_decode<MF, kSkW, 2>), grid, block, dyn, st, b);
+  if (a.r1 * a.r3 * (int64_t)sizeof(typename Elt::T) > 2048)   // over one K group a wave
+    hipLaunchKernelGGL((dev::k_sk_decode<Elt, MF, kSkW, 2>), grid, block, dyn, st, b);
   else
-    hipLaunchKernelGGL((dev::k_sk_decode<MF, kSkW, 1>), grid, block, dyn, st, b);
+    hipLaunchKernelGGL((dev::k_sk_decode<Elt, MF, kSkW, 1>), grid, block, dyn, st, b);
   return hipGetLastError();
 }
 
-hipError_t launch_small_decode(const FwdArgs& a, hipStream_t st) {
+template <class Elt>
+hipError_t launch_small_decode_e(const FwdArgs& a, hipStream_t st) {
   switch (small_mf(a.T)) {
-    case 1: return launch_small_decode_t<1>(a, st);
-    case 2: return launch_small_decode_t<2>(a, st);
-    default: return launch_small_decode_t<4>(a, st);
+    case 1: return launch_small_decode_t<Elt, 1>(a, st);
+    case 2: return launch_small_decode_t<Elt, 2>(a, st);
+    default: return launch_small_decode_t<Elt, 4>(a, st);
   }
+}
+
+hipError_t launch_small_decode(const FwdArgs& a, hipStream_t st) {
+  return a.dtype == kDtypeBF16 ? launch_small_decode_e<EltBF16>(a, st)
+                               : launch_small_decode_e<EltF32>(a, st);
 }
 
 hipError_t launch_front_pair(const FwdArgs& a0, const FwdArgs& a1, hipStream_t st) {
@@ -556,6 +562,15 @@ hipError_t launch_mix_core_t(const void* uexp, const void* core, void* dst, int6
     hipLaunchKernelGGL(dev::k_mix_core_t<float>, grid, block, 0, st,
                        static_cast<const float*>(uexp), static_cast<const float*>(core),
                        static_cast<float*>(dst), E, r1, r3, r2);
+  return hipGetLastError();
+}
+
+hipError_t launch_fold_out_f32(const float* coreT, const float* uoutT, float* dst, int64_t K,
+                               int64_t r2, int64_t d_out, hipStream_t st) {
+  if (K == 0 || d_out == 0) return hipSuccess;
+  if (K % 64 || r2 % 32) return hipErrorInvalidValue;
+  hipLaunchKernelGGL(dev::k_fold_out_f32, dim3(cdiv(K, 64), cdiv(d_out, 64)), dim3(256), 0, st,
+                     coreT, uoutT, dst, K, r2, d_out);
   return hipGetLastError();
 }
 

@@ -2325,6 +2325,73 @@ __global__ __launch_bounds__(256, 2) void k_fold_out_mfma(const uint16_t* __rest
   flush_tile<TL, uint16_t>(stage, dst + n0 * K + k0, K, rows, cols);
 }
 
+// W^T of an fp32 plan, 64 x 64 tiles, K tiles of 32 q (coreT's rows lie in LDS as in memory),
+// summed in fp64 on the MFMAs (16 x 16 x 4) and rounded once: with fp32 sums the folded
+// layer was further from exact than the two GEMMs (3.5e-7 against 2.4e-7 at K 512, r2 256).
+// Accumulator element e of lane l: row 4 e + (l >> 4), column l & 15.
+typedef double f64x4 __attribute__((ext_vector_type(4)));
+__global__ __launch_bounds__(256) void k_fold_out_f32(const float* __restrict__ coreT,
+                                                      const float* __restrict__ uoutT,
+                                                      float* __restrict__ dst, int64_t K,
+                                                      int64_t r2, int64_t d_out) {
+  __shared__ u32x4 smem[1024];
+  u32x4* sa = smem;         // 64 rows n x 8 chunks of 4 q (lds_slot)
+  u32x4* sb = smem + 512;   // 32 rows q x 16 chunks of 4 kk
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int wm = wave >> 1, wn = wave & 1, l16 = lane & 15, kq = lane >> 4;
+  const int64_t k0 = (int64_t)blockIdx.x * 64, n0 = (int64_t)blockIdx.y * 64;
+  const int rows = (int)(d_out - n0 < 64 ? d_out - n0 : 64);
+  f64x4 acc[2][2] = {};
+  u32x4 va[2], vb[2];
+  auto fetch = [&](int64_t q0) __attribute__((always_inline)) {
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      const int c = tid + 256 * i, ra = c >> 3, rb = c >> 4;
+      va[i] = *reinterpret_cast<const u32x4*>(uoutT + (n0 + (ra < rows ? ra : rows - 1)) * r2 + q0 +
+                                              (c & 7) * 4);
+      vb[i] = *reinterpret_cast<const u32x4*>(coreT + (q0 + rb) * K + k0 + (c & 15) * 4);
+    }
+  };
+  fetch(0);
+  for (int64_t q0 = 0; q0 < r2; q0 += 32) {
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      const int c = tid + 256 * i;
+      sa[lds_slot(c >> 3, c & 7)] = va[i];
+      sb[c] = vb[i];
+    }
+    __syncthreads();
+    if (q0 + 32 < r2) fetch(q0 + 32);
+    const float* a = reinterpret_cast<const float*>(sa);
+    const float* b = reinterpret_cast<const float*>(sb);
+#pragma unroll
+    for (int s = 0; s < 8; ++s) {
+      double af[2], bf[2];
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {
+        af[i] = a[lds_slot(wm * 32 + i * 16 + l16, s) * 4 + kq];
+        bf[i] = b[(4 * s + kq) * 64 + wn * 32 + i * 16 + l16];
+      }
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+          acc[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(af[i], bf[j], acc[i][j], 0, 0, 0);
+    }
+  }
+  mfma_drain();
+#pragma unroll
+  for (int i = 0; i < 2; ++i)
+#pragma unroll
+    for (int j = 0; j < 2; ++j)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const int r = wm * 32 + i * 16 + 4 * e + kq;
+        if (r < rows) dst[(n0 + r) * K + k0 + wn * 32 + j * 16 + l16] = (float)acc[i][j][e];
+      }
+}
+
 // W^T of a folded plan: dst[n][kk] = os[n] * sum_q uoutT[n][q] * coreT[q][kk] * cs[kk / r3][q]
 // (bf16 bits in and out, fp32 sums in q order, one rounding), i.e. W = core (K x r2)
 // times U_out (r2 x d_out) stored transposed (d_out rows of K). 32 x 32 output tiles,

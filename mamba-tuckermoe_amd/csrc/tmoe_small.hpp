@@ -600,11 +600,13 @@ struct SkDecodeScratch {
   }
 };
 // Dynamic LDS bytes of k_sk_decode: a router work-group's U_expert and c rows; a
-// consumer's z rows (bf16) and c rows.
+// consumer's z rows (the plan's dtype) and c rows.
 inline size_t sk_decode_dyn_bytes(int mf, const FwdArgs& a) {
   const size_t rows = (size_t)mf * 16;
   const size_t router = ((size_t)a.E * a.r1 + 16 * a.r1) * 4;
-  const size_t consumer = rows * sk_z_stride<uint16_t>((int)a.r3) * 2 + rows * a.r1 * 4;
+  const size_t z = a.dtype == 1 ? sk_z_stride<uint16_t>((int)a.r3) * sizeof(uint16_t)
+                                : sk_z_stride<float>((int)a.r3) * sizeof(float);
+  const size_t consumer = rows * z + rows * a.r1 * 4;
   return router > consumer ? router : consumer;
 }
 
@@ -704,14 +706,13 @@ __device__ __forceinline__ void route_row16(const FwdArgs& a, int64_t t, int sl,
   }
 }
 
-// GB: K groups a consumer wave's weight loads hold at once, issued before the wait: 2 where
-// K = 2048 gives each of the 16 waves two (K <= 1024: one). One token block (MF = 1) stays
+// GB: K groups (64 elements in bf16, 32 in fp32) a consumer wave's weight loads hold at
+// once, issued before the wait: 2 where K gives each of the 16 waves more than one. One token block (MF = 1) stays
 // within 64 registers, so that two work-groups fit a compute unit (d_out 4608: 356 of them).
-template <int MF, int W, int GB>
+template <class Elt, int MF, int W, int GB>
 __global__ __launch_bounds__(64 * W) void k_sk_decode(FwdArgs a) {
   static_assert(W == 16, "one 16-lane row per token of a 64-token block");
   constexpr int kGroups = MF;   // 4-column groups of z a thread holds: 16 MF tokens, r3 <= 256
-  typedef EltBF16 Elt;
   typedef typename Elt::T T;
   __shared__ float red[SkLds<MF, W>::kFloats];
   extern __shared__ u32x4 dynv[];

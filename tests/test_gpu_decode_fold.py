@@ -1,4 +1,4 @@
-"""Unfolded bf16 plans at decode sizes (T <= 64): one folded launch against the W^T packed
+"""Unfolded plans at decode sizes (T <= 64): one folded launch against the W^T packed
 beside the two-GEMM weights. Against the float64 oracle at the bf16 bar, at the edges of its
 token blocks and of the rule (K = rk r3 of 2048 in one and two weight groups a wave, W^T of
 32 MB), and no less exact than the two-GEMM form (both round c z and one 16-bit
@@ -93,3 +93,34 @@ def test_decode_fold_fp8(pkg, dev):
     want = onp.forward_f64(x, ref, k)
     assert np.array_equal(idx.cpu().numpy(), want["idx"])
     assert onp.rel_l2(out.float().cpu().numpy(), want["out"]) <= 1e-2
+
+
+# fp32: one and two weight groups a wave (K 512 and 1024), the expert form, r3 = 64 with a K
+# of 576 (groups that do not split evenly over the waves), ragged d_out
+@pytest.mark.parametrize("T", [1, 15, 32, 33, 64])
+@pytest.mark.parametrize("shape", [
+    (8, 2, 4, 128, 256, 512, 1024), (16, 2, 4, 256, 1024, 1536, 2304),
+    (8, 2, 32, 256, 512, 768, 768), (9, 3, 9, 64, 192, 320, 1040),
+], ids=str)
+def test_decode_fold_fp32(pkg, dev, shape, T):
+    E, k, r1, r3, r2, d_in, d_out = shape
+    w = pkg.Workload("custom", T, d_in, d_out, E, k, r1, r3, r2, torch.float32, 94)
+    params = pkg.synth.make_params(w, affine="random")
+    m = pkg.TuckerMoE(d_in, d_out, w.cfg()).to(dev, w.dtype)
+    m.load_state_dict({k_: v.to(dev) for k_, v in params.items()})
+    assert not m.plan().folded()
+    assert m.plan().forward_path(T) == pkg._lib.TMOE_PATH_DECODE
+    x = pkg.synth.make_x(w)
+    out, idx, wts, _ = _run(m, x.to(dev))
+    m.check_signals()
+    ref = onp.forward_f64(x, params, w.k)
+    err = onp.rel_l2(out.cpu().numpy(), ref["out"])
+    m.set_fold(False)
+    out2, idx2, wts2, _ = _run(m, x.to(dev))
+    err2 = onp.rel_l2(out2.cpu().numpy(), ref["out"])
+    print(f"{shape} T={T}: folded {err:.2e} two GEMMs {err2:.2e}", flush=True)
+    assert np.array_equal(idx.cpu().numpy(), ref["idx"]) and torch.equal(idx, idx2)
+    assert np.abs(wts.cpu().numpy() - ref["w"]).max() < 1e-5
+    # W^T is summed in fp64: no further from exact than the two GEMMs, but for the few
+    # elements of a single row (2304 values at most 10% apart by chance)
+    assert err <= 1e-5 and err2 <= 1e-5 and err <= 1.1 * err2
