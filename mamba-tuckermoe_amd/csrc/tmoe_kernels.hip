@@ -921,7 +921,8 @@ hipError_t latent_weights(const LatentArgs& l, float* w, hipStream_t st) {
   return hipGetLastError();
 }
 
-// The sort of the tokens by pair and (exp) of the entries by expert, in two launches.
+// The sort of the tokens by pair and (exp) of the entries by expert, in two launches;
+// without exp (the forward) the first also transposes G.
 hipError_t launch_latent_sort(const LatentArgs& l, const LatentLayout& L, bool pairs, bool exp,
                               hipStream_t st) {
   char* ws = static_cast<char*>(l.ws);
@@ -952,8 +953,14 @@ hipError_t launch_latent_sort(const LatentArgs& l, const LatentLayout& L, bool p
   q.order = reinterpret_cast<int*>(ws + L.order);
   q.pair_hist = reinterpret_cast<int*>(ws + L.pair_hist);
   q.exp_hist = reinterpret_cast<int*>(ws + L.exp_hist);
-  const dim3 grid(q.pair_blocks + q.exp_blocks), block(256);
-  hipLaunchKernelGGL(dev::k_latent_count, grid, block, 0, st, q);
+  // without the entries (the forward): G transposed beside the counts
+  const int64_t rows = l.E * l.r3, cols = l.r2;
+  const unsigned sort = q.pair_blocks + q.exp_blocks;
+  const unsigned transpose = exp ? 0 : (unsigned)((rows / 32) * (cols / 32));
+  const dim3 grid(sort), block(dev::kSortThreads);
+  hipLaunchKernelGGL(dev::k_latent_count, dim3(sort + transpose), block, 0, st, q,
+                     static_cast<const uint16_t*>(l.G), reinterpret_cast<uint16_t*>(ws + L.gt),
+                     rows, cols);
   if (hipError_t e = hipGetLastError(); e != hipSuccess) return e;
   hipLaunchKernelGGL(dev::k_latent_sort, grid, block, 0, st, q);
   return hipGetLastError();
@@ -1040,7 +1047,6 @@ hipError_t latent_forward(const LatentArgs& l, hipStream_t st) {
   float* w = reinterpret_cast<float*>(ws + L.w);
   hipError_t e;
   if (latent_pairs(l)) {
-    if ((e = launch_transpose(l.G, ws + L.gt, l.E * l.r3, l.r2, es, st)) != hipSuccess) return e;
     if ((e = launch_latent_sort(l, L, true, false, st)) != hipSuccess) return e;
     return l.k == 2 ? launch_latent_pair<2, false>(l, L, st) : launch_latent_pair<1, false>(l, L, st);
   }

@@ -83,7 +83,7 @@ __device__ __forceinline__ int wave_scan_excl(int v, int lane, int& total) {
 // order, the items by every thread. One launch whose work-groups each count every item
 // took 16 us for 16384 tokens, its LDS atomics most of it.
 // start[key] is the key's first place (start[nkeys] = n); emit(pos, i).
-constexpr int kSortSpan = 1024, kSortBlocks = 64, kSortBatch = 32;
+constexpr int kSortThreads = 256, kSortSpan = 1024, kSortBlocks = 64, kSortBatch = 16;
 __device__ __forceinline__ void sort_span(int64_t n, int blk, int nblk, int64_t& lo, int64_t& hi) {
   const int64_t span = ((n + (int64_t)nblk * 64 - 1) / ((int64_t)nblk * 64)) * 64;
   lo = blk * span < n ? blk * span : n;
@@ -105,66 +105,85 @@ template <class Key, class Emit>
 __device__ __forceinline__ void sort_range(int64_t n, int nkeys, int blk, int nblk, int* before,
                                            int* rest, int* start, int* span_buf, const int* hist,
                                            Key key, Emit emit) {
-  const int tid = threadIdx.x, lane = tid & 63, nt = (int)blockDim.x;
+  constexpr int kItems = kSortSpan / kSortThreads, kParts = kSortBlocks / kSortBatch;
+  const int tid = threadIdx.x, lane = tid & 63;
   int64_t lo, hi;
   sort_span(n, blk, nblk, lo, hi);
-  for (int i = tid; i < nkeys; i += nt) {
-    int bf = 0, rs = 0;
-    for (int r0 = 0; r0 < nblk; r0 += kSortBatch) {
-      int h[kSortBatch];
+  // a thread's items of a span: key and payload, loaded ahead of the places
+  int kk[kItems], pay[kItems];
+  auto load = [&](int64_t s0, int m) {
 #pragma unroll
-      for (int u = 0; u < kSortBatch; ++u)
-        h[u] = hist[(int64_t)(r0 + u < nblk ? r0 + u : nblk - 1) * nkeys + i];
-#pragma unroll
-      for (int u = 0; u < kSortBatch; ++u) {
-        bf += r0 + u < blk ? h[u] : 0;
-        rs += r0 + u >= blk && r0 + u < nblk ? h[u] : 0;
-      }
+    for (int u = 0; u < kItems; ++u) {
+      const int i = tid + u * kSortThreads;
+      if (i < m) kk[u] = key(s0 + i, pay[u]);
     }
-    before[i] = bf;
-    rest[i] = rs;
+  };
+  auto span_of = [&](int64_t s0) { return (int)(hi - s0 < kSortSpan ? hi - s0 : kSortSpan); };
+  if (lo < hi) load(lo, span_of(lo));
+  for (int i = tid; i < nkeys; i += kSortThreads) before[i] = rest[i] = 0;
+  __syncthreads();
+  for (int t = tid; t < nkeys * kParts; t += kSortThreads) {   // kSortBatch rows of one key
+    const int i = t % nkeys, r0 = t / nkeys * kSortBatch;
+    int h[kSortBatch];
+#pragma unroll
+    for (int u = 0; u < kSortBatch; ++u)
+      h[u] = hist[(int64_t)(r0 + u < nblk ? r0 + u : nblk - 1) * nkeys + i];
+    int bf = 0, rs = 0;
+#pragma unroll
+    for (int u = 0; u < kSortBatch; ++u) {
+      bf += r0 + u < blk ? h[u] : 0;
+      rs += r0 + u >= blk && r0 + u < nblk ? h[u] : 0;
+    }
+    if (bf) atomicAdd(before + i, bf);
+    if (rs) atomicAdd(rest + i, rs);
   }
   __syncthreads();
   if (tid < 64) {
     int carry = 0;
     for (int b = 0; b < nkeys; b += 64) {
-      const int kk = b + lane;
-      const int bf = kk < nkeys ? before[kk] : 0;
+      const int q = b + lane;
+      const int bf = q < nkeys ? before[q] : 0;
       int total;
-      const int ex = wave_scan_excl(kk < nkeys ? bf + rest[kk] : 0, lane, total) + carry;
-      if (kk < nkeys) {
-        start[kk] = ex;
-        before[kk] = ex + bf;   // the next place of this range's items
+      const int ex = wave_scan_excl(q < nkeys ? bf + rest[q] : 0, lane, total) + carry;
+      if (q < nkeys) {
+        start[q] = ex;
+        before[q] = ex + bf;   // the next place of this range's items
       }
       carry += total;
     }
     if (lane == 0) start[nkeys] = carry;
   }
   for (int64_t s0 = lo; s0 < hi; s0 += kSortSpan) {
-    const int m = (int)(hi - s0 < kSortSpan ? hi - s0 : kSortSpan);
-    for (int i = tid; i < m; i += nt) span_buf[i] = key(s0 + i);
+    const int m = span_of(s0);
+    if (s0 > lo) load(s0, m);
+#pragma unroll
+    for (int u = 0; u < kItems; ++u)
+      if (tid + u * kSortThreads < m) span_buf[tid + u * kSortThreads] = kk[u];
     __syncthreads();
     if (tid < 64) {
       volatile int* next = before;
       for (int b = 0; b < m; b += 64) {
         const bool valid = b + lane < m;
-        const int kk = valid ? span_buf[b + lane] : nkeys;
+        const int kv = valid ? span_buf[b + lane] : nkeys;
         uint64_t same = ~0ull;   // lanes with this lane's key
         for (int bit = 1; bit <= nkeys; bit <<= 1) {
-          const uint64_t q = __ballot((kk & bit) != 0);
-          same &= (kk & bit) ? q : ~q;
+          const uint64_t q = __ballot((kv & bit) != 0);
+          same &= (kv & bit) ? q : ~q;
         }
         const int rank = __popcll(same & ((1ull << lane) - 1));
         if (valid) {
-          const int pos = next[kk] + rank;
+          const int pos = next[kv] + rank;
           span_buf[b + lane] = pos;
-          if (rank == __popcll(same) - 1) next[kk] = pos + 1;
+          if (rank == __popcll(same) - 1) next[kv] = pos + 1;
         }
         __builtin_amdgcn_wave_barrier();
       }
     }
     __syncthreads();
-    for (int i = tid; i < m; i += nt) emit(span_buf[i], s0 + i);
+#pragma unroll
+    for (int u = 0; u < kItems; ++u)
+      if (tid + u * kSortThreads < m)
+        emit(span_buf[tid + u * kSortThreads], s0 + tid + u * kSortThreads, pay[u]);
     __syncthreads();
   }
 }
@@ -175,10 +194,11 @@ __device__ __forceinline__ int latent_pair_keys(const LatentSort& s) {
 __device__ __forceinline__ int latent_pair_key(const LatentSort& s, int lo, int hi) {
   return s.k == 2 ? lo * s.E - lo * (lo - 1) / 2 + (hi - lo) : lo;
 }
-__device__ __forceinline__ int latent_key_of(const LatentSort& s, int64_t b) {
+__device__ __forceinline__ int latent_key_of(const LatentSort& s, int64_t b, int& pay) {
   int lo, hi;
   bool sw;
   latent_pair_of(s, b, lo, hi, sw);
+  pay = (int)b | (sw ? kLatSwap : 0);
   return latent_pair_key(s, lo, hi);
 }
 // an entry's expert; those that select nothing come last (key E)
@@ -187,17 +207,36 @@ __device__ __forceinline__ int latent_exp_of(const LatentSort& s, int64_t i) {
   return e >= 0 && e < s.E ? (int)e : s.E;
 }
 
-__global__ __launch_bounds__(256) void k_latent_count(LatentSort s) {
+// The counts of both sorts; the work-groups past them transpose G (forward): GT (r2, E r3)
+// in 32 x 32 tiles.
+__global__ __launch_bounds__(kSortThreads) void k_latent_count(LatentSort s,
+                                                               const uint16_t* __restrict__ G,
+                                                               uint16_t* __restrict__ GT,
+                                                               int64_t rows, int64_t cols) {
   __shared__ int cnt[kLatMaxKeys];
+  const int tb = (int)blockIdx.x - s.pair_blocks - s.exp_blocks;
+  if (tb >= 0) {
+    uint16_t(*tile)[33] = reinterpret_cast<uint16_t(*)[33]>(cnt);
+    const int nc = (int)(cols / 32);   // rows and cols are multiples of 32
+    const int64_t r0 = (int64_t)(tb / nc) * 32, c0 = (int64_t)(tb % nc) * 32;
+    const int tx = threadIdx.x & 31, ty = threadIdx.x >> 5;
+    for (int y = ty; y < 32; y += 8) tile[y][tx] = G[(r0 + y) * cols + c0 + tx];
+    __syncthreads();
+    for (int y = ty; y < 32; y += 8) GT[(c0 + y) * rows + r0 + tx] = tile[tx][y];
+    return;
+  }
   if ((int)blockIdx.x < s.pair_blocks)
     count_keys(s.B, latent_pair_keys(s), (int)blockIdx.x, s.pair_blocks, cnt, s.pair_hist,
-               [&](int64_t b) { return latent_key_of(s, b); });
+               [&](int64_t b) {
+                 int pay;
+                 return latent_key_of(s, b, pay);
+               });
   else
     count_keys(s.B * s.k, s.E + 1, (int)blockIdx.x - s.pair_blocks, s.exp_blocks, cnt, s.exp_hist,
                [&](int64_t i) { return latent_exp_of(s, i); });
 }
 
-__global__ __launch_bounds__(256) void k_latent_sort(LatentSort s) {
+__global__ __launch_bounds__(kSortThreads) void k_latent_sort(LatentSort s) {
   __shared__ int before[kLatMaxKeys], rest[kLatMaxKeys], start[kLatMaxKeys + 1], buf[kSortSpan];
   const int tid = threadIdx.x, lane = tid & 63;
   if ((int)blockIdx.x < s.pair_blocks) {
@@ -205,13 +244,8 @@ __global__ __launch_bounds__(256) void k_latent_sort(LatentSort s) {
     auto key_of = [&](int lo, int hi) { return latent_pair_key(s, lo, hi); };
     sort_range(
         s.B, nkeys, (int)blockIdx.x, s.pair_blocks, before, rest, start, buf, s.pair_hist,
-        [&](int64_t b) { return latent_key_of(s, b); },
-        [&](int pos, int64_t b) {
-          int lo, hi;
-          bool sw;
-          latent_pair_of(s, b, lo, hi, sw);
-          s.order[pos] = (int)b | (sw ? kLatSwap : 0);
-        });
+        [&](int64_t b, int& pay) { return latent_key_of(s, b, pay); },
+        [&](int pos, int64_t, int pay) { s.order[pos] = pay; });
     if (blockIdx.x != 0) return;
     __syncthreads();
     if (tid < 64) {   // rest[key] = the key's first row tile
@@ -241,11 +275,14 @@ __global__ __launch_bounds__(256) void k_latent_sort(LatentSort s) {
   const int blk = (int)blockIdx.x - s.pair_blocks;
   sort_range(
       s.B * s.k, s.E + 1, blk, s.exp_blocks, before, rest, start, buf, s.exp_hist,
-      [&](int64_t i) { return latent_exp_of(s, i); },
-      [&](int pos, int64_t i) {
+      [&](int64_t i, int& pay) {
+        pay = __float_as_int(s.p_f32 ? static_cast<const float*>(s.p)[i]
+                                     : load_as_f32(static_cast<const uint16_t*>(s.p) + i));
+        return latent_exp_of(s, i);
+      },
+      [&](int pos, int64_t i, int pay) {
         s.etok[pos] = (int)(i / s.k);
-        s.ew[pos] = s.p_f32 ? static_cast<const float*>(s.p)[i]
-                            : load_as_f32(static_cast<const uint16_t*>(s.p) + i);
+        s.ew[pos] = __int_as_float(pay);
       });
   if (blk != 0) return;
   __syncthreads();
