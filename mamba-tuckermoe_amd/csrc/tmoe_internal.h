@@ -270,7 +270,7 @@ hipError_t launch_small_front_raw(const FwdArgs& a, hipStream_t stream);
 hipError_t launch_small_core_epi(const FwdArgs& a, hipStream_t stream);
 hipError_t launch_small_out_epi(const FwdArgs& a, hipStream_t stream);
 bool small_epi_fused_ok(const FwdArgs& a);
-// the whole small-T folded layer in one launch (k_sk_decode): bf16, T <= 64,
+// the whole small-T folded layer in one launch (k_sk_decode): bf16 or fp32, T <= 64,
 // T r3 <= 16384, E <= 16, r1 <= 32, r3 in {64, 128, 256}, sync words present, and
 // the stream not being captured
 bool small_decode_ok(const FwdArgs& a, hipStream_t stream);

@@ -216,13 +216,16 @@ int cu_count() {
   return n;
 }
 
-// k_outproj_wide / k_outproj_mid's contract: bf16, no column scale, no fused
-// epilogue, K a multiple of 64, whole 288- (144-) column tiles, A (mid) allocated
-// for T rounded up to 256 rows (the workspace rounds its tile rows to 256 for
-// these plans).
-bool outproj_tiled_ok(const FwdArgs& a) {
-  if (a.dtype != kDtypeBF16 || a.out_scale || a.epi_mode != kEpiNone) return false;
+// k_outproj_wide / k_outproj_mid's contract: bf16, no column scale, K a multiple of
+// 64, whole 288- (144-) column tiles, A (mid) allocated for T rounded up to 256 rows
+// (the workspace rounds its tile rows to 256 for these plans); outproj_tiled_ok: and
+// no fused epilogue (k_outproj_wide_glu has the GLU's).
+bool outproj_tiles_fit(const FwdArgs& a) {
+  if (a.dtype != kDtypeBF16 || a.out_scale) return false;
   return a.r2 % 64 == 0 && a.d_out % dev::wide::BN == 0 && a.mid_rows_256;
+}
+bool outproj_tiled_ok(const FwdArgs& a) {
+  return a.epi_mode == kEpiNone && outproj_tiles_fit(a);
 }
 
 // The out-projection's 128 x 144 tiles (k_outproj_mid) number at most the compute
@@ -293,6 +296,34 @@ hipError_t launch_outproj_bf16(const FwdArgs& a, hipStream_t st) {
     const dim3 grid((unsigned)(t128 < ncu ? t128 : ncu)), block(64 * C::WM * C::WN);
     hipLaunchKernelGGL((dev::k_outproj_pp<128, C::BN, C::WM, C::WN>), grid, block, 0, st, a);
     return hipGetLastError();
+  }
+  if (a.epi_mode == kEpiGlu && outproj_tiles_fit(a)) {
+    // The 288-column tiles with the GLU epilogue, where they need fewer rounds of the
+    // compute units than the 256 x 192 tiles below, or their 128-token form fits one.
+    // Measured at d_out = 4608, K = 512 (us; one round: 256 x 192 27, 256 x 288 33 to 35,
+    // 128 x 288 23): T = 2048 (1 round of 128 x 288) 26.9 -> 23.4; 2500 (1 : 1) 27.9
+    // against 32.5, not taken; 4096 (2 : 1) 52.0 -> 35.5; 5000 (2 : 2) 54.5 against 56.2,
+    // not taken; 8192 (3 : 2) 83.0 -> 67.7. At most half a round (above): 128 x 192 17,
+    // 128 x 288 20 to 21.
+    const int64_t ntn = a.d_out / dev::wide::BN;
+    const int64_t t128 = cdiv(a.T, dev::wide::Cfg<1>::BM) * ntn;
+    const int64_t t256 = cdiv(a.T, dev::wide::Cfg<2>::BM) * ntn;
+    const uint16_t* A = static_cast<const uint16_t*>(a.mid);
+    const uint16_t* Bt = static_cast<const uint16_t*>(a.uoutT);
+    const uint16_t* gate = static_cast<const uint16_t*>(a.epi_a);
+    uint16_t* out = static_cast<uint16_t*>(a.out);
+    const int T = (int)a.T, N = (int)a.d_out, K = (int)a.r2;
+    if (t128 <= ncu) {
+      hipLaunchKernelGGL(dev::k_outproj_wide_glu<1>, dim3((unsigned)t128), dim3(256), 0, st, A, Bt,
+                         out, gate, a.bias, T, N, K);
+      return hipGetLastError();
+    }
+    if (cdiv(t256, ncu) < cdiv(tiles, ncu)) {
+      const dim3 grid((unsigned)(t256 < ncu ? t256 : ncu));
+      hipLaunchKernelGGL(dev::k_outproj_wide_glu<2>, grid, dim3(256), 0, st, A, Bt, out, gate,
+                         a.bias, T, N, K);
+      return hipGetLastError();
+    }
   }
   const dim3 grid((unsigned)(tiles < ncu ? tiles : ncu)), block(64 * C::WM * C::WN);
   hipLaunchKernelGGL((dev::k_outproj_pp<C::BM, C::BN, C::WM, C::WN>), grid, block, 0, st, a);

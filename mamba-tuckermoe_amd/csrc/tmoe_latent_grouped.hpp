@@ -17,9 +17,9 @@
 //                    dp = the sum of its column tiles' parts
 //
 // Measured at 16384 tokens, E 8, k 2, r3 256, r2 1024 (kernel trace, MI355X), against the
-// dense kernels: forward 40 us + 12 us of sort (dense 71), dx and dp 43 (H 96, dx / dp 32),
-// dG 36 + xs 7 + planes 8 (dense 140 + transposes 37 + planes 6); a forward and backward
-// 343 -> 150 us.
+// dense kernels: forward 41 us (dense 71), dx and dp 44 (H 96, dx / dp 32), dG 37 + xs 7 +
+// planes 8 (dense 140 + transposes 37 + planes 6), the sort 12 in each direction (counts 5,
+// with the forward's transpose of G beside them); a forward and backward 346 -> 145 us.
 //
 // The sort is a stable counting sort on integers, so every sum has a fixed order. An
 // index outside [0, E) selects nothing (weight 0, dp 0).

@@ -29,10 +29,15 @@
 // holds a quarter of the A bytes it would otherwise (z instead of c (x) z), and
 // the 4x larger c (x) z is never written.
 //
+// GLU: the epilogue reads the gate's chunk for each chunk that a lane stores and stores
+// R(R(silu(gate)) y). Its 18.9M silu at T = 4096, d_out = 4608 are 8 us of vector
+// arithmetic (2 quarter-rate instructions each, one wave per SIMD) that nothing of the
+// same tile overlaps: 35.5 us (K = 512) against 26.9 without it and 52.0 for the 256 x 192
+// tiles of k_outproj_pp with the epilogue. Loads one block ahead instead of three: 38.6.
+//
 // Shape contract (checked by the host): K % 64 == 0, N % 288 == 0 (W^T rows
 // read in whole tiles), A (or z and c) allocated for T rounded up to 256 rows
-// (rows past T are read, their results never stored), no column scale and no
-// fused epilogue; KR: K = 4 * 256.
+// (rows past T are read, their results never stored), no column scale; KR: K = 4 * 256.
 #pragma once
 
 namespace tmoe {
@@ -118,13 +123,14 @@ __device__ __forceinline__ void wide_step(f32x16 (&acc)[FM][wide::FN], const u32
 // work-group. A (M rows, K), Bt (N rows, K), C (M, N) bf16 bits; bias (N) fp32.
 // KR: A is z (M rows, 256) and cr is c (M rows, 4 floats), K = 1024.
 // smem: 2 Cfg<FM>::kStage 16-byte slots of LDS.
-template <int FM_, class Sched, bool KR = false>
-__device__ __forceinline__ void wide_loop(const uint16_t* __restrict__ A,
-                                          const uint16_t* __restrict__ Bt,
-                                          uint16_t* __restrict__ C,
-                                          const float* __restrict__ bias, int M, int N, int K,
-                                          u32x4* smem, Sched& sched,
-                                          const float* __restrict__ cr = nullptr) {
+// GLU: C = R(R(silu(gate)) y), gate (M, N) possibly C itself.
+template <int FM_, class Sched, bool KR, bool GLU>
+__device__ __forceinline__ void wide_loop_any(const uint16_t* __restrict__ A,
+                                              const uint16_t* __restrict__ Bt, uint16_t* C,
+                                              const float* __restrict__ bias, int M, int N, int K,
+                                              u32x4* smem, Sched& sched,
+                                              const float* __restrict__ cr,
+                                              const uint16_t* gate) {
   using wide::FN;
   using wide::BN;
   using wide::kAgprBlk;
@@ -278,6 +284,27 @@ __device__ __forceinline__ void wide_loop(const uint16_t* __restrict__ A,
     int tm2 = tm, tn2 = tn;
     const bool has_next = sched.advance(tm2, tn2);
     const bool early = has_next && nkt > 1;
+    // GLU: the gate's 16-byte chunks of a 32-column block, each loaded by the lane
+    // that stores that chunk, kAhead - 1 blocks ahead (the first ones before the next tile's DMAs)
+    constexpr int kAhead = 4;
+    u32x4 ge[kAhead][FM][2];
+    auto load_gate = [&](int j) __attribute__((always_inline)) {
+      if constexpr (GLU) {
+        int ln = threadIdx.x & 63;
+        asm volatile("" : "+v"(ln));
+#pragma unroll
+        for (int i = 0; i < FM; ++i) {
+          // rows past M read the last row (never stored)
+          const int row = min(tm * BM + wave * (32 * FM) + i * 32 + (ln & 31), M - 1);
+          const uint16_t* g = gate + (int64_t)row * N + tn * BN + j * 32 + 8 * (ln >> 5);
+#pragma unroll
+          for (int p = 0; p < 2; ++p)
+            ge[j % kAhead][i][p] = *reinterpret_cast<const u32x4*>(g + 16 * p);
+        }
+      }
+    };
+#pragma unroll
+    for (int j = 0; j + 1 < kAhead; ++j) load_gate(j);
     // the next tile's c (every A fragment of this tile has been read): older than
     // its DMAs, so the counted waits below also cover it
     if (has_next) load_c(tm2);
@@ -300,6 +327,7 @@ __device__ __forceinline__ void wide_loop(const uint16_t* __restrict__ A,
       const bool hi = ln >= 32;
 #pragma unroll
       for (int j = 0; j < FN; ++j) {
+        if (j + kAhead - 1 < FN) load_gate(j + kAhead - 1);
         // the block's 32 bias values: uniform loads
         float bj[32];
         {
@@ -337,7 +365,18 @@ __device__ __forceinline__ void wide_loop(const uint16_t* __restrict__ A,
                                                                 false, false);
               const auto sy = __builtin_amdgcn_permlane32_swap(pk[2 * p][1], pk[2 * p + 1][1],
                                                                 false, false);
-              const u32x4 val = {sx[0], sy[0], sx[1], sy[1]};
+              u32x4 val = {sx[0], sy[0], sx[1], sy[1]};
+              if constexpr (GLU) {   // R(R(silu(g)) * y), as epi_value's
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                  const uint32_t g = ge[j % kAhead][i][p][e], y = val[e];
+                  const uint32_t sg = pack_bf16x2(silu_as(bf16_bits_to_f32(g & 0xffffu), EltBF16{}),
+                                                  silu_as(bf16_bits_to_f32(g >> 16), EltBF16{}));
+                  val[e] = pack_bf16x2(
+                      bf16_bits_to_f32(sg & 0xffffu) * bf16_bits_to_f32(y & 0xffffu),
+                      bf16_bits_to_f32(sg >> 16) * bf16_bits_to_f32(y >> 16));
+                }
+              }
               const int col = n0 + j * 32 + 16 * p + 8 * (ln >> 5);
               *reinterpret_cast<u32x4*>(C + (int64_t)row * N + col) = val;
             }
@@ -361,6 +400,16 @@ __device__ __forceinline__ void wide_loop(const uint16_t* __restrict__ A,
   }
 }
 
+
+template <int FM_, class Sched, bool KR = false>
+__device__ __forceinline__ void wide_loop(const uint16_t* __restrict__ A,
+                                          const uint16_t* __restrict__ Bt,
+                                          uint16_t* __restrict__ C,
+                                          const float* __restrict__ bias, int M, int N, int K,
+                                          u32x4* smem, Sched& sched,
+                                          const float* __restrict__ cr = nullptr) {
+  wide_loop_any<FM_, Sched, KR, false>(A, Bt, C, bias, M, N, K, smem, sched, cr, nullptr);
+}
 
 // Work-group b's tiles: b, b + grid, ... of the (M / BM) x (N / BN) tile grid, in
 // tile_coords_of's XCD-aware order.
@@ -407,6 +456,21 @@ __global__ __launch_bounds__(256) void k_outproj_wide_kr(const uint16_t* __restr
   __shared__ u32x4 smem[2 * Cf::kStage];
   WideGridSched sched{0, N / wide::BN, ((M + Cf::BM - 1) / Cf::BM) * (N / wide::BN)};
   wide_loop<FM_, WideGridSched, true>(Z, Bt, C, bias, M, N, K, smem, sched, c);
+}
+
+// The same GEMM through the kEpiGlu epilogue: C = R(R(silu(gate)) y), gate (M, N) read in
+// the epilogue; it may be C itself (each lane reads the chunks that it then writes).
+template <int FM_>
+__global__ __launch_bounds__(256) void k_outproj_wide_glu(const uint16_t* __restrict__ A,
+                                                          const uint16_t* __restrict__ Bt,
+                                                          uint16_t* C, const uint16_t* gate,
+                                                          const float* __restrict__ bias, int M,
+                                                          int N, int K) {
+  typedef wide::Cfg<FM_> Cf;
+  __shared__ u32x4 smem[2 * Cf::kStage];
+  WideGridSched sched{0, N / wide::BN, ((M + Cf::BM - 1) / Cf::BM) * (N / wide::BN)};
+  wide_loop_any<FM_, WideGridSched, false, true>(A, Bt, C, bias, M, N, K, smem, sched, nullptr,
+                                                 gate);
 }
 
 #undef TMOE_MFMA_A
