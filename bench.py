@@ -285,10 +285,14 @@ def bench_latent(args) -> None:
     torch.cuda.synchronize()
     ms = ev0.elapsed_time(ev1) / args.steps
     algo = 8.0 * T * k * r3 * r2          # out, dx, dp, dG: 2 T k r3 r2 each
-    executed = 2.0 * T * r3 * r2 * E * 3  # dense over E: forward, H, dG
+    # forward, the product of dx and dp, dG: over each token's k experts where the grouped
+    # kernels run (latent_pairs in tmoe_kernels.hip; their tiles' padding not counted), else
+    # dense over E
+    grouped = 13 * (T + E * (E + 1) // 2 * 64) * k <= 10 * T * E
+    executed = 2.0 * T * r3 * r2 * (k if grouped else E) * 3
     peak = PEAK_TFLOPS["bf16"]
     log(f"[bench-latent] T={T}: {ms * 1e3:.1f} us per forward+backward; "
-        f"{executed / (ms * 1e-3) / 1e12:.0f} TFLOP/s executed (dense over E)")
+        f"{executed / (ms * 1e-3) / 1e12:.0f} TFLOP/s executed ({'by expert' if grouped else 'dense over E'})")
     print(json.dumps({
         "metric": LATENT_METRIC, "value": T / (ms * 1e-3), "unit": "tokens/s", "n_gpus": 1,
         "steps": args.steps, "warmup": args.warmup, "ms_per_step": ms, "higher_is_better": True,
@@ -480,7 +484,8 @@ def measure(pkg, w, args, *, steps, warmup, rotate_mb, no_fold, no_fuse, cpu, la
     rk = plan.core_rank()
     path = plan.forward_path(T)
     form = ("folded: c (x) z against W = core U_out, one GEMM of width %d" % (rk * w.r3)
-            if folded else "two GEMMs: core (rank %d) then U_out" % rk)
+            if folded or path == pkg._lib.TMOE_PATH_DECODE
+            else "two GEMMs: core (rank %d) then U_out" % rk)
     log(f"[{label}] plan form: {form}; kernels: {pkg._lib.PATH_NAMES.get(path, path)}")
     ws_bytes = plan.workspace_bytes(T)
     set_bytes = T * w.d_in * es + T * w.d_out * es + ws_bytes + packed0.numel()
@@ -537,7 +542,8 @@ def measure(pkg, w, args, *, steps, warmup, rotate_mb, no_fold, no_fuse, cpu, la
         pkg._lib.prof_enable(False)
     stage_avg_us = {n: stage_ms[j] / calls * 1e3 for j, n in enumerate(pkg._lib.STAGE_NAMES)}
     fl_algo = w.flops()
-    fl = w.flops_executed(T, rk, folded)        # the dominant kernel's own work
+    # the dominant kernel's own work; the decode launch is folded in any plan
+    fl = w.flops_executed(T, rk, folded or path == pkg._lib.TMOE_PATH_DECODE)
     fl["front"] = fl["router"] + fl["in_proj"]   # one kernel computes both
     kr = path == pkg._lib.TMOE_PATH_LARGE_KR
     sb = (w.stage_bytes_kr(T, rk) if kr else

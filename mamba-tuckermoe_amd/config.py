@@ -103,16 +103,17 @@ class Workload:
 
     def stage_bytes_folded(self, T: Optional[int] = None, rk: Optional[int] = None) -> dict:
         """stage_bytes of a folded plan: the core stage reads z and c and writes
-        c (x) z (T, rk*r3); the out-projection reads it and W^T (d_out, rk*r3) bf16.
+        c (x) z (T, rk*r3); the out-projection reads it and W^T (d_out, rk*r3), in the dtype.
         Where the front writes c (x) z itself (no z, no core kernel) these bytes stay
         attributed to the core stage; the front's and out-projection's figures are
         those of the split kernels."""
         T = self.T if T is None else T
         rk = self.r1 if rk is None else rk
         st = self.stage_bytes(T)
+        es = 4 if self.dtype == torch.float32 else 2
         K = rk * self.r3
-        st["core"] = T * self.r3 * 2 + T * rk * 4 + T * K * 2
-        st["out_proj"] = T * K * 2 + self.d_out * K * 2 + 4 * self.d_out + T * self.d_out * 2
+        st["core"] = T * self.r3 * es + T * rk * 4 + T * K * es
+        st["out_proj"] = T * K * es + self.d_out * K * es + 4 * self.d_out + T * self.d_out * es
         return st
 
     def stage_bytes_kr(self, T: Optional[int] = None, rk: Optional[int] = None) -> dict:
@@ -131,9 +132,13 @@ class Workload:
 
     def one_launch(self, T: int, rk: int, folded: bool) -> bool:
         """Whether a forward of T tokens is the library's single decode launch
-        (k_sk_decode; the selection rule of small_decode_ok in tmoe_kernels.hip,
-        outside graph capture)."""
-        return (folded and self.dtype == torch.bfloat16 and 0 < T <= 64 and self.E <= 16
+        (k_sk_decode; the selection rule of small_decode_ok in tmoe_kernels.hip and, for
+        plans not folded at other T, decode_fold_ok in tmoe_internal.h; outside graph
+        capture, folding not switched off)."""
+        es = 4 if self.dtype == torch.float32 else 2
+        K = rk * self.r3
+        fits = K <= 2048 and K * self.d_out * es <= 32 << 20
+        return ((folded or fits) and 0 < T <= 64 and self.E <= 16
                 and self.r3 in (64, 128, 256) and rk <= 32)
 
     def layer_bytes_folded(self, T: Optional[int] = None, rk: Optional[int] = None) -> int:
@@ -146,7 +151,7 @@ class Workload:
         es = 4 if self.dtype == torch.float32 else 2
         K = rk * self.r3
         return (st["front"] - T * self.r3 * es - T * self.r1 * 4
-                + st["out_proj"] - T * K * 2 + T * rk * 4)
+                + st["out_proj"] - T * K * es + T * rk * 4)
 
     def hbm_bytes(self, T: Optional[int] = None) -> int:
         """Compulsory HBM bytes per forward: x in, out, every weight once (fp8
