@@ -137,7 +137,12 @@ int tmoe_plan_folded(const tmoe_plan* plan);
  * other, re-pack from the parameters. */
 int tmoe_packed_layout_version(void);
 
-/* Bytes of device workspace tmoe_forward needs for T tokens (T >= 0). */
+/* Bytes of device workspace tmoe_forward wants for T tokens (T >= 0). Not monotone in
+ * T: at some T the fastest form holds extra partial sums. tmoe_forward,
+ * tmoe_forward_epi and tmoe_forward_glu also take a smaller workspace that holds T's
+ * form without them (fp32 without K slices; at 64 < T <= 256 the bf16 form of fewer
+ * bytes), which is slower and whose sums are in another order; only a workspace too
+ * small for that is TMOE_EINVAL. */
 size_t tmoe_workspace_bytes(const tmoe_plan* plan, int64_t T);
 
 /* Re-lays the module parameters into the kernels' operand layouts.
@@ -180,7 +185,7 @@ int tmoe_pack_weights_fp8(const tmoe_plan* plan, const void* router_w,
  *   topk_w   (T, k) f32, nullable: the routing weights (mode 0: softmax over the k
  *            selected logits, model.py:77)
  *   logits   (T, E) f32, nullable: router scores x @ router_w^T (model.py:75)
- *   workspace of at least tmoe_workspace_bytes(plan, T) bytes. Its contents need
+ *   workspace of tmoe_workspace_bytes(plan, T) bytes (or fewer, see there). Its contents need
  *            no initialisation: kernels whose work-groups hand data to each other
  *            inside one launch (the T <= 64 decode launch, the E = 256 front,
  *            the one-launch large-T forward) tag their signal words with a value
@@ -233,8 +238,8 @@ int tmoe_forward_epi(const tmoe_plan* plan, const void* x, int64_t T, const void
  * serving loops, harnesses that forbid hipMalloc): the forward's workspace is a
  * static device array of tmoe_static_scratch_bytes() bytes (48 MiB: T up to 16384
  * at the reference's C3 shape) that each GPU the library runs on holds until the
- * process ends; this call allocates nothing. T whose workspace
- * (tmoe_workspace_bytes) exceeds it gives TMOE_EUNSUPPORTED before any GPU work.
+ * process ends; this call allocates nothing. T none of whose forms fits it (see
+ * tmoe_workspace_bytes) gives TMOE_EUNSUPPORTED before any GPU work.
  * All calls on one GPU share that GPU's array: calls that overlap on one GPU (on
  * different streams, or from different threads without ordering) race. The array
  * used is that of the device `stream` belongs to (the current device for the null

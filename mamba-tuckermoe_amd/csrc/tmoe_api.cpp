@@ -139,7 +139,7 @@ bool batch_folded(const tmoe_plan* p, int64_t T) {
 }
 
 // lean: without the fp32 plans' K slices (their planes) and without folded batches, for a
-// caller whose scratch does not hold them.
+// workspace that does not hold them (fit_layout).
 Layout workspace_layout(const tmoe_plan* p, int64_t T, bool lean = false) {
   Layout L{};
   const bool batch = !lean && batch_folded(p, T);
@@ -203,6 +203,16 @@ Layout workspace_layout(const tmoe_plan* p, int64_t T, bool lean = false) {
                          sizeof(uint32_t));
   L.total = o;
   return L;
+}
+
+// The layout of a forward of T tokens in `bytes` of workspace: the full one where it fits,
+// else the lean one (whose total may still exceed `bytes`). A folded batch or the fp32
+// planes take more than a larger T's forward does (fp32 1536 -> 6144: 22.4 MB at T = 2048,
+// 12.2 at 4097), so that a workspace sized for the largest T of a program need not hold
+// every smaller T's full layout.
+Layout fit_layout(const tmoe_plan* p, int64_t T, size_t bytes) {
+  const Layout L = workspace_layout(p, T);
+  return bytes < L.total ? workspace_layout(p, T, true) : L;
 }
 
 // The kernels' arguments for one forward of plan p (epilogue fields unset).
@@ -627,7 +637,7 @@ namespace {
 int forward_impl(const tmoe_plan* p, const void* x, int64_t T, const void* packed, void* out,
                  int32_t* topk_idx, float* topk_w, float* logits, void* workspace,
                  size_t workspace_bytes, int epi_mode, const void* epi_a, const void* epi_b,
-                 void* stream, bool prof_ok, bool lean = false) {
+                 void* stream, bool prof_ok) {
   if (!p) return fail(TMOE_EINVAL, "tmoe_forward: null plan");
   if (epi_mode != TMOE_EPI_NONE && epi_mode != TMOE_EPI_GLU && epi_mode != TMOE_EPI_RESIDUAL_SCALE)
     return fail(TMOE_EINVAL, "tmoe_forward_epi: epi_mode %d is not a TMOE_EPI_* value", epi_mode);
@@ -643,7 +653,7 @@ int forward_impl(const tmoe_plan* p, const void* x, int64_t T, const void* packe
     return fail(TMOE_EINVAL, "tmoe_forward: null x/packed/out/workspace");
   if (!aligned16(x) || !aligned16(packed) || !aligned16(workspace) || !aligned16(out))
     return fail(TMOE_EINVAL, "tmoe_forward: x/packed/out/workspace must be 16-byte aligned");
-  const Layout L = workspace_layout(p, T, lean);
+  const Layout L = fit_layout(p, T, workspace_bytes);
   if (workspace_bytes < L.total)
     return fail(TMOE_EINVAL, "tmoe_forward: workspace of %zu bytes, %zu needed for T=%lld",
                 workspace_bytes, L.total, (long long)T);
@@ -733,9 +743,7 @@ int tmoe_forward_static(const tmoe_plan* p, const void* x, int64_t T, const void
     return fail(TMOE_EUNSUPPORTED, "tmoe_forward_static: T=%lld too large", (long long)T);
   if (T == 0) return TMOE_OK;
   // every check that needs no GPU comes before the scratch lookup
-  size_t need = workspace_layout(p, T).total;
-  const bool lean = need > tmoe::kStaticScratchBytes;
-  if (lean) need = workspace_layout(p, T, true).total;
+  const size_t need = fit_layout(p, T, tmoe::kStaticScratchBytes).total;
   if (need > tmoe::kStaticScratchBytes)
     return fail(TMOE_EUNSUPPORTED,
                 "tmoe_forward_static: T=%lld needs %zu bytes of scratch, more than the static "
@@ -748,8 +756,7 @@ int tmoe_forward_static(const tmoe_plan* p, const void* x, int64_t T, const void
   if (hipError_t e = tmoe::static_scratch(static_cast<hipStream_t>(stream), &ws); e != hipSuccess)
     return hip_fail(e, "tmoe_forward_static: static scratch address");
   return forward_impl(p, x, T, packed, out, topk_idx, topk_w, logits, ws,
-                      tmoe::kStaticScratchBytes, TMOE_EPI_NONE, nullptr, nullptr, stream, false,
-                      lean);
+                      tmoe::kStaticScratchBytes, TMOE_EPI_NONE, nullptr, nullptr, stream, false);
 }
 
 int tmoe_forward_glu(const tmoe_plan* p, const void* x, int64_t T, const void* packed_gate,
@@ -767,7 +774,7 @@ int tmoe_forward_glu(const tmoe_plan* p, const void* x, int64_t T, const void* p
       !aligned16(ws_gate) || !aligned16(ws_up))
     return fail(TMOE_EINVAL, "tmoe_forward_glu: pointers must be 16-byte aligned");
   if (ws_gate == ws_up) return fail(TMOE_EINVAL, "tmoe_forward_glu: the two workspaces coincide");
-  const Layout L = workspace_layout(p, T);
+  const Layout L = fit_layout(p, T, workspace_bytes);
   if (workspace_bytes < L.total)
     return fail(TMOE_EINVAL, "tmoe_forward_glu: workspaces of %zu bytes, %zu needed for T=%lld",
                 workspace_bytes, L.total, (long long)T);
