@@ -33,7 +33,7 @@
 extern "C" {
 #endif
 
-#define TMOE_ABI_VERSION 12
+#define TMOE_ABI_VERSION 13
 
 /* error codes */
 #define TMOE_OK            0
@@ -254,7 +254,8 @@ int tmoe_forward_static(const tmoe_plan* plan, const void* x, int64_t T, const v
  * current device (on a machine without a GPU: as on a 256-compute-unit MI355X).
  * No counterpart in the reference; for measurement tools, which attribute time
  * per kernel. Returns one of TMOE_PATH_* (0 for T == 0) or a negative error. */
-#define TMOE_PATH_SMALL  1  /* T <= 256: skinny kernels, two or three launches        */
+#define TMOE_PATH_SMALL  1  /* T <= 256: two to four launches (skinny kernels, or a
+                               folded batch: tmoe_forward_form)                         */
 #define TMOE_PATH_DECODE 2  /* T <= 64: the whole layer in one folded launch            */
 #define TMOE_PATH_LARGE  3  /* front, (core or c (x) z), out-projection launches      */
 #define TMOE_PATH_FUSED  4  /* large T, folded: the whole layer in one launch         */
@@ -264,6 +265,15 @@ int tmoe_forward_static(const tmoe_plan* plan, const void* x, int64_t T, const v
                                 E <= 32: the whole layer in one launch (K-sliced front and
                                 128 x 144 out-projection tiles)                          */
 int tmoe_forward_path(const tmoe_plan* plan, int64_t T);
+
+/* What an eager tmoe_forward of T tokens with a full workspace contracts, as
+ * tmoe_forward_path: TMOE_FORM_* bits (0 for T == 0) or a negative error. */
+#define TMOE_FORM_FOLDED       1  /* c (x) z against W = core U_out (at any T of a folded
+                                     plan; at some T <= 256 of others)                  */
+#define TMOE_FORM_BATCH        2  /* a folded batch, 64 < T <= 256: the front's epilogue
+                                     writes c (x) z, then one GEMM (in K slices)        */
+#define TMOE_FORM_FRONT_SLICED 4  /* the front runs in K slices                         */
+int tmoe_forward_form(const tmoe_plan* plan, int64_t T);
 
 /* Lost in-launch signals. No counterpart in the reference (its forward has no
  * kernels that wait for each other; torch raises its errors from the call).

@@ -21,7 +21,7 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(HERE, "libtmoe.so")
 NATIVE_PATH = os.path.join(HERE, "_tmoe_native.so")
 
-ABI_VERSION = 12
+ABI_VERSION = 13
 TMOE_OK, TMOE_EINVAL, TMOE_EUNSUPPORTED, TMOE_EHIP, TMOE_ESIGNAL = 0, -1, -2, -3, -4
 TMOE_F32, TMOE_BF16, TMOE_BF16_FP8W = 0, 1, 2
 TMOE_ROUTER_SOFTMAX_TOPK, TMOE_ROUTER_CAPPED = 0, 1
@@ -32,6 +32,7 @@ TMOE_STATUS_SIGNAL = 1
 TMOE_PATH_SMALL, TMOE_PATH_DECODE, TMOE_PATH_LARGE, TMOE_PATH_FUSED = 1, 2, 3, 4
 TMOE_PATH_LARGE_KR = 5
 TMOE_PATH_FUSED_MID = 6
+TMOE_FORM_FOLDED, TMOE_FORM_BATCH, TMOE_FORM_FRONT_SLICED = 1, 2, 4
 PATH_NAMES = {1: "small-T kernels", 2: "one launch (k_sk_decode)",
               3: "front + out-projection launches", 4: "one launch (k_fused_large)",
               5: "front (z, c) + out-projection forming c (x) z (k_outproj_wide_kr)",
@@ -50,6 +51,7 @@ EXPORTED = (
     "tmoe_static_scratch_bytes", "tmoe_forward_static",
     "tmoe_latent_workspace_bytes", "tmoe_latent_forward", "tmoe_latent_backward",
     "tmoe_signal_status", "tmoe_set_wait_polls", "tmoe_forward_path",
+    "tmoe_forward_form",
     "tmoe_prof_enable", "tmoe_prof_read",
 )
 
@@ -141,6 +143,8 @@ def lib() -> ctypes.CDLL:
         L.tmoe_signal_status.argtypes = [vp, ctypes.c_int, ctypes.POINTER(ctypes.c_uint32)]
         L.tmoe_forward_path.restype = ctypes.c_int
         L.tmoe_forward_path.argtypes = [vp, i64]
+        L.tmoe_forward_form.restype = ctypes.c_int
+        L.tmoe_forward_form.argtypes = [vp, i64]
         L.tmoe_set_wait_polls.restype = ctypes.c_int64
         L.tmoe_set_wait_polls.argtypes = [i64]
         L.tmoe_prof_enable.restype = ctypes.c_int
@@ -246,6 +250,10 @@ class Plan:
     def forward_path(self, T: int) -> int:
         """TMOE_PATH_* of an eager forward of T tokens on the current device."""
         return check(lib().tmoe_forward_path(self._ptr, int(T)))
+
+    def forward_form(self, T: int) -> int:
+        """TMOE_FORM_* bits of an eager forward of T tokens on the current device."""
+        return check(lib().tmoe_forward_form(self._ptr, int(T)))
 
     def signal_status(self, clear: bool = True) -> int:
         """The TMOE_STATUS_* bits that completed kernels of this plan's forwards set

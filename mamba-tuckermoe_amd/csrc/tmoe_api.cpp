@@ -928,6 +928,15 @@ int tmoe_forward_path(const tmoe_plan* p, int64_t T) {
   return TMOE_PATH_LARGE;
 }
 
+int tmoe_forward_form(const tmoe_plan* p, int64_t T) {
+  const int path = tmoe_forward_path(p, T);
+  if (path <= 0) return path;
+  const Layout L = workspace_layout(p, T);
+  const bool batch = batch_folded(p, T);
+  return (p->fold || batch || path == TMOE_PATH_DECODE ? TMOE_FORM_FOLDED : 0) |
+         (batch ? TMOE_FORM_BATCH : 0) | (L.fsplit > 1 ? TMOE_FORM_FRONT_SLICED : 0);
+}
+
 int tmoe_signal_status(const tmoe_plan* plan, int clear, uint32_t* mask) {
   g_err[0] = 0;
   if (mask) *mask = 0;

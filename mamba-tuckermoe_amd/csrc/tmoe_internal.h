@@ -130,6 +130,8 @@ constexpr int kEpiNone = 0, kEpiGlu = 1, kEpiResScale = 2;
 // C3 shapes (folded): T = 256 takes 42.8 us there against 49.4 us on the large-tile
 // kernels (49 us for any T from 96 up), T = 512 59.0 us against 41-43 us.
 constexpr int64_t kSmallT = 256;
+// ... and up to kDecodeMaxT the one-launch decode kernel where it can (small_decode_ok)
+constexpr int64_t kDecodeMaxT = 64;
 
 // k_core_pp (the persistent core for bf16 plans): ranks r1 in {1, 2, 4}, r1 * r2 a
 // multiple of its 256-row tiles, and for fp8 weights at most kCorePScales channel
@@ -151,6 +153,7 @@ inline bool core_p_grouped(int64_t r1) { return r1 > 4; }
 constexpr int64_t raw_stride(int64_t r3, int64_t E) { return r3 + (E + 3) / 4 * 4; }
 constexpr int64_t kFrontMinKTiles = 16;
 constexpr int64_t kFrontSliceKTiles = 3;
+constexpr int64_t kBatchSliceKTiles = 24, kBatchSliceKTilesWide = 40;
 constexpr int kMaxFrontPlanes = 8;
 constexpr int64_t kFrontXcds = 8, kFrontGroupsPerXcd = 32;
 // Tokens of a K-sliced front tile: 64 in bf16; 32 in fp32, whose MFMAs bound the slice
@@ -161,12 +164,18 @@ constexpr int64_t front_slice_rows(int64_t es) { return es == 2 ? 64 : 32; }
 inline int front_split(int64_t T, int64_t d_in, int64_t E_pad, int64_t es) {
   // E_pad = 256 measured slower sliced (C4: front 44.6 us against 34.8 us for the
   // split z / router front plus 7.7 us of k_expand_cz)
-  if (T <= 64 || E_pad > 128) return 1;
+  if (T <= kDecodeMaxT || E_pad > 128) return 1;
   const int64_t rows = front_slice_rows(es);
   const int64_t tiles = (T + rows - 1) / rows, nkt = d_in * es / 128;
   // measured at d_in = 1536, bf16: slices win up to T = 4096 (64 tiles); at 128 tiles
   // the 32-token front is faster
   if (T > 4096 || nkt < kFrontMinKTiles) return 1;
+  // a folded batch (T <= kSmallT) has the skinny front instead, and few slices leave the
+  // per-token epilogues few work-groups. Layer, us, at T = 65..256, unsliced : sliced, K 1024,
+  // d_out 256: E_pad 32: d_in 1024 21.0 : 23.2, 1152 to 1408 equal, 1536 23.4 : 20.9, 3072
+  // 29.7 : 22.7; E_pad 64: 1024 21.7 : 26.2, 1536 24.0 : 23.0; E_pad 128 (d_out 2304): 1024
+  // 22.5 : 30.0, 1536 24.9 : 26.1, 2560 28.8 : 28.7, 3072 31.3 : 29.3
+  if (T <= kSmallT && nkt < (E_pad > 64 ? kBatchSliceKTilesWide : kBatchSliceKTiles)) return 1;
   int64_t s = kFrontGroupsPerXcd / ((tiles + kFrontXcds - 1) / kFrontXcds);
   if (s > nkt / kFrontSliceKTiles) s = nkt / kFrontSliceKTiles;
   if (s > kMaxFrontPlanes) s = kMaxFrontPlanes;
@@ -275,7 +284,6 @@ bool small_epi_fused_ok(const FwdArgs& a);
 // the stream not being captured
 bool small_decode_ok(const FwdArgs& a, hipStream_t stream);
 hipError_t launch_small_decode(const FwdArgs& a, hipStream_t stream);
-constexpr int64_t kDecodeMaxT = 64;
 // Unfolded plans whose decode-size batches (T <= kDecodeMaxT) still run folded, in
 // that one launch, against a W^T packed beside the two-GEMM weights: K = rk r3 of at most
 // 2048 (two K groups a consumer wave) and W^T of at most 32 MB (read whole by every
