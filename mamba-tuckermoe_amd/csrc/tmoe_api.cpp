@@ -132,10 +132,13 @@ struct Layout {
   int osplit;   // FwdArgs::out_split
 };
 
-// Whether a forward of T tokens is a folded batch (tmoe::batch_out_split).
+// Whether a forward of T tokens is a folded batch (tmoe::kBatchFoldTiles).
 bool batch_folded(const tmoe_plan* p, int64_t T) {
   if (p->kdtype != TMOE_BF16 || T <= tmoe::kDecodeMaxT || T > tmoe::kSmallT) return false;
-  return p->fold || (p->decode_fold && tmoe::batch_out_tiles(T, p->s.d_out) <= tmoe::kBatchFoldTiles);
+  if (p->fold)
+    return tmoe::batch_fold_pays(T, p->s.d_out, p->rk * p->s.r3,
+                                 tmoe::front_split(T, p->s.d_in, p->E_pad, p->es));
+  return p->decode_fold && tmoe::batch_out_tiles(T, p->s.d_out) <= tmoe::kBatchFoldTiles;
 }
 
 // lean: without the fp32 plans' K slices (their planes) and without folded batches, for a

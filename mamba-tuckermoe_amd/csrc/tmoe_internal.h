@@ -219,7 +219,7 @@ inline bool core_p_supported(int64_t r1, int64_t r2, bool bf16, bool fp8w) {
 }
 
 // Folded batches between the decode launch and the large-tile kernels (kDecodeMaxT < T <=
-// kSmallT): folded plans, and plans with decode_fold's W^T whose 64 x 128 out-projection tiles
+// kSmallT): folded plans (batch_fold_pays), and plans with decode_fold's W^T whose 64 x 128 out-projection tiles
 // number at most kBatchFoldTiles (one a compute unit; past it the fold's extra multiply-adds,
 // 3 times as many at the reference's 1536 -> 6144, outweigh the core's launches). The front's
 // per-token epilogue writes c (x) z; the out-projection is a plain GEMM of it against W^T, K
@@ -238,6 +238,19 @@ inline int batch_out_split(int64_t T, int64_t d_out, int64_t K) {
   if (s > K / 256) s = K / 256;
   if (s > kMaxOutSlices) s = kMaxOutSlices;
   return s > 1 ? (int)s : 1;
+}
+// Whether a plan folded at every T takes the folded batch instead of the skinny
+// out-projection that forms c (x) z in registers (k_sk_out), both behind the skinny front.
+// That one needs no pass over K slices, and its time goes by its rounds of 16-column work-
+// groups over blocks of 64 tokens (one a compute unit) and by K. Layer, us, skinny : batch at
+// d_in 768: one round (d_out 768, 64 < T <= 256) 19.5 : 19.4-20.3 at K 1024, 17 : 19.5 at K 512,
+// 29 : 19.5 at K 2048; K of one slice 15.5 : 15; two rounds (d_out 2304) T = 65 19.5 : 19.9, 72
+// 19.9 : 20.0, 80 20.9 : 20.4, 128 27 : 21.5, 256 35 : 23; 4096 columns, T = 65 23.5 : 21.7
+// (its second round is full). Where the batch slices the front it is faster at any of these.
+inline bool batch_fold_pays(int64_t T, int64_t d_out, int64_t K, int front_slices) {
+  if (front_slices > 1 || K > 1024 || batch_out_split(T, d_out, K) == 1) return true;
+  const int64_t cols = (d_out + 15) / 16, blocks = (T + 63) / 64, last = T - 64 * (blocks - 1);
+  return cols * blocks > kCoreUnits && (last >= 16 || cols * (blocks - 1) >= kCoreUnits);
 }
 
 // The latent expert contraction of the training module (tmoe_latent.hpp) and its

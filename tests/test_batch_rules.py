@@ -23,3 +23,39 @@ def test_batch_front_slices(pkg, E, d_in, sliced):
         assert bool(_form(pkg, T, d_in=d_in, d_out=4096, E=E) & S) == sliced, T
     assert bool(_form(pkg, 257, d_in=d_in, d_out=4096, E=E) & S) == (E <= 128)
     assert not _form(pkg, 64, d_in=d_in, d_out=4096, E=E) & S
+
+
+# a folded plan takes the batch form (d_out, K = r1 r3, T): in one round of the skinny
+# out-projection's work-groups not, unless K is past 1024 or of one slice; in two rounds from
+# 16 tokens in the last block of 64 on, or where the blocks before it fill the chip
+@pytest.mark.parametrize("d_out,r1,r3,T,batch", [
+    (768, 4, 256, 65, False), (768, 4, 256, 256, False), (1024, 4, 256, 256, False),
+    (1040, 4, 256, 256, True), (1040, 4, 256, 192, False), (1040, 4, 256, 207, False),
+    (1040, 4, 256, 208, True), (2048, 4, 256, 128, False), (2064, 4, 256, 79, False),
+    (2064, 4, 256, 80, True), (4080, 4, 256, 65, False), (4096, 4, 256, 65, True),
+    (768, 2, 256, 128, False), (768, 4, 128, 128, False), (768, 1, 256, 65, True),
+    (768, 4, 64, 256, True),
+])
+def test_folded_plan_batches(pkg, d_out, r1, r3, T, batch):
+    f = pkg._lib
+    got = _form(pkg, T, d_in=768, d_out=d_out, r1=r1, r3=r3)
+    assert got & f.TMOE_FORM_FOLDED and bool(got & f.TMOE_FORM_BATCH) == batch
+    # behind a sliced front, and past K of 1024
+    assert _form(pkg, T, d_in=1536, d_out=d_out, r1=r1, r3=r3) & f.TMOE_FORM_BATCH
+    assert not _form(pkg, 64, d_in=768, d_out=d_out, r1=r1, r3=r3) & f.TMOE_FORM_BATCH
+    assert not _form(pkg, 257, d_in=768, d_out=d_out, r1=r1, r3=r3) & f.TMOE_FORM_BATCH
+
+
+def test_other_batches(pkg):
+    """K past 1024 of a folded plan; unfolded plans up to 256 tiles of 64 x 128; fp32 and
+    NO_FOLD never."""
+    f = pkg._lib
+    both = f.TMOE_FORM_FOLDED | f.TMOE_FORM_BATCH
+    assert _form(pkg, 65, d_in=768, d_out=64, r1=32, r2=512) == both     # folded, K 2048
+    for T in (65, 193, 256):
+        assert _form(pkg, T, d_in=768, d_out=768, r1=32, r2=512) == both
+        assert _form(pkg, T, d_in=768, d_out=768, r1=32, r2=512, dtype=torch.float32) == 0
+        assert _form(pkg, T, d_in=768, d_out=768, r1=32, r2=512, flags=f.TMOE_FLAG_NO_FOLD) == 0
+    shape = dict(d_in=256, d_out=10880, r1=8, r2=64, r3=64)
+    assert _form(pkg, 192, **shape) == both and _form(pkg, 193, **shape) == 0
+    assert _form(pkg, 64, **shape) == f.TMOE_FORM_FOLDED and _form(pkg, 0, **shape) == 0

@@ -1,5 +1,5 @@
 """Folded bf16 batches between the decode launch and the large-tile kernels: 64 < T <= 256,
-for unfolded plans while the 64 x 128 out-projection tiles number at most 256. Against
+where they pay (test_batch_rules.py has the rules), for unfolded plans while the 64 x 128 out-projection tiles number at most 256. Against
 the float64 oracle at the bf16 bar, at the edges of the token and column tiles, of the rule
 and of the K slices (1, several, 8), with each front (small, K-sliced, plain), the fused
 epilogues of the sub-blocks, fp8 weights and under graph capture."""
@@ -46,28 +46,33 @@ def _check(m, x, dev, ref, k):
     return out
 
 
-# (E, k, r1, r3, r2, d_in, d_out) and T: folded with a sliced and with the small front, a wide
-# router, a ragged last column tile; the reference's ranks at the smallest T, one row past a
-# tile, the last T of the range and the first past it; 256 tiles and past them (the two
-# GEMMs); rank 4 unfolded; K = 64 (one slice)
-@pytest.mark.parametrize("shape,Ts", [
-    ((16, 2, 4, 256, 1024, 1536, 2304), (65, 129, 200, 256)),
-    ((64, 4, 4, 256, 1024, 512, 304), (65, 255)),
-    ((8, 2, 32, 256, 512, 768, 768), (65, 193, 256, 257)),
-    ((8, 2, 32, 256, 512, 1536, 6144), (128, 255)),
-    ((8, 2, 4, 256, 512, 768, 4608), (129, 250)),
-    ((8, 2, 8, 256, 256, 256, 8192), (192, 193, 256)), ((8, 2, 8, 64, 64, 256, 10880), (192, 193)),
-    ((4, 1, 1, 64, 256, 256, 64), (70, 256)),
+# (E, k, r1, r3, r2, d_in, d_out), the T's that run as a folded batch, and T's on the other side
+# of a rule's edge: folded with a sliced and with the small front, a wide router, a ragged last
+# column tile; folded in one round of the skinny out-projection (no batch); the reference's
+# ranks at the smallest T, one row past a tile, the last T of the range and the first past it;
+# 256 tiles and past them (the two GEMMs); rank 4 unfolded; K = 64 (one slice)
+@pytest.mark.parametrize("shape,Ts,others", [
+    ((16, 2, 4, 256, 1024, 1536, 2304), (65, 129, 200, 256), (64, 257)),
+    ((64, 4, 4, 256, 1024, 512, 2320), (80, 255), (65, 79)),
+    ((64, 4, 4, 256, 1024, 512, 304), (), (65, 255)),
+    ((8, 2, 32, 256, 512, 768, 768), (65, 193, 256), (257,)),
+    ((8, 2, 32, 256, 512, 1536, 6144), (128, 255), ()),
+    ((8, 2, 4, 256, 512, 768, 4608), (129, 250), ()),
+    ((8, 2, 8, 256, 256, 256, 8192), (192, 193, 256), ()),
+    ((8, 2, 8, 64, 64, 256, 10880), (192,), (193,)),
+    ((4, 1, 1, 64, 256, 256, 64), (70, 256), ()),
 ], ids=lambda v: str(v))
-def test_batch_fold(pkg, dev, shape, Ts):
-    for T in Ts:
+def test_batch_fold(pkg, dev, shape, Ts, others):
+    for T in Ts + others:
         w, ref, m, x = _layer(pkg, dev, shape, T)
+        assert bool(m.plan().forward_form(T) & pkg._lib.TMOE_FORM_BATCH) == (T in Ts), T
         _check(m, x, dev, ref, w.k)
 
 
 def test_batch_fold_fp8(pkg, dev):
     for shape in ((16, 2, 4, 256, 1024, 1536, 2304), (8, 2, 4, 256, 512, 768, 4608)):
         w, ref, m, x = _layer(pkg, dev, shape, 100, fp8=True)
+        assert m.plan().forward_form(100) & pkg._lib.TMOE_FORM_BATCH
         _check(m, x, dev, ref, w.k)
 
 
@@ -75,6 +80,8 @@ def test_batch_fold_capture_and_flags(pkg, dev):
     """Captured (the K-sliced front's two launches) and without in-launch signals: the same
     bits; set_fold(False) keeps the two GEMMs."""
     w, ref, m, x = _layer(pkg, dev, (8, 2, 32, 256, 512, 1536, 768), 150)
+    assert m.plan().forward_form(150) == (pkg._lib.TMOE_FORM_FOLDED | pkg._lib.TMOE_FORM_BATCH |
+                                          pkg._lib.TMOE_FORM_FRONT_SLICED)
     out = _check(m, x, dev, ref, w.k)
     xs = x.to(dev)
     g = torch.cuda.CUDAGraph()
