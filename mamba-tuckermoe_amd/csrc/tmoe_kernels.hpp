@@ -118,7 +118,9 @@ struct RowLoader {          // plain row-major, K-contiguous operand
 // A operand of the core GEMM: A[t, r*r3 + s] = c[t, r] * z[t, s], rounded to the
 // operand type. A K tile never straddles two r blocks (r3 is a multiple of the
 // tile's element count).
-template <class Elt>
+// kSliced: the loop's K tile 0 is tile kt0 (a K slice); a template, since the addition alone
+// cost the unsliced bf16 core 3 to 5% (16384 x 1024, K 2048: 63 -> 66 us).
+template <class Elt, bool kSliced>
 struct KhatriRaoLoader {
   struct Raw {
     u32x4 v;
@@ -129,11 +131,11 @@ struct KhatriRaoLoader {
   const float* c;           // first row of the tile, (., r1)
   int r1, r3;
   int rows_valid;
-  int kt0;                  // the K tile that the loop calls 0 (K slices)
+  int kt0;
   __device__ __forceinline__ Raw fetch(int row, int ch, int kt) const {
     constexpr int kTileK = kTileKBytes / (int)sizeof(typename Elt::T);
     const int r = row < rows_valid ? row : rows_valid - 1;
-    const int k0 = (kt0 + kt) * kTileK;
+    const int k0 = (kSliced ? kt0 + kt : kt) * kTileK;
     const int rr = k0 / r3;
     const int s0 = k0 - rr * r3;
     Raw o;
@@ -1728,13 +1730,15 @@ __global__ __launch_bounds__(64 * WM * WN) void k_core(FwdArgs a) {
   const int rows_valid = (int)(a.T - m0 < BM ? a.T - m0 : BM);
   const int64_t K = a.r1 * a.r3;
   const int64_t b_row_bytes = K * (int64_t)sizeof(T);
-  // K slice sl of S = gridDim.y (fp32 plans, whose scales CoreRescale does not need): its
-  // plane of mpart takes the place of mid
-  const int S = (int)gridDim.y, sl = (int)blockIdx.y;
+  // fp32: K slice sl of S = gridDim.y (these plans have no scales for CoreRescale); its plane
+  // of mpart takes the place of mid
+  constexpr bool kSliced = std::is_same<Elt, EltF32>::value;
+  const int S = kSliced ? (int)gridDim.y : 1, sl = kSliced ? (int)blockIdx.y : 0;
   const int nkt = (int)(b_row_bytes / kTileKBytes);
-  const int kt0 = sl * nkt / S, kt1 = (sl + 1) * nkt / S;
-  KhatriRaoLoader<Elt> al{reinterpret_cast<const char*>(a.z) + m0 * a.r3 * (int64_t)sizeof(T),
-                          a.c + m0 * a.r1, (int)a.r1, (int)a.r3, rows_valid, kt0};
+  const int kt0 = kSliced ? sl * nkt / S : 0, kt1 = kSliced ? (sl + 1) * nkt / S : nkt;
+  KhatriRaoLoader<Elt, kSliced> al{
+      reinterpret_cast<const char*>(a.z) + m0 * a.r3 * (int64_t)sizeof(T), a.c + m0 * a.r1,
+      (int)a.r1, (int)a.r3, rows_valid, kt0};
   RowLoader bl{reinterpret_cast<const char*>(a.coreT) + n0 * b_row_bytes +
                    (int64_t)kt0 * kTileKBytes,
                b_row_bytes, (int)(a.r2 - n0)};
