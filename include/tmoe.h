@@ -335,6 +335,14 @@ int tmoe_rmsnorm_rows(const void* x, int64_t T, int64_t d, const void* weight, f
 #define TMOE_LATENT_P_F32 0x100
 size_t tmoe_latent_workspace_bytes(int64_t B, int64_t E, int64_t r3, int64_t r2, int dtype,
                                    int backward);
+/* Which kernels a call of these sizes runs (on a machine without a GPU: as on a
+ * 256-compute-unit MI355X): TMOE_LATENT_* bits, 0 where every product is dense over the
+ * experts, or a negative error. */
+#define TMOE_LATENT_PAIRS 1  /* tokens grouped by their pair of experts (the forward, or
+                                dx and dp with backward != 0)                          */
+#define TMOE_LATENT_DG    2  /* backward: dG over each expert's own entries            */
+int tmoe_latent_form(int64_t B, int64_t E, int64_t k, int64_t r3, int64_t r2, int dtype,
+                     int backward);
 int tmoe_latent_forward(const void* x, const void* G, const int64_t* idx, const void* p,
                         int64_t B, int64_t E, int64_t k, int64_t r3, int64_t r2, int dtype,
                         void* out, void* workspace, size_t workspace_bytes, void* stream);

@@ -37,6 +37,7 @@ PATH_NAMES = {1: "small-T kernels", 2: "one launch (k_sk_decode)",
               3: "front + out-projection launches", 4: "one launch (k_fused_large)",
               5: "front (z, c) + out-projection forming c (x) z (k_outproj_wide_kr)",
               6: "one launch (k_fused_mid)"}
+TMOE_LATENT_PAIRS, TMOE_LATENT_DG = 1, 2
 TMOE_LATENT_P_F32 = 0x100   # or'ed into a latent call's dtype: p and dp are fp32
 N_STAGES = 3
 STAGE_NAMES = ("front", "core", "out_proj")
@@ -49,7 +50,8 @@ EXPORTED = (
     "tmoe_pack_weights", "tmoe_pack_weights_fp8",
     "tmoe_forward", "tmoe_forward_epi", "tmoe_forward_glu", "tmoe_rmsnorm_rows",
     "tmoe_static_scratch_bytes", "tmoe_forward_static",
-    "tmoe_latent_workspace_bytes", "tmoe_latent_forward", "tmoe_latent_backward",
+    "tmoe_latent_workspace_bytes", "tmoe_latent_form", "tmoe_latent_forward",
+    "tmoe_latent_backward",
     "tmoe_signal_status", "tmoe_set_wait_polls", "tmoe_forward_path",
     "tmoe_forward_form",
     "tmoe_prof_enable", "tmoe_prof_read",
@@ -133,6 +135,8 @@ def lib() -> ctypes.CDLL:
         L.tmoe_rmsnorm_rows.argtypes = [vp, i64, i64, vp, ctypes.c_float, ctypes.c_int, vp, vp]
         L.tmoe_latent_workspace_bytes.restype = sz
         L.tmoe_latent_workspace_bytes.argtypes = [i64, i64, i64, i64, ctypes.c_int, ctypes.c_int]
+        L.tmoe_latent_form.restype = ctypes.c_int
+        L.tmoe_latent_form.argtypes = [i64, i64, i64, i64, i64, ctypes.c_int, ctypes.c_int]
         L.tmoe_latent_forward.restype = ctypes.c_int
         L.tmoe_latent_forward.argtypes = [vp, vp, vp, vp, i64, i64, i64, i64, i64, ctypes.c_int,
                                           vp, vp, sz, vp]

@@ -851,6 +851,16 @@ size_t tmoe_latent_workspace_bytes(int64_t B, int64_t E, int64_t r3, int64_t r2,
   return tmoe::latent_workspace_bytes(B, E, r3, r2, dtype == TMOE_BF16 ? 2 : 4, backward != 0);
 }
 
+int tmoe_latent_form(int64_t B, int64_t E, int64_t k, int64_t r3, int64_t r2, int dtype,
+                     int backward) {
+  g_err[0] = 0;
+  dtype &= ~TMOE_LATENT_P_F32;
+  if (int rc = latent_check("tmoe_latent_form", B, E, k, r3, r2, dtype)) return rc;
+  tmoe::LatentArgs l{};
+  l.dtype = dtype; l.B = B; l.E = E; l.k = k; l.r3 = r3; l.r2 = r2;
+  return B == 0 ? 0 : tmoe::latent_form(l, backward != 0);
+}
+
 int tmoe_latent_forward(const void* x, const void* G, const int64_t* idx, const void* p,
                         int64_t B, int64_t E, int64_t k, int64_t r3, int64_t r2, int dtype,
                         void* out, void* workspace, size_t workspace_bytes, void* stream) {

@@ -274,6 +274,8 @@ struct LatentArgs {
 // Workspace bytes of latent_forward (backward = false) or latent_backward.
 size_t latent_workspace_bytes(int64_t B, int64_t E, int64_t r3, int64_t r2, int es,
                               bool backward);
+// TMOE_LATENT_* bits of what latent_forward / latent_backward run for l's sizes and dtype.
+int latent_form(const LatentArgs& l, bool backward);
 hipError_t latent_forward(const LatentArgs& l, hipStream_t stream);
 hipError_t latent_backward(const LatentArgs& l, hipStream_t stream);
 

@@ -866,7 +866,7 @@ constexpr int kDgBM = 128, kDgBN = 128;
 bool latent_grouped_shape(int64_t E, int64_t r3, int64_t r2) {
   return r3 % 128 == 0 && r2 % 128 == 0 && E <= dev::kLatMaxE;
 }
-// Forward and dx / dp by pairs of experts: k <= 2, and the row tiles' products (each of
+// dx / dp (and the forward, latent_pairs_forward) by pairs of experts: k <= 2, and the row tiles' products (each of
 // the E (E + 1) / 2 pairs pads half a tile on average) well below the dense form's E per
 // token. The grouped kernels reach about 0.45 of the dense ones' rate (420 against 970
 // TFLOP/s forward at 16384 tokens) but skip dx / dp's pass over H, so the line is drawn at
@@ -875,6 +875,29 @@ bool latent_pairs(const LatentArgs& l) {
   if (l.dtype != kDtypeBF16 || l.k > 2 || !latent_grouped_shape(l.E, l.r3, l.r2)) return false;
   const int64_t keys = l.k == 2 ? l.E * (l.E + 1) / 2 : l.E;
   return 13 * (l.B + keys * (dev::kLatBM / 2)) * l.k <= 10 * l.B * l.E;
+}
+// The forward has no pass over H to skip, so that it also weighs its own two forms, in us
+// fitted to 326 measured pairs (E 2 to 16, k 1 and 2, ranks 128 and 256 x 128 to 2048, 64 to 65536
+// tokens; the dense fit within 10%, the grouped one within 17%, the slower form taken by more
+// than 3% in four cases): the dense one by its rounds of 256 x 256 tiles and its K, the grouped
+// one by its padded rows. dense : grouped at 16384 and 32768 tokens: E 2, k 1, 256 x 1024 31 : 34 and
+// 51 : 49, 128 x 512 19 : 24 and 23 : 31; E 3, k 2, 256 x 1024 40 : 44 and 66 : 72; E 4, k 2, 256 x 1024
+// 46 : 45 and 80 : 72, 128 x 512 25 : 26 and 29 : 38; E 8, k 2, 256 x 1024 71 : 47 and 130 : 75.
+bool latent_pairs_forward(const LatentArgs& l) {
+  if (!latent_pairs(l)) return false;
+  const int64_t keys = l.k == 2 ? l.E * (l.E + 1) / 2 : l.E, ncu = cu_count();
+  const int64_t tiles = (int64_t)cdiv(l.B, CoreCfgBF16::BM) * cdiv(l.r2, CoreCfgBF16::BN);
+  const double K = (double)(l.E * l.r3), out = (double)l.B * l.r2;
+  // a round that leaves half of the compute units idle runs its tiles faster
+  const double dense = 9 + 0.39e-6 * out +
+                       (2 * tiles <= ncu ? 2.7 + 0.0235 * K
+                                         : (double)cdiv(tiles, ncu) * (1.2 + 0.0266 * K));
+  const double rows = (double)(l.B + keys * (dev::kLatBM / 2)), cols = (double)(l.k * l.r2);
+  // an output past the last-level cache: its rows are stored in 128-byte pieces
+  const double spill = out * 2 > 134e6 ? 0.6e-6 * (out * 2 - 134e6) : 0;
+  const double grouped =
+      14.3 + rows * (0.18e-3 + cols * (0.24e-6 + 2.4e-9 * (double)l.r3)) + spill;
+  return grouped <= dense;
 }
 // dG over each expert's own entries: below the dense form's B E rows.
 bool latent_dg_grouped(const LatentArgs& l) {
@@ -1066,6 +1089,11 @@ hipError_t latent_dg_by_expert(const LatentArgs& l, const LatentLayout& L, bool 
 
 }  // namespace
 
+int latent_form(const LatentArgs& l, bool bwd) {
+  if (!bwd) return latent_pairs_forward(l) ? 1 : 0;
+  return (latent_pairs(l) ? 1 : 0) | (latent_dg_grouped(l) ? 2 : 0);
+}
+
 size_t latent_workspace_bytes(int64_t B, int64_t E, int64_t r3, int64_t r2, int es, bool bwd) {
   return latent_layout(B, E, r3, r2, es, bwd).total;
 }
@@ -1077,7 +1105,7 @@ hipError_t latent_forward(const LatentArgs& l, hipStream_t st) {
   char* ws = static_cast<char*>(l.ws);
   float* w = reinterpret_cast<float*>(ws + L.w);
   hipError_t e;
-  if (latent_pairs(l)) {
+  if (latent_pairs_forward(l)) {
     if ((e = launch_latent_sort(l, L, true, false, st)) != hipSuccess) return e;
     return l.k == 2 ? launch_latent_pair<2, false>(l, L, st) : launch_latent_pair<1, false>(l, L, st);
   }
