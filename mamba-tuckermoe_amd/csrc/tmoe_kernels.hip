@@ -861,6 +861,7 @@ struct LatentLayout {
 };
 
 constexpr int kDgBM = 128, kDgBN = 128;
+constexpr int64_t kLatMinChunk = 256;   // entries of a dG chunk, but for an expert's rest
 
 // Shapes of the grouped kernels: 128-wide tiles of both ranks, at most 64 experts.
 bool latent_grouped_shape(int64_t E, int64_t r3, int64_t r2) {
@@ -940,10 +941,14 @@ LatentLayout latent_layout(int64_t B, int64_t E, int64_t r3, int64_t r2, int es,
     L.tiles = o; o = al256(o + (size_t)L.max_tiles * 16);
     if (bwd) {
       // chunks of entries (chunk_target full ones, and a rest per expert): at most two
-      // work-groups a compute unit over all their tiles, one round of the chip
-      const int64_t per = (r3 / 128) * (r2 / 128);
+      // work-groups a compute unit over all their tiles, one round of the chip. A chunk has
+      // at least kLatMinChunk entries, so that a small B has few planes (E 8, 256 x 1024, B 256:
+      // 14 of them, 14 MB, where the chip's share is 32); kg: the most slots a token has where
+      // dG is grouped (latent_dg_grouped)
+      const int64_t per = (r3 / 128) * (r2 / 128), kg = kmax < 4 * E / 5 ? kmax : 4 * E / 5;
+      const int64_t n = B * kg, full = n / kLatMinChunk, rest = E < n ? E : n;
       L.chunk_target = (int)(512 / per > E ? 512 / per - E : 1);
-      L.max_chunks = L.chunk_target + E;
+      L.max_chunks = (L.chunk_target < full ? L.chunk_target : full) + rest;
       L.xs = L.h;   // (B k, r3) with k <= E: no larger than H
       L.etok = o; o = al256(o + (size_t)B * kmax * 4);
       L.ew = o; o = al256(o + (size_t)B * kmax * 4);
@@ -995,7 +1000,7 @@ hipError_t launch_latent_sort(const LatentArgs& l, const LatentLayout& L, bool p
   q.exp_blocks = exp ? blocks(l.B * l.k) : 0;
   if (exp) {
     const int64_t c = cdiv(l.B * l.k, L.chunk_target);
-    q.chunk = (int)(c < 256 ? 256 : c);
+    q.chunk = (int)(c < kLatMinChunk ? kLatMinChunk : c);
     q.max_chunks = (int)L.max_chunks;
     q.chunks = reinterpret_cast<int4*>(ws + L.chunks);
     q.exp_chunks = reinterpret_cast<int2*>(ws + L.exp_chunks);

@@ -82,3 +82,35 @@ def test_grouped_is_deterministic(pkg, dev):
     a, b = _check(pkg, dev, *args), _check(pkg, dev, *args)
     for n in a:
         assert torch.equal(a[n], b[n]), n
+
+
+@pytest.mark.parametrize("E,k,r3,r2,counts", [
+    (5, 4, 128, 128, (257, 257, 257, 257, 260)),        # every expert a full chunk and a rest
+    (8, 2, 128, 128, (1, 1, 1, 1, 1, 1, 1, 1)),         # rests only
+    (8, 2, 256, 256, (4096, 1, 1, 1, 1, 1, 1, 2098)),   # few long ones
+], ids=str)
+def test_backward_stays_in_its_workspace(pkg, dev, E, k, r3, r2, counts):
+    """Expert loads with the most dG chunks that the workspace's planes are counted for: the
+    bytes past it stay as they were, dG is right."""
+    f, n = pkg._lib, sum(counts)
+    B = n // k
+    assert B * k == n
+    flat = torch.repeat_interleave(torch.arange(E), torch.tensor(counts))
+    idx = flat[torch.randperm(n, generator=torch.Generator().manual_seed(1))].reshape(B, k)
+    x, G, _, _, dout = _inputs(B, E, k, r3, r2, 11, True)
+    p = torch.rand(B, k, generator=torch.Generator().manual_seed(2))
+    dt = f.TMOE_BF16 | f.TMOE_LATENT_P_F32
+    L = f.lib()
+    assert L.tmoe_latent_form(B, E, k, r3, r2, dt, 1) & f.TMOE_LATENT_DG
+    nbytes = L.tmoe_latent_workspace_bytes(B, E, r3, r2, dt, 1)
+    ws = torch.full((nbytes + 65536,), 0xA5, dtype=torch.uint8, device=dev)
+    xs, Gs, i, ps, d = (t.to(dev) for t in (x, G, idx, p, dout))
+    dx, dG, dp = torch.empty_like(xs), torch.empty_like(Gs), torch.empty_like(ps)
+    f.check(L.tmoe_latent_backward(
+        xs.data_ptr(), Gs.data_ptr(), i.data_ptr(), ps.data_ptr(), d.data_ptr(), B, E, k, r3, r2,
+        dt, dx.data_ptr(), dG.data_ptr(), dp.data_ptr(), ws.data_ptr(), nbytes,
+        torch.cuda.current_stream().cuda_stream))
+    torch.cuda.synchronize()
+    assert bool((ws[nbytes:] == 0xA5).all())
+    for got, ref in zip((dx, dG, dp), ln.backward(x, G, idx, p, dout)):
+        assert onp.rel_l2(got.float().cpu().numpy(), ref) <= 1e-2

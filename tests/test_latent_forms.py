@@ -38,3 +38,13 @@ def test_latent_forms(pkg, E, k, r3, r2, B, fwd, pairs, dg):
 def test_latent_form_rejects(pkg):
     assert _form(pkg, 64, 8, 9, 256, 1024, False) == pkg._lib.TMOE_EINVAL
     assert _form(pkg, 64, 65, 2, 256, 1024, True) == pkg._lib.TMOE_EUNSUPPORTED
+
+
+def test_backward_workspace_follows_B(pkg):
+    """The grouped dG's planes (one (r3, r2) fp32 plane per 256 entries and one per expert) are
+    sized by the tokens, not by the chip: 1 MB each here."""
+    f = pkg._lib.lib().tmoe_latent_workspace_bytes
+    by_B = [f(B, 8, 256, 1024, pkg._lib.TMOE_BF16, 1) for B in (1, 64, 256, 1024, 4096, 16384)]
+    assert by_B == sorted(by_B)
+    assert by_B[0] < 9 << 20 and by_B[2] < 18 << 20   # 33 MB with the chip's 32 planes
+    assert f(64, 2, 256, 1024, pkg._lib.TMOE_BF16, 1) < 5 << 20
