@@ -201,7 +201,9 @@ int tmoe_pack_weights_fp8(const tmoe_plan* plan, const void* router_w,
  * T == 0 is a no-op. Stream-ordered, no allocation, no host synchronisation. Under
  * HIP graph capture the kernels whose signal flags have several consumers are not
  * used (their flags would read as already set on a replay): decode-size batches,
- * the large-T forward and the E = 256 front take their multi-launch paths. */
+ * the large-T forward and the E = 256 front take their multi-launch paths. For the
+ * decode launch of a plan that is not folded at other T (tmoe_plan_folded == 0) that
+ * path is the same kernel in two launches and gives the same bits. */
 int tmoe_forward(const tmoe_plan* plan, const void* x, int64_t T, const void* packed,
                  void* out, int32_t* topk_idx, float* topk_w, float* logits,
                  void* workspace, size_t workspace_bytes, void* stream);

@@ -300,7 +300,7 @@ tmoe::FwdArgs folded_args(const tmoe_plan* p, const tmoe::FwdArgs& a, const void
 }
 
 // The arguments of the folded one-launch forward of a plan that is not folded
-// otherwise (decode_fold); the caller checks T and small_decode_ok.
+// otherwise (decode_fold); the caller checks T and small_decode_shape_ok.
 tmoe::FwdArgs decode_fold_args(const tmoe_plan* p, const tmoe::FwdArgs& a, const void* packed) {
   tmoe::FwdArgs f = a;
   f.r2 = p->rk * p->s.r3;
@@ -327,12 +327,19 @@ void small_stages(const tmoe_plan* p, const void* packed, tmoe::FwdArgs& a, hipS
     st[2] = tmoe::launch_outproj;
     return;
   }
-  bool decode = fold && tmoe::small_decode_ok(a, stream);
   if (p->decode_fold && a.T <= tmoe::kDecodeMaxT) {
+    // captured or not, the same form: in one launch, or its two halves under capture
     const tmoe::FwdArgs f = decode_fold_args(p, a, packed);
-    if ((decode = tmoe::small_decode_ok(f, stream))) a = f;
+    if (tmoe::small_decode_shape_ok(f)) {
+      a = f;
+      const bool one = tmoe::small_decode_ok(a, stream);
+      st[0] = one ? tmoe::launch_small_decode : tmoe::launch_small_decode_front;
+      st[1] = launch_nothing;
+      st[2] = one ? launch_nothing : tmoe::launch_small_decode_out;
+      return;
+    }
   }
-  if (decode) {   // one launch
+  if (fold && tmoe::small_decode_ok(a, stream)) {   // one launch
     st[0] = tmoe::launch_small_decode;
     st[1] = launch_nothing;
     st[2] = launch_nothing;

@@ -299,6 +299,10 @@ bool small_epi_fused_ok(const FwdArgs& a);
 // the stream not being captured
 bool small_decode_ok(const FwdArgs& a, hipStream_t stream);
 hipError_t launch_small_decode(const FwdArgs& a, hipStream_t stream);
+// its two halves, a launch each (no flags: graph capture), bit for bit the same; shapes as
+// small_decode_shape_ok
+hipError_t launch_small_decode_front(const FwdArgs& a, hipStream_t stream);
+hipError_t launch_small_decode_out(const FwdArgs& a, hipStream_t stream);
 // Unfolded plans whose decode-size batches (T <= kDecodeMaxT) still run folded, in
 // that one launch, against a W^T packed beside the two-GEMM weights: K = rk r3 of at most
 // 2048 (two K groups a consumer wave) and W^T of at most 32 MB (read whole by every

@@ -497,32 +497,47 @@ bool small_decode_ok(const FwdArgs& a, hipStream_t st) {
   return small_decode_shape_ok(a) && !stream_capturing(st);
 }
 
-template <class Elt, int MF>
+template <class Elt, int MF, int kPart>
 hipError_t launch_small_decode_t(const FwdArgs& a, hipStream_t st) {
   FwdArgs b = a;
-  b.epoch = next_epoch();
-  const dim3 grid((unsigned)((a.r3 / 16 + 1) * dev::kDecodeRowGroups + cdiv(a.d_out, 16))),
-      block(64 * kSkW);
+  if (kPart == dev::kDecodeAll) b.epoch = next_epoch();
+  const unsigned producers = (unsigned)((a.r3 / 16 + 1) * dev::kDecodeRowGroups);
+  const dim3 block(64 * kSkW), grid((kPart != dev::kDecodeConsumers ? producers : 0) +
+                                    (kPart != dev::kDecodeProducers ? cdiv(a.d_out, 16) : 0));
   const size_t dyn = dev::sk_decode_dyn_bytes(MF, a);
-  if (a.r1 * a.r3 * (int64_t)sizeof(typename Elt::T) > 2048)   // over one K group a wave
-    hipLaunchKernelGGL((dev::k_sk_decode<Elt, MF, kSkW, 2>), grid, block, dyn, st, b);
+  if (kPart != dev::kDecodeProducers &&
+      a.r1 * a.r3 * (int64_t)sizeof(typename Elt::T) > 2048)   // over one K group a wave
+    hipLaunchKernelGGL((dev::k_sk_decode<Elt, MF, kSkW, 2, kPart>), grid, block, dyn, st, b);
   else
-    hipLaunchKernelGGL((dev::k_sk_decode<Elt, MF, kSkW, 1>), grid, block, dyn, st, b);
+    hipLaunchKernelGGL((dev::k_sk_decode<Elt, MF, kSkW, 1, kPart>), grid, block, dyn, st, b);
   return hipGetLastError();
 }
 
-template <class Elt>
+template <class Elt, int kPart>
 hipError_t launch_small_decode_e(const FwdArgs& a, hipStream_t st) {
+  // a producer has at most 16 tokens at any T
+  if constexpr (kPart == dev::kDecodeProducers) return launch_small_decode_t<Elt, 1, kPart>(a, st);
   switch (small_mf(a.T)) {
-    case 1: return launch_small_decode_t<Elt, 1>(a, st);
-    case 2: return launch_small_decode_t<Elt, 2>(a, st);
-    default: return launch_small_decode_t<Elt, 4>(a, st);
+    case 1: return launch_small_decode_t<Elt, 1, kPart>(a, st);
+    case 2: return launch_small_decode_t<Elt, 2, kPart>(a, st);
+    default: return launch_small_decode_t<Elt, 4, kPart>(a, st);
   }
 }
 
+template <int kPart>
+hipError_t launch_small_decode_p(const FwdArgs& a, hipStream_t st) {
+  return a.dtype == kDtypeBF16 ? launch_small_decode_e<EltBF16, kPart>(a, st)
+                               : launch_small_decode_e<EltF32, kPart>(a, st);
+}
+
 hipError_t launch_small_decode(const FwdArgs& a, hipStream_t st) {
-  return a.dtype == kDtypeBF16 ? launch_small_decode_e<EltBF16>(a, st)
-                               : launch_small_decode_e<EltF32>(a, st);
+  return launch_small_decode_p<dev::kDecodeAll>(a, st);
+}
+hipError_t launch_small_decode_front(const FwdArgs& a, hipStream_t st) {
+  return launch_small_decode_p<dev::kDecodeProducers>(a, st);
+}
+hipError_t launch_small_decode_out(const FwdArgs& a, hipStream_t st) {
+  return launch_small_decode_p<dev::kDecodeConsumers>(a, st);
 }
 
 hipError_t launch_front_pair(const FwdArgs& a0, const FwdArgs& a1, hipStream_t st) {

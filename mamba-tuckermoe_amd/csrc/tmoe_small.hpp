@@ -709,7 +709,10 @@ __device__ __forceinline__ void route_row16(const FwdArgs& a, int64_t t, int sl,
 // GB: K groups (64 elements in bf16, 32 in fp32) a consumer wave's weight loads hold at
 // once, issued before the wait: 2 where K gives each of the 16 waves more than one. One token block (MF = 1) stays
 // within 64 registers, so that two work-groups fit a compute unit (d_out 4608: 356 of them).
-template <class Elt, int MF, int W, int GB>
+// kPart: the whole layer (kDecodeAll), or under graph capture, where no flag may be waited for,
+// the producers and the consumers as a launch each: the same code, so the same bits.
+constexpr int kDecodeAll = 0, kDecodeProducers = 1, kDecodeConsumers = 2;
+template <class Elt, int MF, int W, int GB, int kPart>
 __global__ __launch_bounds__(64 * W) void k_sk_decode(FwdArgs a) {
   static_assert(W == 16, "one 16-lane row per token of a 64-token block");
   constexpr int kGroups = MF;   // 4-column groups of z a thread holds: 16 MF tokens, r3 <= 256
@@ -719,10 +722,10 @@ __global__ __launch_bounds__(64 * W) void k_sk_decode(FwdArgs a) {
   float* dyn = reinterpret_cast<float*>(dynv);
   const int R3 = (int)a.r3, R1 = (int)a.r1, E = (int)a.E, NZ = R3 / 16;
   const int Tn = (int)a.T;
-  const int bid = blockIdx.x;
   const SkDecodeScratch sc(a);
   const int NP = (NZ + 1) * kDecodeRowGroups;
-  if (bid < NP) {
+  const int bid = (int)blockIdx.x + (kPart == kDecodeConsumers ? NP : 0);
+  if (kPart == kDecodeProducers || (kPart == kDecodeAll && bid < NP)) {
     // ---- producers: 16 columns of [z | logits] for up to 16 tokens ----
     const int blk = bid / kDecodeRowGroups, rg = bid - blk * kDecodeRowGroups;
     const int rpg = (Tn + kDecodeRowGroups - 1) / kDecodeRowGroups;
@@ -762,7 +765,7 @@ __global__ __launch_bounds__(64 * W) void k_sk_decode(FwdArgs a) {
           store_coherent(sc.cs + r0 * R1 + q, cl[q]);
       }
     }
-    sync_publish(a.sync + sync_flag(bid), a.epoch);
+    if constexpr (kPart == kDecodeAll) sync_publish(a.sync + sync_flag(bid), a.epoch);
     return;
   }
   // ---- consumers: 16 columns of out = (c (x) z) W^T + bias ----
@@ -791,7 +794,8 @@ __global__ __launch_bounds__(64 * W) void k_sk_decode(FwdArgs a) {
 #pragma unroll
     for (int q = 0; q < 4; ++q) gv[j][q] = g < NG ? a.gain[col + q] : 0.f;
   }
-  const bool ok = sync_await(a.sync + sync_flag(0), NP, a.epoch, a.sync,
+  const bool ok = kPart == kDecodeConsumers ||
+                  sync_await(a.sync + sync_flag(0), NP, a.epoch, a.sync,
                              reinterpret_cast<int*>(red), false, a.wait_polls, a.status);
   // every load first: the z groups and c
   const __amdgpu_buffer_rsrc_t rz = coherent_rsrc(sc.zr, (int64_t)Tn * R3);

@@ -22,9 +22,9 @@ SHAPES = [
 ]
 
 
-def _layer(pkg, dev, shape, T):
+def _layer(pkg, dev, shape, T, dtype=torch.bfloat16):
     E, k, r1, r3, r2, d_in, d_out = shape
-    w = pkg.Workload("custom", T, d_in, d_out, E, k, r1, r3, r2, torch.bfloat16, 91)
+    w = pkg.Workload("custom", T, d_in, d_out, E, k, r1, r3, r2, dtype, 91)
     params = pkg.synth.make_params(w, affine="random")
     m = pkg.TuckerMoE(w.d_in, w.d_out, w.cfg()).to(dev, w.dtype)
     m.load_state_dict({k_: v.to(dev) for k_, v in params.items()})
@@ -59,23 +59,32 @@ def test_decode_fold(pkg, dev, shape, T):
     assert torch.equal(idx, idx2) and err <= 1e-2 and err2 <= 1e-2
 
 
-def test_decode_fold_capture_and_workspace(pkg, dev):
-    """A captured forward takes the two-GEMM launches; eager ones around it stay equal."""
-    _, _, m, x = _layer(pkg, dev, SHAPES[0], 20)
-    xs = x.to(dev)
-    ref = _run(m, xs)[0]
-    g = torch.cuda.CUDAGraph()
-    with torch.no_grad(), torch.cuda.graph(g):
-        out = m(xs)
-    two = None
-    for _ in range(3):
-        out.zero_()
-        g.replay()
-        torch.cuda.synchronize()
-        two = out.clone() if two is None else two
-        assert torch.equal(out, two)
-        assert torch.equal(_run(m, xs)[0], ref)
-    assert onp.rel_l2(two.float().cpu().numpy(), ref.double().cpu().numpy()) <= 1e-2
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32], ids=["bf16", "fp32"])
+@pytest.mark.parametrize("T", [1, 16, 20, 64])
+def test_decode_fold_capture(pkg, dev, dtype, T):
+    """A captured forward (the kernel's two halves, a launch each) has the eager one's bits,
+    routing outputs included, on every replay."""
+    for shape in ((8, 2, 4, 256, 512, 768, 768), (8, 2, 4, 128, 256, 512, 1040),
+                  (16, 3, 8, 64, 192, 256, 272)) + tuple(
+            SHAPES[1:2] if dtype == torch.bfloat16 else ()):
+        _, _, m, x = _layer(pkg, dev, shape, T, dtype)
+        if m.plan().folded():
+            shape = shape[:4] + (64,) + shape[5:]     # r2 of 64: not folded at other T
+            _, _, m, x = _layer(pkg, dev, shape, T, dtype)
+        assert not m.plan().folded()
+        assert m.plan().forward_path(T) == pkg._lib.TMOE_PATH_DECODE
+        xs = x.to(dev)
+        ref = _run(m, xs)
+        g = torch.cuda.CUDAGraph()
+        with torch.no_grad(), torch.cuda.graph(g):
+            got = m.forward_with_routing(xs)
+        for _ in range(3):
+            for t in got[:3]:
+                t.zero_()
+            g.replay()
+            torch.cuda.synchronize()
+            for a, b, c in zip(got[:3], ref[:3], _run(m, xs)[:3]):
+                assert torch.equal(a, b) and torch.equal(c, b), (shape, T)
 
 
 def test_decode_fold_fp8(pkg, dev):
