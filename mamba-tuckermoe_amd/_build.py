@@ -7,6 +7,7 @@ __graft_entry__.build() does).
 from __future__ import annotations
 
 import os
+import re
 import shutil
 import subprocess
 import sysconfig
@@ -49,13 +50,22 @@ def hipcc() -> str:
     raise RuntimeError("hipcc not found: the gfx950 library cannot be built")
 
 
+def native_tag() -> str:
+    """What _tmoe_native.so is compiled for: the version of the C ABI's header, torch's and
+    Python's (_lib.native() loads no other)."""
+    import torch
+    with open(os.path.join(INCLUDE, "tmoe.h")) as f:
+        abi = re.search(r"#define TMOE_ABI_VERSION (\d+)", f.read()).group(1)
+    return f"abi {abi} torch {torch.__version__} {sysconfig.get_config_var('SOABI')}"
+
+
 def native_cmd(out: str) -> list:
     """The host compiler's line for _tmoe_native.so, against the torch that runs it."""
     import torch
     inc = os.path.join(os.path.dirname(torch.__file__), "include")
     lib = os.path.join(os.path.dirname(torch.__file__), "lib")
     return [os.environ.get("CXX") or "g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall",
-            "-Wno-unknown-pragmas",
+            "-Wno-unknown-pragmas", f'-DTMOE_NATIVE_TAG="{native_tag()}"',
             f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", "-I", INCLUDE,
             "-isystem", inc, "-isystem", os.path.join(inc, "torch", "csrc", "api", "include"),
             "-isystem", sysconfig.get_paths()["include"], os.path.join(CSRC, NATIVE_SOURCE),
@@ -64,7 +74,9 @@ def native_cmd(out: str) -> list:
 
 def build(verbose: bool = False) -> str:
     """Compiles every source (concurrently) and links libtmoe.so, libtmoe_probe.so and
-    _tmoe_native.so; returns libtmoe.so's path."""
+    _tmoe_native.so; returns libtmoe.so's path. Where only _tmoe_native.so cannot be built
+    (torch's or Python's headers missing), the others, all that callers of the C ABI need,
+    are built before that is raised."""
     objdir = os.path.join(HERE, "_build")
     os.makedirs(objdir, exist_ok=True)
     cmds, groups = [], []
@@ -78,15 +90,28 @@ def build(verbose: bool = False) -> str:
             objs.append(obj)
         groups.append((lib, objs))
     native_tmp = NATIVE_LIB + ".tmp"
-    cmds.append(native_cmd(native_tmp))
-    _run_all(cmds, verbose)
-    os.replace(native_tmp, NATIVE_LIB)
+    native_failed = None
+    try:
+        native = native_cmd(native_tmp)
+    except Exception as e:   # no torch, or one without the headers' paths
+        native_failed = f"{NATIVE_LIB}: {e}"
+        native = None
+    errors = _run_all(cmds + ([native] if native else []), verbose)
+    if native:
+        native_failed = errors.pop()
+        if not native_failed:
+            os.replace(native_tmp, NATIVE_LIB)
+    for e in errors:
+        if e:
+            raise RuntimeError(e)
     for lib, objs in groups:
         tmp = lib + ".tmp"
         cmd = [hipcc(), f"--offload-arch={ARCH}", "-shared", "-fPIC", *objs, "-o", tmp,
                "-Wl,-rpath,/opt/rocm/lib"]
         _run(cmd, verbose)
         os.replace(tmp, lib)
+    if native_failed:
+        raise RuntimeError(native_failed)
     return LIB
 
 
@@ -95,23 +120,22 @@ _NOISE = "'-packed-fp32-ops' is not a recognized feature"
 
 
 def _run_all(cmds, verbose):
-    """Runs the compile commands side by side; raises on the first that failed."""
+    """Runs the compile commands side by side; an error text or None for each."""
     procs = []
     for cmd in cmds:
         if verbose:
             print(" ".join(cmd), flush=True)
         procs.append((cmd, subprocess.Popen(cmd, stdout=subprocess.PIPE, stderr=subprocess.PIPE,
                                             text=True)))
-    failed = None
+    errors = []
     for cmd, pr in procs:
         _, stderr = pr.communicate()
         err = "\n".join(l for l in stderr.splitlines() if _NOISE not in l)
-        if pr.returncode != 0 and failed is None:
-            failed = f"build failed ({pr.returncode}): {' '.join(cmd)}\n{err}"
-        elif verbose and err.strip():
+        errors.append(f"build failed ({pr.returncode}): {' '.join(cmd)}\n{err}"
+                      if pr.returncode != 0 else None)
+        if pr.returncode == 0 and verbose and err.strip():
             print(err)
-    if failed:
-        raise RuntimeError(failed)
+    return errors
 
 
 def _run(cmd, verbose):

@@ -13,6 +13,7 @@ from __future__ import annotations
 import ctypes
 import importlib.util
 import os
+import sysconfig
 import threading
 
 import torch  # noqa: F401  (loads torch's HIP runtime before libtmoe.so)
@@ -175,9 +176,20 @@ def native():
             if not os.path.exists(NATIVE_PATH):
                 raise RuntimeError(f"{NATIVE_PATH} is not built; build it with "
                                    "__graft_entry__.build(). There is no fallback path.")
+            want = f"abi {ABI_VERSION} torch {torch.__version__} {sysconfig.get_config_var('SOABI')}"
             spec = importlib.util.spec_from_file_location("_tmoe_native", NATIVE_PATH)
-            mod = importlib.util.module_from_spec(spec)
-            spec.loader.exec_module(mod)
+            try:
+                mod = importlib.util.module_from_spec(spec)
+                spec.loader.exec_module(mod)
+            except ImportError as e:
+                raise RuntimeError(f"{NATIVE_PATH} does not load here ({want}): {e}; build it "
+                                   "again with __graft_entry__.build()") from e
+            # compiled against one torch's C++ headers (_build.native_tag): with another its
+            # calls would be undefined
+            built_for = getattr(mod, "built_for", None)
+            if built_for != want:
+                raise RuntimeError(f"{NATIVE_PATH} was built for {built_for!r}, this is {want!r}; "
+                                   "build it again with __graft_entry__.build()")
             mod.bind(*(ctypes.cast(getattr(L, f), ctypes.c_void_p).value for f in (
                 "tmoe_workspace_bytes", "tmoe_signal_status", "tmoe_forward_epi",
                 "tmoe_forward_glu", "tmoe_rmsnorm_rows")))

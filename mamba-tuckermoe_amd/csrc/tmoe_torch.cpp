@@ -234,5 +234,10 @@ PyMODINIT_FUNC PyInit__tmoe_native() {
   g_alias = PyUnicode_InternFromString("_tmoe_alias");
   if (!g_gen || !g_alias) return nullptr;
   g_module.m_methods = methods;
-  return PyModule_Create(&g_module);
+  PyObject* m = PyModule_Create(&g_module);
+  if (m && PyModule_AddStringConstant(m, "built_for", TMOE_NATIVE_TAG) < 0) {
+    Py_DECREF(m);
+    return nullptr;
+  }
+  return m;
 }
