@@ -13,7 +13,11 @@ from oracle import tucker_moe_np as onp
 pytestmark = pytest.mark.gpu
 
 
-def _check(pkg, dev, x, G, idx, p, dout):
+def _check(pkg, dev, x, G, idx, p, dout, forms=None):
+    if forms is not None:   # the kernels of (forward, backward) this case is for
+        f = pkg._lib
+        sizes = (x.shape[0], G.shape[0], idx.shape[1], G.shape[1], G.shape[2], f.TMOE_BF16)
+        assert (f.lib().tmoe_latent_form(*sizes, 0), f.lib().tmoe_latent_form(*sizes, 1)) == forms
     xs, Gs, ps = (t.to(dev).requires_grad_(True) for t in (x, G, p))
     out = pkg.FusedLatentMoE.apply(xs, Gs, idx.to(dev), ps)
     out.backward(dout.to(dev))
@@ -45,23 +49,33 @@ def _inputs(B, E, k, r3, r2, seed, p32):
     return x, G, idx, p, torch.randn(B, r2, generator=g).bfloat16()
 
 
+# (forward, backward) bits of tmoe_latent_form: dense but for dG; all grouped
+DG, ALL = (0, 2), (1, 3)
+
+
 # (E, k, r3, r2, B): k = 2 pairs from B = 1110 on at E = 8 (the rule's first size and one
 # below it), k = 1 from 91 at E = 16, 4 of 16 experts (dG alone grouped), one token,
-# entries that do not fill a K tile, the widest router, one tile of r2
-@pytest.mark.parametrize("E,k,r3,r2,B", [
-    (8, 2, 256, 1024, 1109), (8, 2, 256, 1024, 1110), (8, 2, 128, 128, 2049),
-    (16, 1, 256, 512, 90), (16, 1, 256, 512, 91), (16, 1, 128, 384, 129),
-    (16, 4, 256, 256, 1), (16, 4, 256, 256, 65), (64, 2, 128, 128, 4300), (8, 6, 128, 128, 333),
+# entries that do not fill a K tile, one tile of r2; the widest router (2080 pairs, most of
+# them of a token or two) on both sides of its line and well past it; few experts, whose
+# forward is dense where the backward is grouped
+@pytest.mark.parametrize("E,k,r3,r2,B,forms", [
+    (8, 2, 256, 1024, 1109, DG), (8, 2, 256, 1024, 1110, ALL), (8, 2, 128, 128, 2049, ALL),
+    (16, 1, 256, 512, 90, DG), (16, 1, 256, 512, 91, ALL), (16, 1, 128, 384, 129, ALL),
+    (16, 4, 256, 256, 1, DG), (16, 4, 256, 256, 65, DG), (64, 2, 128, 128, 4300, DG),
+    (8, 6, 128, 128, 333, DG), (64, 2, 128, 128, 5637, DG), (64, 2, 128, 128, 5638, ALL),
+    (64, 2, 128, 256, 8001, ALL), (64, 1, 128, 128, 4099, ALL),
 ])
 @pytest.mark.parametrize("p32", [False, True], ids=["pbf16", "pf32"])
-def test_grouped(pkg, dev, E, k, r3, r2, B, p32):
-    _check(pkg, dev, *_inputs(B, E, k, r3, r2, B + E, p32))
+def test_grouped(pkg, dev, E, k, r3, r2, B, forms, p32):
+    _check(pkg, dev, *_inputs(B, E, k, r3, r2, B + E, p32), forms=forms)
 
 
 @pytest.mark.parametrize("kind", ["one", "repeat", "outside", "none"])
-@pytest.mark.parametrize("k", [1, 2, 4])
-def test_grouped_odd_routing(pkg, dev, kind, k):
-    B, E = 1500, 16
+@pytest.mark.parametrize("B,E,k,forms", [
+    (1500, 16, 1, ALL), (1500, 16, 2, DG), (1500, 16, 4, DG), (2000, 16, 2, ALL),
+    (1400, 8, 2, ALL), (5700, 64, 2, ALL),
+])
+def test_grouped_odd_routing(pkg, dev, kind, B, E, k, forms):
     x, G, idx, p, dout = _inputs(B, E, k, 128, 256, 5, True)
     if kind == "one":              # every token the same expert first: one group of all
         idx = torch.where(idx == 3, idx[:, :1], idx)
@@ -74,7 +88,7 @@ def test_grouped_odd_routing(pkg, dev, kind, k):
         idx[2::8] = 1 << 40
     else:
         idx[:] = -5
-    _check(pkg, dev, x, G, idx, p, dout)
+    _check(pkg, dev, x, G, idx, p, dout, forms=forms)
 
 
 def test_grouped_is_deterministic(pkg, dev):
