@@ -915,9 +915,17 @@ bool latent_pairs_forward(const LatentArgs& l) {
       14.3 + rows * (0.18e-3 + cols * (0.24e-6 + 2.4e-9 * (double)l.r3)) + spill;
   return grouped <= dense;
 }
-// dG over each expert's own entries: below the dense form's B E rows.
+// dG over each expert's own entries: below the dense form's B E rows. With many slots the sort
+// of the B k entries (64 work-groups) and their scaled rows outgrow what the narrower products
+// save, the sooner the fewer columns: past 4 slots only with r2 of 512 or up to 8192 tokens, past
+// 8 also only with at most half of the experts selected. Backward, us, dense : grouped, at 65536
+// tokens, r3 256: k 4 of 8, r2 128 390 : 382; 6 of 8, r2 128 425 : 481 (8192 tokens 107 : 102), r2 512
+// 725 : 680; 8 of 16, r2 128 712 : 781, r2 512 1274 : 1139; 12 of 16, r2 512 1434 : 1486, r2 1024
+// 2210 : 2355 (2048 tokens 125 : 131); 16 of 64, r2 512 5690 : 4650.
 bool latent_dg_grouped(const LatentArgs& l) {
-  return l.dtype == kDtypeBF16 && latent_grouped_shape(l.E, l.r3, l.r2) && 5 * l.k <= 4 * l.E;
+  if (l.dtype != kDtypeBF16 || !latent_grouped_shape(l.E, l.r3, l.r2) || 5 * l.k > 4 * l.E)
+    return false;
+  return l.k <= 4 || ((l.r2 >= 512 || l.B <= 8192) && (l.k <= 8 || 2 * l.k <= l.E));
 }
 
 LatentLayout latent_layout(int64_t B, int64_t E, int64_t r3, int64_t r2, int es, bool bwd) {

@@ -49,8 +49,8 @@ def _inputs(B, E, k, r3, r2, seed, p32):
     return x, G, idx, p, torch.randn(B, r2, generator=g).bfloat16()
 
 
-# (forward, backward) bits of tmoe_latent_form: dense but for dG; all grouped
-DG, ALL = (0, 2), (1, 3)
+# (forward, backward) bits of tmoe_latent_form: dense but for dG; all grouped; none
+DG, ALL, DENSE = (0, 2), (1, 3), (0, 0)
 
 
 # (E, k, r3, r2, B): k = 2 pairs from B = 1110 on at E = 8 (the rule's first size and one
@@ -64,6 +64,7 @@ DG, ALL = (0, 2), (1, 3)
     (16, 4, 256, 256, 1, DG), (16, 4, 256, 256, 65, DG), (64, 2, 128, 128, 4300, DG),
     (8, 6, 128, 128, 333, DG), (64, 2, 128, 128, 5637, DG), (64, 2, 128, 128, 5638, ALL),
     (64, 2, 128, 256, 8001, ALL), (64, 1, 128, 128, 4099, ALL),
+    (8, 6, 128, 128, 8192, DG), (8, 6, 128, 128, 8193, DENSE), (16, 9, 128, 128, 700, DENSE),
 ])
 @pytest.mark.parametrize("p32", [False, True], ids=["pbf16", "pf32"])
 def test_grouped(pkg, dev, E, k, r3, r2, B, forms, p32):

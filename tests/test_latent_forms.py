@@ -18,6 +18,11 @@ def _form(pkg, B, E, k, r3, r2, backward, dtype=torch.bfloat16):
     (16, 4, 256, 256, 16384, 0, 0, 1), (8, 6, 128, 128, 333, 0, 0, 1),
     (8, 7, 128, 128, 333, 0, 0, 0), (2, 2, 256, 1024, 4096, 0, 0, 0),
     (8, 2, 64, 1024, 4096, 0, 0, 0), (8, 2, 256, 192, 4096, 0, 0, 0),
+    # many slots: by the columns, the tokens and the share of the experts
+    (8, 4, 256, 128, 65536, 0, 0, 1), (8, 5, 256, 128, 8192, 0, 0, 1), (8, 5, 256, 128, 8193, 0, 0, 0),
+    (8, 5, 256, 384, 8193, 0, 0, 0), (8, 5, 256, 512, 65536, 0, 0, 1), (16, 8, 128, 512, 65536, 0, 0, 1),
+    (16, 9, 256, 1024, 2048, 0, 0, 0), (18, 9, 256, 1024, 2048, 0, 0, 1), (64, 16, 256, 128, 8193, 0, 0, 0),
+    (64, 16, 256, 512, 8193, 0, 0, 1),
     # few experts and a full chip: dense forward, grouped backward
     (2, 1, 256, 1024, 16384, 0, 1, 1), (2, 1, 128, 512, 16384, 0, 1, 1),
     (3, 2, 256, 1024, 16384, 0, 1, 1), (3, 2, 128, 512, 32768, 0, 1, 1),
