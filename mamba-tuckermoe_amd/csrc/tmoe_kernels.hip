@@ -564,10 +564,11 @@ hipError_t launch_core(const FwdArgs& a, hipStream_t st) {
     }
   }
   if (a.dtype == kDtypeBF16) return launch_core_t<EltBF16, CoreCfgBF16>(a, st);
-  // fp32, 64 x 64 tiles in core_f32_split slices while 128 x 128 ones would number at most
-  // one a compute unit (1021 x 512, K 2048: 25 + 5 us of adding the slices against 140 for
-  // 32 work-groups of 128 x 128)
-  if (core_f32_tiles(a.T, a.r2) > 4 * cu_count()) return launch_core_t<EltF32, CoreCfgF32>(a, st);
+  // fp32, 64 x 64 tiles in core_f32_split slices while they number at most three a compute
+  // unit (1021 x 512, K 2048: 25 + 5 us of adding the slices against 140 for 32 work-groups of
+  // 128 x 128). A round of them takes a little over a quarter of one of 128 x 128 tiles: r2 1024,
+  // K 1024, 768 of them (3072 tokens) 76 against 91 us, 784 95 : 91, 1024 98 : 94
+  if (core_f32_tiles(a.T, a.r2) > 3 * cu_count()) return launch_core_t<EltF32, CoreCfgF32>(a, st);
   return launch_core_t<EltF32, CoreCfgF32S>(a, st);
 }
 

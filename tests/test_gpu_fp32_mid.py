@@ -29,12 +29,14 @@ def _forward(m, x):
 
 # (E, k, r1, r3, r2, d_in, d_out): d_in of 16 K tiles (the first sliced one) and of 15 (not
 # sliced); the expert form (E < r1) with 8 core slices and r2 of one tile; a router of 100
-# columns; ragged column tiles of both GEMMs
+# columns; ragged column tiles of both GEMMs; the last T of the core's 64 x 64 tiles and the
+# first of its 128 x 128 ones
 @pytest.mark.parametrize("shape,T", [
     ((8, 2, 32, 256, 512, 1536, 1008), 257), ((8, 2, 32, 256, 512, 1536, 1008), 1021),
     ((16, 2, 4, 256, 192, 512, 208), 300), ((16, 2, 4, 256, 192, 576, 208), 288),
     ((8, 2, 4, 64, 64, 448, 64), 1000), ((100, 4, 8, 128, 320, 512, 656), 2049),
     ((8, 2, 4, 64, 64, 512, 16), 4096), ((4, 1, 2, 128, 1024, 640, 2304), 4097),
+    ((4, 1, 2, 128, 1024, 640, 272), 3072), ((4, 1, 2, 128, 1024, 640, 272), 3073),
 ], ids=lambda v: str(v))
 def test_fp32_mid(pkg, dev, shape, T):
     w, params, m, x = _layer(pkg, dev, shape, T)
