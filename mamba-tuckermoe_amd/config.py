@@ -132,14 +132,15 @@ class Workload:
 
     def one_launch(self, T: int, rk: int, folded: bool) -> bool:
         """Whether a forward of T tokens is the library's single decode launch
-        (k_sk_decode; the selection rule of small_decode_ok in tmoe_kernels.hip and, for
-        plans not folded at other T, decode_fold_ok in tmoe_internal.h; outside graph
-        capture, folding not switched off)."""
-        es = 4 if self.dtype == torch.float32 else 2
-        K = rk * self.r3
-        fits = K <= 2048 and K * self.d_out * es <= 32 << 20
-        return ((folded or fits) and 0 < T <= 64 and self.E <= 16
-                and self.r3 in (64, 128, 256) and rk <= 32)
+        (k_sk_decode) outside graph capture: the selection rule of small_decode_ok in
+        tmoe_kernels.hip for folded plans, for others what the library says of a plan of
+        these sizes (folding not switched off)."""
+        if folded:
+            return (0 < T <= 64 and self.E <= 16 and self.r3 in (64, 128, 256) and rk <= 32)
+        from . import _lib
+        plan = _lib.Plan(self.d_in, self.d_out, self.E, self.k, self.r1, self.r2, self.r3,
+                         self.dtype, 1e-5, fp8_weights=self.fp8)
+        return T > 0 and plan.forward_path(T) == _lib.TMOE_PATH_DECODE
 
     def layer_bytes_folded(self, T: Optional[int] = None, rk: Optional[int] = None) -> int:
         """Compulsory bytes of a folded forward in one launch: x, the front weights,

@@ -39,8 +39,8 @@ struct tmoe_plan {
   int64_t rk;
   // folded form (large T): W^T (d_out, rk*r3) at off_fold, one GEMM of c (x) z against W
   bool fold;
-  // W^T also packed for a plan that is not folded, for its decode-size batches
-  // (tmoe::decode_fold_ok)
+  // W^T also packed for a plan that is not folded, for the batches of at most kSmallT
+  // tokens that run folded (tmoe::decode_fold_ok)
   bool decode_fold;
   size_t off_fold;
   // status block (tmoe::kStatusWords words of pinned host memory mapped for the
@@ -139,6 +139,13 @@ bool batch_folded(const tmoe_plan* p, int64_t T) {
     return tmoe::batch_fold_pays(T, p->s.d_out, p->rk * p->s.r3,
                                  tmoe::front_split(T, p->s.d_in, p->E_pad, p->es));
   return p->decode_fold && tmoe::batch_out_tiles(T, p->s.d_out) <= tmoe::kBatchFoldTiles;
+}
+
+// Whether a forward of T tokens of a plan that is not folded otherwise is for the folded decode
+// launch (tmoe::decode_fold_pays).
+bool decode_folded(const tmoe_plan* p, int64_t T) {
+  return p->decode_fold && T <= tmoe::kDecodeMaxT &&
+         tmoe::decode_fold_pays(T, p->rk, p->s.r3, p->s.r2, p->s.d_out, (int64_t)p->es);
 }
 
 // lean: without the fp32 plans' K slices (their planes) and without folded batches, for a
@@ -327,7 +334,7 @@ void small_stages(const tmoe_plan* p, const void* packed, tmoe::FwdArgs& a, hipS
     st[2] = tmoe::launch_outproj;
     return;
   }
-  if (p->decode_fold && a.T <= tmoe::kDecodeMaxT) {
+  if (decode_folded(p, a.T)) {
     // captured or not, the same form: in one launch, or its two halves under capture
     const tmoe::FwdArgs f = decode_fold_args(p, a, packed);
     if (tmoe::small_decode_shape_ok(f)) {
@@ -455,7 +462,7 @@ int tmoe_plan_create(const tmoe_shape* shape, tmoe_plan** plan_out) {
   if (p->core_p) { p->off_core_p = o; o = align256(o + (size_t)p->rk * s.r2 * s.r3 * p->es); }
   p->off_fold = 0;
   p->decode_fold = !p->fold && !(s.flags & TMOE_FLAG_NO_FOLD) &&
-                   tmoe::decode_fold_ok(s.E, p->rk, s.r3, s.d_out, (int64_t)p->es);
+                   tmoe::decode_fold_ok(s.E, p->rk, s.r3, s.r2, s.d_out, (int64_t)p->es);
   if (p->fold || p->decode_fold) {
     p->off_fold = o;
     o = align256(o + (size_t)s.d_out * K * p->es);
@@ -490,8 +497,9 @@ int tmoe_plan_folded(const tmoe_plan* plan) { return plan && plan->fold ? 1 : 0;
 // experts than ranks packed in the expert form (identity U_expert, core G); 5: folded
 // plans add W^T = (core U_out)^T; 7: bf16 plans with r3 = 256 and E_pad = 32 add the
 // front operand in fragment order (k_front_ks); 8: W^T also for unfolded plans whose
-// decode-size batches run folded.
-int tmoe_packed_layout_version(void) { return 8; }
+// decode-size batches run folded; 9: of those only where a T of at most kSmallT does
+// (decode_fold_pays).
+int tmoe_packed_layout_version(void) { return 9; }
 
 size_t tmoe_workspace_bytes(const tmoe_plan* plan, int64_t T) {
   if (!plan || T < 0) return 0;
@@ -933,7 +941,7 @@ int tmoe_forward_path(const tmoe_plan* p, int64_t T) {
       tmoe::FwdArgs f = folded_args(p, a, fake, nullptr);
       if (tmoe::small_decode_shape_ok(f)) return TMOE_PATH_DECODE;
     }
-    if (p->decode_fold && T <= tmoe::kDecodeMaxT &&
+    if (decode_folded(p, T) &&
         tmoe::small_decode_shape_ok(decode_fold_args(p, a, fake)))
       return TMOE_PATH_DECODE;
     return TMOE_PATH_SMALL;

@@ -306,14 +306,47 @@ hipError_t launch_small_decode_out(const FwdArgs& a, hipStream_t stream);
 // Unfolded plans whose decode-size batches (T <= kDecodeMaxT) still run folded, in
 // that one launch, against a W^T packed beside the two-GEMM weights: K = rk r3 of at most
 // 2048 (two K groups a consumer wave) and W^T of at most 32 MB (read whole by every
-// forward, about 6 us). The two-GEMM form takes three launches there: the reference
-// model's FFN (three layers and a norm) 61 us at T = 1 and 135 at T = 64, folded 41 and 80;
-// its 1536 -> 6144 layer 31 and 43, folded 14 and 29; in fp32 the 1536 -> 2304 layer 31 and 50,
-// folded 12 and 20, the 512 -> 1024 layer at T = 64 28, folded 18 (with its routing).
+// forward), packed where some T <= kSmallT runs folded. The two-GEMM form takes three
+// launches there: the reference model's FFN (three layers and a norm) 61 us at T = 1 and 135
+// at T = 64, folded 41 and 80; its 1536 -> 6144 layer 31 and 43, folded 14 and 29; in fp32 the
+// 1536 -> 2304 layer 31 and 50, folded 12 and 20, the 512 -> 1024 layer at T = 64 28, folded
+// 18 (with its routing).
 constexpr int64_t kDecodeFoldK = 2048, kDecodeFoldBytes = 32 << 20;
-inline bool decode_fold_ok(int64_t E, int64_t rk, int64_t r3, int64_t d_out, int64_t es) {
-  return E <= 16 && rk <= 32 && rk * r3 <= kDecodeFoldK &&
-         rk * r3 * d_out * es <= kDecodeFoldBytes;
+// Whether T <= kDecodeMaxT tokens of such a plan are faster folded. The launch's 16-column
+// work-groups take one, two, three rounds of the compute units at 4096, 8192, 12288
+// columns; each round stages T rows of z and reads its share of W^T, which holds `extra` bytes
+// more than core and U_out together. Kernel time, us, folded : two GEMMs, bf16 but where said,
+// r3 = 256, over 1680 measured (plan, T); W^T warm, cold ones of 600 MB in turn cross at the same lines:
+//   one round: folded always (K 2048, 2304 columns T = 1 8.3 : 14, T = 64 16 : 36)
+//   two, T <= 32: K 2048, 8192 columns, T = 1: r2 64 (31 MB extra) 15.3 : 12.7, 256 (28) 14.3 : 13.1,
+//     512 (23) 15.1 : 14.3, 1024 (13) 15.1 : 15.5; K 1024, r2 512 (7) 11 : 13
+//   two, T > 32: 64 tokens at rank 2, 8192 columns 25.7 : 23.5, 6144 22.7 : 24; rank 4, r2 64
+//     27.5 : 26.2, r2 512 28 : 30; rank 2 in fp32 31.1 : 33.1
+//   three: rank 4, r2 512, 12288 columns T = 32 24.7 : 25.7, T = 48 34.2 : 31.1; rank 2 T = 24 21.0 :
+//     20.3; r2 64 (23 MB) T = 1 14.8 : 13.6; r3 = 128, K 512 T = 1 13.3 : 13.8, T = 64 27.7 : 27.5;
+//     r3 = 64, K 1024, r2 256 (18 MB) T = 1 14.2 : 13.8, T = 24 18.1 : 20.1
+//   four: 16384 columns, rank 4, r2 512 T = 1 19 : 15, T = 64 51 : 36
+inline bool decode_fold_pays(int64_t T, int64_t rk, int64_t r3, int64_t r2, int64_t d_out,
+                             int64_t es) {
+  const int64_t rounds = (d_out + 4095) / 4096, K = rk * r3;
+  if (rounds <= 1) return true;
+  if (rounds > 3) return false;
+  const int64_t extra = es * (K * d_out - r2 * (K + d_out));
+  const bool small_core = r3 == 256 && rk * r2 <= 512;   // the two GEMMs' middle launch is short
+  if (rounds == 2) {
+    if (T <= 32) return extra <= 19000000;
+    return d_out <= 6144 || es == 4 || !small_core;
+  }
+  if (r3 == 256) return T <= 32 && !small_core && extra <= 12000000;
+  return T > 16 || extra <= 12000000;
+}
+inline bool decode_fold_ok(int64_t E, int64_t rk, int64_t r3, int64_t r2, int64_t d_out,
+                           int64_t es) {
+  if (E > 16 || rk > 32 || rk * r3 > kDecodeFoldK || rk * r3 * d_out * es > kDecodeFoldBytes)
+    return false;
+  for (int64_t T : {16, 32, 64})   // one of each range of the rule
+    if (decode_fold_pays(T, rk, r3, r2, d_out, es)) return true;
+  return es == 2 && batch_out_tiles(kDecodeMaxT + 1, d_out) <= kBatchFoldTiles;
 }
 // floats of its scratch at FwdArgs::raw: z columns (T, r3), c (T, r1)
 constexpr int64_t sk_decode_scratch_floats(int64_t T, int64_t r3, int64_t r1) {

@@ -1,4 +1,4 @@
-"""Which forms batches of 65 to 256 tokens take (host-side rules, as on a 256-compute-unit
+"""Which forms batches of up to 256 tokens take (host-side rules, as on a 256-compute-unit
 MI355X)."""
 import pytest
 import torch
@@ -59,3 +59,39 @@ def test_other_batches(pkg):
     shape = dict(d_in=256, d_out=10880, r1=8, r2=64, r3=64)
     assert _form(pkg, 192, **shape) == both and _form(pkg, 193, **shape) == 0
     assert _form(pkg, 64, **shape) == f.TMOE_FORM_FOLDED and _form(pkg, 0, **shape) == 0
+
+
+# plans that are not folded otherwise, by rounds of 4096 columns: (r1, r3, r2, d_out, dtype) and
+# the T of 16, 17, 32, 33, 64 that run folded
+BF, F32 = torch.bfloat16, torch.float32
+ALL, UP32, FROM33 = (16, 17, 32, 33, 64), (16, 17, 32), (33, 64)
+
+
+@pytest.mark.parametrize("r1,r3,r2,d_out,dtype,folded", [
+    (8, 256, 64, 4096, BF, ALL), (2, 256, 256, 4096, F32, ALL),        # one round
+    (8, 256, 512, 6144, BF, ALL), (8, 256, 256, 8192, BF, FROM33),     # two: W^T's extra bytes
+    (8, 256, 512, 8192, BF, FROM33), (8, 256, 1024, 8192, BF, ALL), (4, 256, 512, 8192, BF, ALL),
+    (2, 256, 256, 8192, BF, UP32), (2, 256, 256, 6144, BF, ALL),       # two: a short core
+    (2, 256, 256, 8192, F32, ALL), (2, 128, 256, 8192, BF, ALL),
+    (4, 256, 512, 9216, BF, UP32), (4, 256, 512, 12288, BF, UP32),     # three
+    (2, 256, 256, 9216, BF, ()), (4, 256, 64, 9216, BF, ()), (4, 128, 256, 12288, BF, ALL),
+    (16, 64, 256, 12288, BF, (17, 32, 33, 64)), (2, 256, 256, 9216, F32, ()),
+    (4, 256, 512, 12304, BF, ()), (2, 256, 256, 16384, BF, ()),        # four
+])
+def test_decode_forms(pkg, r1, r3, r2, d_out, dtype, folded):
+    f = pkg._lib
+    for T in ALL:
+        got = _form(pkg, T, d_in=768, d_out=d_out, E=16, r1=r1, r3=r3, r2=r2, dtype=dtype)
+        assert got == (f.TMOE_FORM_FOLDED if T in folded else 0), T
+
+
+@pytest.mark.parametrize("d_out,dtype,packed", [
+    (12288, F32, False), (4096, F32, True), (16384, BF, True), (16400, BF, False),
+])
+def test_wt_only_where_some_batch_reads_it(pkg, d_out, dtype, packed):
+    """W^T beside the two-GEMM weights: in bf16 also for batches past 64 tokens alone."""
+    args = (768, d_out, 16, 2, 2, 256, 256, dtype, 1e-5)
+    extra = (pkg._lib.Plan(*args).packed_bytes() -
+             pkg._lib.Plan(*args, flags=pkg._lib.TMOE_FLAG_NO_FOLD).packed_bytes())
+    assert extra == (512 * d_out * (2 if dtype == BF else 4) if packed else 0)
+    assert not pkg._lib.Plan(*args).folded()
