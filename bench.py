@@ -199,7 +199,8 @@ def bench_ffn(args) -> None:
     executed = 0
     for n in ("ffn_gate", "ffn_up", "ffn_down"):
         pl = getattr(m0, n).plan()
-        executed += f.layer(n).flops_executed(T, pl.core_rank(), pl.folded())["total"]
+        in_folded_form = bool(pl.forward_form(T) & pkg._lib.TMOE_FORM_FOLDED)
+        executed += f.layer(n).flops_executed(T, pl.core_rank(), in_folded_form)["total"]
     peak = PEAK_TFLOPS[dt_name]
     tflops = flops / (ms * 1e-3) / 1e12
     tflops_exec = executed / (ms * 1e-3) / 1e12
@@ -286,13 +287,15 @@ def bench_latent(args) -> None:
     ms = ev0.elapsed_time(ev1) / args.steps
     algo = 8.0 * T * k * r3 * r2          # out, dx, dp, dG: 2 T k r3 r2 each
     # forward, the product of dx and dp, dG: over each token's k experts where the grouped
-    # kernels run (latent_pairs in tmoe_kernels.hip; their tiles' padding not counted), else
-    # dense over E
-    grouped = 13 * (T + E * (E + 1) // 2 * 64) * k <= 10 * T * E
-    executed = 2.0 * T * r3 * r2 * (k if grouped else E) * 3
+    # kernels run (their tiles' padding not counted), else dense over E
+    lib, L = pkg._lib, pkg._lib.lib()
+    fwd, bwd = (L.tmoe_latent_form(T, E, k, r3, r2, lib.TMOE_BF16, b) for b in (0, 1))
+    by_expert = [fwd & lib.TMOE_LATENT_PAIRS, bwd & lib.TMOE_LATENT_PAIRS, bwd & lib.TMOE_LATENT_DG]
+    grouped = all(by_expert)
+    executed = 2.0 * T * r3 * r2 * sum(k if g else E for g in by_expert)
     peak = PEAK_TFLOPS["bf16"]
     log(f"[bench-latent] T={T}: {ms * 1e3:.1f} us per forward+backward; "
-        f"{executed / (ms * 1e-3) / 1e12:.0f} TFLOP/s executed ({'by expert' if grouped else 'dense over E'})")
+        f"{executed / (ms * 1e-3) / 1e12:.0f} TFLOP/s executed ({'by expert' if grouped else 'dense over E in part'})")
     print(json.dumps({
         "metric": LATENT_METRIC, "value": T / (ms * 1e-3), "unit": "tokens/s", "n_gpus": 1,
         "steps": args.steps, "warmup": args.warmup, "ms_per_step": ms, "higher_is_better": True,
@@ -414,7 +417,7 @@ def hw_probes(pkg, w, res) -> dict:
         out["missing"] = lib_path
     # hipBLASLt on the out-projection's GEMM: (T x K) x (K x d_out), bf16 in, fp32 accumulate
     dev = torch.device("cuda:0")
-    K = w.r1 * w.r3 if res["config"]["form"] == "folded" else w.r2
+    K = w.r1 * w.r3 if res["config"]["form"].startswith("folded") else w.r2
 
     def lib_gemm(M, N, Kd):
         a = torch.randn(M, Kd, device=dev).to(torch.bfloat16)
@@ -480,12 +483,12 @@ def measure(pkg, w, args, *, steps, warmup, rotate_mb, no_fold, no_fuse, cpu, la
                                                   "U_out_q", "U_out_scale")])
     plan = m.plan()
     packed0 = m.packed()
-    folded = plan.folded()
+    # some forwards of a plan that is not folded (decode sizes, batches of 65 to 256) are
+    folded = bool(plan.forward_form(T) & pkg._lib.TMOE_FORM_FOLDED)
     rk = plan.core_rank()
     path = plan.forward_path(T)
     form = ("folded: c (x) z against W = core U_out, one GEMM of width %d" % (rk * w.r3)
-            if folded or path == pkg._lib.TMOE_PATH_DECODE
-            else "two GEMMs: core (rank %d) then U_out" % rk)
+            if folded else "two GEMMs: core (rank %d) then U_out" % rk)
     log(f"[{label}] plan form: {form}; kernels: {pkg._lib.PATH_NAMES.get(path, path)}")
     ws_bytes = plan.workspace_bytes(T)
     set_bytes = T * w.d_in * es + T * w.d_out * es + ws_bytes + packed0.numel()
@@ -542,8 +545,7 @@ def measure(pkg, w, args, *, steps, warmup, rotate_mb, no_fold, no_fuse, cpu, la
         pkg._lib.prof_enable(False)
     stage_avg_us = {n: stage_ms[j] / calls * 1e3 for j, n in enumerate(pkg._lib.STAGE_NAMES)}
     fl_algo = w.flops()
-    # the dominant kernel's own work; the decode launch is folded in any plan
-    fl = w.flops_executed(T, rk, folded or path == pkg._lib.TMOE_PATH_DECODE)
+    fl = w.flops_executed(T, rk, folded)        # the dominant kernel's own work
     fl["front"] = fl["router"] + fl["in_proj"]   # one kernel computes both
     kr = path == pkg._lib.TMOE_PATH_LARGE_KR
     sb = (w.stage_bytes_kr(T, rk) if kr else
