@@ -132,7 +132,7 @@ struct Layout {
   int osplit;   // FwdArgs::out_split
 };
 
-// Whether a forward of T tokens is a folded batch (tmoe::kBatchFoldTiles).
+// Whether a forward of T tokens is a folded batch (tmoe::kBatchFoldTiles); never at large T.
 bool batch_folded(const tmoe_plan* p, int64_t T) {
   if (p->kdtype != TMOE_BF16 || T <= tmoe::kDecodeMaxT || T > tmoe::kSmallT) return false;
   if (p->fold)
@@ -209,7 +209,7 @@ Layout workspace_layout(const tmoe_plan* p, int64_t T, bool lean = false) {
     o = align256(o + (size_t)tmoe::sync_words(
                              T, std::max<int64_t>(T <= tmoe::kDecodeMaxT
                                                       ? tmoe::sk_decode_flags(p->s.r3) : 0,
-                                                  tmoe::front_sliced_flags(T, L.fsplit))) *
+                                                  tmoe::front_sliced_flags(T, L.fsplit, (int64_t)p->es))) *
                          sizeof(uint32_t));
   L.total = o;
   return L;
@@ -816,7 +816,7 @@ int tmoe_forward_glu(const tmoe_plan* p, const void* x, int64_t T, const void* p
     }
     return TMOE_OK;
   }
-  const Launch mid = fold ? launch_cz : tmoe::launch_core;
+  const Launch mid = p->fold ? launch_cz : tmoe::launch_core;
   if ((e = tmoe::launch_front_pair(g, u, st)) != hipSuccess ||
       (e = mid(g, st)) != hipSuccess || (e = mid(u, st)) != hipSuccess ||
       (e = tmoe::launch_outproj(g, st)) != hipSuccess ||
@@ -946,7 +946,7 @@ int tmoe_forward_path(const tmoe_plan* p, int64_t T) {
       return TMOE_PATH_DECODE;
     return TMOE_PATH_SMALL;
   }
-  if (p->fold || L.osplit > 0) {
+  if (p->fold) {
     const tmoe::FwdArgs f = folded_args(p, a, fake, nullptr);
     if (!(p->s.flags & TMOE_FLAG_NO_FUSE) && tmoe::fused_large_shape_ok(f)) return TMOE_PATH_FUSED;
     if (!(p->s.flags & TMOE_FLAG_NO_FUSE) && tmoe::fused_mid_shape_ok(f))

@@ -181,10 +181,11 @@ inline int front_split(int64_t T, int64_t d_in, int64_t E_pad, int64_t es) {
   if (s > kMaxFrontPlanes) s = kMaxFrontPlanes;
   return s > 1 ? (int)s : 1;
 }
-// signal flags of the K-sliced front in one launch: one per (64-token tile, slice)
-// for the slice, and (k_fused_mid) one more per (tile, slice) for its epilogue
-inline int64_t front_sliced_flags(int64_t T, int split) {
-  return split > 1 ? 2 * ((T + 63) / 64) * split : 0;
+// signal flags of the K-sliced front in one launch: one per (tile of front_slice_rows,
+// slice) for the slice, and (k_fused_mid, bf16) one more per (tile, slice) for its epilogue
+inline int64_t front_sliced_flags(int64_t T, int split, int64_t es) {
+  const int64_t rows = front_slice_rows(es), tiles = (T + rows - 1) / rows;
+  return split > 1 ? (es == 2 ? 2 : 1) * tiles * split : 0;
 }
 
 // Output tiles (256 tokens x 64 channels) of the grouped core and the split S of
@@ -219,10 +220,10 @@ inline bool core_p_supported(int64_t r1, int64_t r2, bool bf16, bool fp8w) {
 }
 
 // Folded batches between the decode launch and the large-tile kernels (kDecodeMaxT < T <=
-// kSmallT): folded plans (batch_fold_pays), and plans with decode_fold's W^T whose 64 x 128 out-projection tiles
-// number at most kBatchFoldTiles (one a compute unit; past it the fold's extra multiply-adds,
-// 3 times as many at the reference's 1536 -> 6144, outweigh the core's launches). The front's
-// per-token epilogue writes c (x) z; the out-projection is a plain GEMM of it against W^T, K
+// kSmallT): folded plans (batch_fold_pays), and plans with decode_fold's W^T whose 64 x 128
+// out-projection tiles number at most kBatchFoldTiles (one a compute unit; past it the fold's
+// extra multiply-adds, 3 times as many at the reference's 1536 -> 6144, outweigh the core's
+// launches). The front's per-token epilogue writes c (x) z; the out-projection is a plain GEMM of it against W^T, K
 // in slices of at least 4 K tiles of 64 while the tiles leave compute units idle. Per layer,
 // before and now: 1536 -> 6144 at T = 65 43.3 -> 27.3 us, 256 53.3 -> 30.5; the output
 // sub-block 50-54 -> 34; the folded 1536 -> 2304 layer at T = 128 31.8 -> 22.5, 256 39.2 ->

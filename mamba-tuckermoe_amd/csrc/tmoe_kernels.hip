@@ -883,11 +883,11 @@ constexpr int64_t kLatMinChunk = 256;   // entries of a dG chunk, but for an exp
 bool latent_grouped_shape(int64_t E, int64_t r3, int64_t r2) {
   return r3 % 128 == 0 && r2 % 128 == 0 && E <= dev::kLatMaxE;
 }
-// dx / dp (and the forward, latent_pairs_forward) by pairs of experts: k <= 2, and the row tiles' products (each of
-// the E (E + 1) / 2 pairs pads half a tile on average) well below the dense form's E per
-// token. The grouped kernels reach about 0.45 of the dense ones' rate (420 against 970
-// TFLOP/s forward at 16384 tokens) but skip dx / dp's pass over H, so the line is drawn at
-// 1.3 products of the grouped form against one of the dense.
+// dx / dp (and the forward, latent_pairs_forward) by pairs of experts: k <= 2, and the row
+// tiles' products (each of the E (E + 1) / 2 pairs pads half a tile on average) well below the
+// dense form's E per token. The grouped kernels reach about 0.45 of the dense ones' rate (440
+// against 1010 TFLOP/s forward at 16384 tokens) but skip dx / dp's pass over H, so the line is
+// drawn at 1.3 products of the grouped form against one of the dense.
 bool latent_pairs(const LatentArgs& l) {
   if (l.dtype != kDtypeBF16 || l.k > 2 || !latent_grouped_shape(l.E, l.r3, l.r2)) return false;
   const int64_t keys = l.k == 2 ? l.E * (l.E + 1) / 2 : l.E;
@@ -1025,7 +1025,6 @@ hipError_t launch_latent_sort(const LatentArgs& l, const LatentLayout& L, bool p
   if (exp) {
     const int64_t c = cdiv(l.B * l.k, L.chunk_target);
     q.chunk = (int)(c < kLatMinChunk ? kLatMinChunk : c);
-    q.max_chunks = (int)L.max_chunks;
     q.chunks = reinterpret_cast<int4*>(ws + L.chunks);
     q.exp_chunks = reinterpret_cast<int2*>(ws + L.exp_chunks);
     q.etok = reinterpret_cast<int*>(ws + L.etok);

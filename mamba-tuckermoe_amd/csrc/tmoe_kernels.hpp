@@ -2249,7 +2249,9 @@ __global__ __launch_bounds__(64 * WM * WN) void k_outproj_pp(FwdArgs a) {
 // ---- packing kernels -----------------------------------------------------
 // k_fold_out_t without scales, on the MFMAs: a 128 (rows n) x 128 (kk) tile of W^T a
 // work-group of 4 waves, K tiles of 64 q; uoutT's rows are q-contiguous, coreT's are K steps
-// (tr_frag). fp32 sums, one rounding. Packing a layer of K 1024, d_out 2304, r2 1024: 254 us
+// (tr_frag). fp32 sums in the MFMAs' order, one rounding (k_fold_out_t adds in q order: some
+// entries round the other way, 1.3e-4 to 1.8e-4 between layers of either, both as far from
+// exact). Packing a layer of K 1024, d_out 2304, r2 1024: 254 us
 // with k_fold_out_t, 46 with this kernel.
 __global__ __launch_bounds__(256, 2) void k_fold_out_mfma(const uint16_t* __restrict__ coreT,
                                                           const uint16_t* __restrict__ uoutT,

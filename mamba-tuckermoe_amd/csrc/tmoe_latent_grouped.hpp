@@ -16,10 +16,14 @@
 //   k_latent_finish  dG = the sum of each expert's planes, in chunk order;
 //                    dp = the sum of its column tiles' parts
 //
-// Measured at 16384 tokens, E 8, k 2, r3 256, r2 1024 (kernel trace, MI355X), against the
-// dense kernels: forward 41 us (dense 71), dx and dp 44 (H 96, dx / dp 32), dG 37 + xs 7 +
-// planes 8 (dense 140 + transposes 37 + planes 6), the sort 12 in each direction (counts 5,
-// with the forward's transpose of G beside them); a forward and backward 346 -> 145 us.
+// Measured at 16384 tokens, E 8, k 2, r3 256, r2 1024 (MI355X; one kernel trace of either form):
+//   forward    pairs 38.7, sort 12.3, G's transpose among its counts (dense: product 67.8, G
+//              transposed 5.6, weights 4.3)
+//   dx and dp  39.1 (dense: H 83.5, dx / dp 30.9)
+//   dG         xs 6.8, products 35.5, planes and dp 8.7, both sorts of the backward 10.9 (dense:
+//              transposes 34.8, products 132.8, planes 5.3, weights and the zero bias 7.9)
+// These kernel times add to 152 us (dense 373); a forward and backward in a stream without the
+// trace take 149 (dense 348).
 //
 // The sort is a stable counting sort on integers, so every sum has a fixed order. An
 // index outside [0, E) selects nothing (weight 0, dp 0).
@@ -43,7 +47,6 @@ struct LatentSort {
   int E, k;
   int pair_blocks, exp_blocks;  // work-groups of each sort (exp_blocks 0: forward)
   int chunk;                    // entries per dG chunk (at most)
-  int max_chunks;
   int *pair_hist, *exp_hist;    // key counts per work-group
   int* meta;                    // [0]: row tiles, [1]: dG chunks
   int4* tiles;                  // (start, tokens, expert lo, expert hi) per row tile
@@ -328,9 +331,10 @@ struct LatentPair {
 // each slot's expert. 4 waves of 64 x 64; with two slots a wave's two column blocks are
 // the same 32 columns of its slots' products, so that the weighted sum and dp stay in
 // a lane. Bound by the latency of one K tile's DMA (about 1.2 us a K tile and round of
-// work-groups), not by its 17 GFLOP (7 us) or its 306 MB from L2. Both operands arrive by LDS DMA (the token rows gathered by each lane's own
-// row addresses) in two stages of one 64-wide K tile; 64 KB of LDS and <= 256 registers
-// a wave put two work-groups on a compute unit, one's loads under the other's MFMAs.
+// work-groups), not by its 17 GFLOP (7 us) or its 306 MB from L2. Both operands arrive by LDS
+// DMA (the token rows gathered by each lane's own row addresses) in two stages of one 64-wide
+// K tile; 64 KB of LDS and <= 256 registers a wave put two work-groups on a compute unit,
+// one's loads under the other's MFMAs.
 template <int NSLOT, bool BWD>
 __global__ __launch_bounds__(256, 2) void k_latent_pair(LatentPair q) {
   constexpr int CS = 128 / NSLOT;
@@ -369,8 +373,8 @@ __global__ __launch_bounds__(256, 2) void k_latent_pair(LatentPair q) {
   // this lane's rows: the slots' probabilities, in the tile's expert order, and (backward)
   // its x values
   float pw[2][NSLOT];
-  int64_t src[2];         // b k (+ the slot of the pair's first expert in bit 62)
-  bool sw[2];
+  int64_t src[2];         // b k
+  bool sw[2];             // the pair's first expert is the token's slot 1
   uint2 xv[2][NSLOT == 2 ? 4 : 8];
 #pragma unroll
   for (int i = 0; i < 2; ++i) {
