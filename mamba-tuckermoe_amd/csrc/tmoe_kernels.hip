@@ -505,11 +505,18 @@ hipError_t launch_small_decode_t(const FwdArgs& a, hipStream_t st) {
   const dim3 block(64 * kSkW), grid((kPart != dev::kDecodeConsumers ? producers : 0) +
                                     (kPart != dev::kDecodeProducers ? cdiv(a.d_out, 16) : 0));
   const size_t dyn = dev::sk_decode_dyn_bytes(MF, a);
-  if (kPart != dev::kDecodeProducers &&
-      a.r1 * a.r3 * (int64_t)sizeof(typename Elt::T) > 2048)   // over one K group a wave
-    hipLaunchKernelGGL((dev::k_sk_decode<Elt, MF, kSkW, 2, kPart>), grid, block, dyn, st, b);
-  else
-    hipLaunchKernelGGL((dev::k_sk_decode<Elt, MF, kSkW, 1, kPart>), grid, block, dyn, st, b);
+  // two K groups a wave, both loaded before the wait, where the consumers are one round of the
+  // compute units and up to 32 tokens leave the registers: 2304 columns, K 2048 T = 1 8.35 -> 8.1
+  // us, T = 32 10.3 -> 9.9. Elsewhere one at a time is as fast or faster: K 4096, 9216 columns T =
+  // 32 36.4 -> 34.6, T = 64 55.9 -> 52.5; K 2048, 14352 columns T = 1 25.8 -> 23.5, T = 48 44.9 -> 41.5
+  if constexpr (kPart != dev::kDecodeProducers && MF <= 2) {
+    const int64_t row = a.r1 * a.r3 * (int64_t)sizeof(typename Elt::T);
+    if (row > 2048 && row <= 4096 && a.d_out <= 16 * kCoreUnits) {
+      hipLaunchKernelGGL((dev::k_sk_decode<Elt, MF, kSkW, 2, kPart>), grid, block, dyn, st, b);
+      return hipGetLastError();
+    }
+  }
+  hipLaunchKernelGGL((dev::k_sk_decode<Elt, MF, kSkW, 1, kPart>), grid, block, dyn, st, b);
   return hipGetLastError();
 }
 

@@ -707,9 +707,8 @@ __device__ __forceinline__ void route_row16(const FwdArgs& a, int64_t t, int sl,
 }
 
 // GB: K groups (64 elements in bf16, 32 in fp32) a consumer wave's weight loads hold at
-// once, issued before the wait: 2 where K gives each of the 16 waves more than one. One token
-// block (MF = 1) stays within 64 registers, so that two work-groups fit a compute unit (d_out
-// 4608: 356 of them).
+// once, issued before the wait (launch_small_decode_t has the rule). One token block (MF = 1)
+// stays within 64 registers, so that two work-groups fit a compute unit (d_out 4608: 356 of them).
 // kPart: the whole layer (kDecodeAll), or under graph capture, where no flag may be waited for,
 // the producers and the consumers as a launch each: the same code, so the same bits.
 constexpr int kDecodeAll = 0, kDecodeProducers = 1, kDecodeConsumers = 2;
