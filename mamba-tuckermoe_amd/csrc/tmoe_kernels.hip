@@ -768,15 +768,16 @@ hipError_t launch_eye(float* dst, int64_t n, hipStream_t st) {
 
 hipError_t launch_outproj(const FwdArgs& a, hipStream_t st) {
   if (a.dtype == kDtypeBF16) return launch_outproj_bf16(a, st);
-  // fp32: the tile whose rounds of the compute units take least, in 64 x 64 units (the
-  // fp32 MFMAs bound every tile alike; 1021 x 6144 x 512: 64 x 128 tiles, three rounds,
-  // 60.5 us against 73.5 for 128 x 128, one and a half; T = 257, d_out 2304, K 1024: the
-  // layer 64 us with 64 x 64 tiles, 81 with 64 x 128)
+  // fp32: the tile whose rounds of the compute units take least, in 64 x 64 units (1021 x 6144 x
+  // 512: 64 x 128 tiles, three rounds, 60.5 us against 73.5 for 128 x 128, one and a half; T = 257,
+  // d_out 2304, K 1024: the layer 64 us with 64 x 64 tiles, 81 with 64 x 128). A unit takes the 64 x
+  // 64 tiles some 6% longer, so that they must save a sixteenth: 6500 x 6144, K 512 in 39 of their
+  // rounds against 40 units of 128 x 128 the layer takes 464 : 449 us, 2500 x 4608 (12 : 12) 171 : 170
   const int64_t ncu = cu_count(), m64 = cdiv(a.T, 64);
   const int64_t r1 = cdiv(m64 * cdiv(a.d_out, 64), ncu);
   const int64_t r2 = 2 * (int64_t)cdiv(m64 * cdiv(a.d_out, 128), ncu);
   const int64_t r4 = 4 * (int64_t)cdiv((int64_t)cdiv(a.T, 128) * cdiv(a.d_out, 128), ncu);
-  if (r1 < r2 && r1 < r4) return launch_outproj_t<EltF32, OutCfgF32XS>(a, st);
+  if (16 * r1 < 15 * (r2 < r4 ? r2 : r4)) return launch_outproj_t<EltF32, OutCfgF32XS>(a, st);
   return r2 < r4 ? launch_outproj_t<EltF32, OutCfgF32S>(a, st)
                  : launch_outproj_t<EltF32, OutCfgF32>(a, st);
 }
