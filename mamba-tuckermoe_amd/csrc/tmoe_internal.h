@@ -245,13 +245,19 @@ inline int batch_out_split(int64_t T, int64_t d_out, int64_t K) {
 // That one needs no pass over K slices, and its time goes by its rounds of 16-column work-
 // groups over blocks of 64 tokens (one a compute unit) and by K. Layer, us, skinny : batch at
 // d_in 768: one round (d_out 768, 64 < T <= 256) 19.5 : 19.4-20.3 at K 1024, 17 : 19.5 at K 512,
-// 29 : 19.5 at K 2048; K of one slice 15.5 : 15; two rounds (d_out 2304) T = 65 19.5 : 19.9, 72
-// 19.9 : 20.0, 80 20.9 : 20.4, 128 27 : 21.5, 256 35 : 23; 4096 columns, T = 65 23.5 : 21.7
-// (its second round is full). Where the batch slices the front it is faster at any of these.
+// 29 : 19.5 at K 2048; K of one slice 17.1 : 17.8 (K 384), 16.8 : 17.0 (256), 16.0 : 16.1 (128); two
+// rounds of one slice 18.4 : 15.1 (K 256, d_out 2304, T = 128). A second round of few work-groups or
+// few tokens is short: d_out 2304 T = 65 19.5 : 19.9, 80 23.0 : 21.4 at K 1024, 20.1 : 21.0 at 512, 96
+// 25.4 : 21.9 and 20.9 : 21.0; d_out 3072 (128 of them) T = 80 21.7 : 21.0 at K 512; 4096 columns, T =
+// 65 23.5 : 21.7 (its second round is full). Where the batch slices the front it is faster at any of
+// these.
 inline bool batch_fold_pays(int64_t T, int64_t d_out, int64_t K, int front_slices) {
-  if (front_slices > 1 || K > 1024 || batch_out_split(T, d_out, K) == 1) return true;
+  if (front_slices > 1 || K > 1024) return true;
   const int64_t cols = (d_out + 15) / 16, blocks = (T + 63) / 64, last = T - 64 * (blocks - 1);
-  return cols * blocks > kCoreUnits && (last >= 16 || cols * (blocks - 1) >= kCoreUnits);
+  const int64_t past = cols * blocks - kCoreUnits;   // work-groups of the skinny second round
+  if (past <= 0) return false;
+  if (batch_out_split(T, d_out, K) == 1 || cols * (blocks - 1) >= kCoreUnits) return true;
+  return last >= (K >= 1024 || past >= 64 ? 16 : 32);
 }
 
 // The latent expert contraction of the training module (tmoe_latent.hpp) and its

@@ -26,15 +26,19 @@ def test_batch_front_slices(pkg, E, d_in, sliced):
 
 
 # a folded plan takes the batch form (d_out, K = r1 r3, T): in one round of the skinny
-# out-projection's work-groups not, unless K is past 1024 or of one slice; in two rounds from
-# 16 tokens in the last block of 64 on, or where the blocks before it fill the chip
+# out-projection's work-groups not, unless K is past 1024; in two rounds with one K slice, or
+# from 16 tokens in the last block of 64 on (32 where K is short and the second round few), or
+# where the blocks before it fill the chip
 @pytest.mark.parametrize("d_out,r1,r3,T,batch", [
     (768, 4, 256, 65, False), (768, 4, 256, 256, False), (1024, 4, 256, 256, False),
     (1040, 4, 256, 256, True), (1040, 4, 256, 192, False), (1040, 4, 256, 207, False),
     (1040, 4, 256, 208, True), (2048, 4, 256, 128, False), (2064, 4, 256, 79, False),
     (2064, 4, 256, 80, True), (4080, 4, 256, 65, False), (4096, 4, 256, 65, True),
-    (768, 2, 256, 128, False), (768, 4, 128, 128, False), (768, 1, 256, 65, True),
-    (768, 4, 64, 256, True),
+    (768, 2, 256, 128, False), (768, 4, 128, 128, False), (768, 1, 256, 65, False),
+    (768, 4, 64, 256, False), (1040, 4, 64, 256, True), (2048, 1, 256, 65, False),
+    (2064, 1, 256, 65, True), (2064, 6, 64, 65, True), (2064, 2, 256, 95, False),
+    (2064, 2, 256, 96, True), (2304, 3, 256, 95, False), (2544, 3, 256, 95, False),
+    (2560, 3, 256, 80, True), (2560, 3, 256, 79, False), (4096, 2, 256, 65, True),
 ])
 def test_folded_plan_batches(pkg, d_out, r1, r3, T, batch):
     f = pkg._lib

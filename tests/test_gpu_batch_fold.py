@@ -50,7 +50,8 @@ def _check(m, x, dev, ref, k):
 # of a rule's edge: folded with a sliced and with the small front, a wide router, a ragged last
 # column tile; folded in one round of the skinny out-projection (no batch); the reference's
 # ranks at the smallest T, one row past a tile, the last T of the range and the first past it;
-# 256 tiles and past them (the two GEMMs); rank 4 unfolded; K = 64 (one slice)
+# 256 tiles and past them (the two GEMMs); rank 4 unfolded; K = 64 (one slice) in one round
+# (no batch) and in two; K 768 on both sides of its line
 @pytest.mark.parametrize("shape,Ts,others", [
     ((16, 2, 4, 256, 1024, 1536, 2304), (65, 129, 200, 256), (64, 257)),
     ((64, 4, 4, 256, 1024, 512, 2320), (80, 255), (65, 79)),
@@ -60,7 +61,8 @@ def _check(m, x, dev, ref, k):
     ((8, 2, 4, 256, 512, 768, 4608), (129, 250), ()),
     ((8, 2, 8, 256, 256, 256, 8192), (192, 193, 256), ()),
     ((8, 2, 8, 64, 64, 256, 10880), (192,), (193,)),
-    ((4, 1, 1, 64, 256, 256, 64), (70, 256), ()),
+    ((4, 1, 1, 64, 256, 256, 64), (), (70, 256)), ((4, 1, 1, 64, 256, 256, 4112), (65, 70, 256), ()),
+    ((4, 2, 3, 256, 1024, 256, 2304), (96, 250), (65, 95)),
 ], ids=lambda v: str(v))
 def test_batch_fold(pkg, dev, shape, Ts, others):
     for T in Ts + others:
