@@ -145,7 +145,8 @@ bool batch_folded(const tmoe_plan* p, int64_t T) {
 // launch (tmoe::decode_fold_pays).
 bool decode_folded(const tmoe_plan* p, int64_t T) {
   return p->decode_fold && T <= tmoe::kDecodeMaxT &&
-         tmoe::decode_fold_pays(T, p->rk, p->s.r3, p->s.r2, p->s.d_out, (int64_t)p->es);
+         tmoe::decode_fold_pays(T, p->s.d_in, p->rk, p->s.r3, p->s.r2, p->s.d_out,
+                                (int64_t)p->es);
 }
 
 // lean: without the fp32 plans' K slices (their planes) and without folded batches, for a
@@ -462,7 +463,7 @@ int tmoe_plan_create(const tmoe_shape* shape, tmoe_plan** plan_out) {
   if (p->core_p) { p->off_core_p = o; o = align256(o + (size_t)p->rk * s.r2 * s.r3 * p->es); }
   p->off_fold = 0;
   p->decode_fold = !p->fold && !(s.flags & TMOE_FLAG_NO_FOLD) &&
-                   tmoe::decode_fold_ok(s.E, p->rk, s.r3, s.r2, s.d_out, (int64_t)p->es);
+                   tmoe::decode_fold_ok(s.E, s.d_in, p->rk, s.r3, s.r2, s.d_out, (int64_t)p->es);
   if (p->fold || p->decode_fold) {
     p->off_fold = o;
     o = align256(o + (size_t)s.d_out * K * p->es);

@@ -322,37 +322,46 @@ constexpr int64_t kDecodeFoldK = 2048, kDecodeFoldBytes = 32 << 20;
 // Whether T <= kDecodeMaxT tokens of such a plan are faster folded. The launch's 16-column
 // work-groups take one, two, three rounds of the compute units at 4096, 8192, 12288
 // columns; each round stages T rows of z and reads its share of W^T, which holds `extra` bytes
-// more than core and U_out together. Kernel time, us, folded : two GEMMs, bf16 but where said,
-// r3 = 256, over 1680 measured (plan, T); W^T warm, cold ones of 600 MB in turn cross at the same lines:
+// more than core and U_out together. What it saves are the two GEMMs' launches, the longer the
+// more core_width = rk r2 and, past 32 tokens, d_in. Kernel time, us, folded : two GEMMs, bf16,
+// d_in 768 and r3 256 but where said, over 4134 measured (plan, T), of which the rule folds 3506 and
+// one of these is more than 2.5% slower; with cold weights (600 MB of layers in turn) the lines are
+// the same:
 //   one round: folded always (K 2048, 2304 columns T = 1 8.3 : 14, T = 64 16 : 36)
 //   two, T <= 32: K 2048, 8192 columns, T = 1: r2 64 (31 MB extra) 15.3 : 12.7, 256 (28) 14.3 : 13.1,
-//     512 (23) 15.1 : 14.3, 1024 (13) 15.1 : 15.5; K 1024, r2 512 (7) 11 : 13
-//   two, T > 32: 64 tokens at rank 2, 8192 columns 25.7 : 23.5, 6144 22.7 : 24; rank 4, r2 64
-//     27.5 : 26.2, r2 512 28 : 30; rank 2 in fp32 31.1 : 33.1
-//   three: rank 4, r2 512, 12288 columns T = 32 24.7 : 25.7, T = 48 34.2 : 31.1; rank 2 T = 24 21.0 :
-//     20.3; r2 64 (23 MB) T = 1 14.8 : 13.6; r3 = 128, K 512 T = 1 13.3 : 13.8, T = 64 27.7 : 27.5;
-//     r3 = 64, K 1024, r2 256 (18 MB) T = 1 14.2 : 13.8, T = 24 18.1 : 20.1
+//     512 (23) 15.1 : 14.3, 1024 (13) 15.1 : 15.5; r3 128, r2 512 (23) T = 1 14.8 : 14.4, T = 32 19.6 : 23.0
+//   two, 64 tokens: rank 2, r2 256, 8192 columns 25.7 : 23.5, 6144 22.7 : 24; rank 4, r2 64 27.5 : 26.2,
+//     r2 512 28 : 30; d_in 128: rank 6, r2 256, 7168 columns 29.2 : 26.6, rank 4, r2 512 27 : 28; d_in
+//     1536: folded always; fp32, d_in 128: rank 4, r2 256, 8192 columns 37.2 : 35.3
+//   three: rank 4, r2 512, 12288 columns T = 32 24.7 : 25.7, T = 48 34.2 : 31.1; rank 3, r2 256 T = 32
+//     21.1 : 20.4; fp32 rank 3, r2 512, T = 1 19.3 : 17.6; r3 128, K 256, r2 64, 12288 columns T = 1 13.3 :
+//     13.1, T = 32 16.2 : 19.2, T = 64 25.6 : 20.9 (d_in 128)
 //   four: 16384 columns, rank 4, r2 512 T = 1 19 : 15, T = 64 51 : 36
-inline bool decode_fold_pays(int64_t T, int64_t rk, int64_t r3, int64_t r2, int64_t d_out,
-                             int64_t es) {
-  const int64_t rounds = (d_out + 4095) / 4096, K = rk * r3;
+inline bool decode_fold_pays(int64_t T, int64_t d_in, int64_t rk, int64_t r3, int64_t r2,
+                             int64_t d_out, int64_t es) {
+  const int64_t rounds = (d_out + 4095) / 4096, K = rk * r3, core_width = rk * r2;
   if (rounds <= 1) return true;
   if (rounds > 3) return false;
   const int64_t extra = es * (K * d_out - r2 * (K + d_out));
-  const bool small_core = r3 == 256 && rk * r2 <= 512;   // the two GEMMs' middle launch is short
   if (rounds == 2) {
-    if (T <= 32) return extra <= 19000000;
-    return d_out <= 6144 || es == 4 || !small_core;
+    if (T <= 32) return extra <= (r3 == 256 ? 19000000 : 24000000);
+    if (r3 < 256 || d_in >= 1024) return true;
+    const bool wide = d_in >= 512;
+    if (es == 4) return core_width > (wide || d_out <= 6144 ? 256 : 1024);
+    return core_width > (wide ? 512 : 1536) || (wide && d_out <= 6144);
   }
-  if (r3 == 256) return T <= 32 && !small_core && extra <= 12000000;
-  return T > 16 || extra <= 12000000;
+  if (r3 == 256) return es == 2 && T <= 32 && core_width > 1024 && extra <= 12000000;
+  if (T <= 16) return core_width > 512 && extra <= 12000000;
+  if (T <= 32) return true;
+  return core_width > 1024 || (d_in >= 512 && core_width > 512) ||
+         (d_in >= 1024 && (core_width >= 512 || r3 == 64));
 }
-inline bool decode_fold_ok(int64_t E, int64_t rk, int64_t r3, int64_t r2, int64_t d_out,
-                           int64_t es) {
+inline bool decode_fold_ok(int64_t E, int64_t d_in, int64_t rk, int64_t r3, int64_t r2,
+                           int64_t d_out, int64_t es) {
   if (E > 16 || rk > 32 || rk * r3 > kDecodeFoldK || rk * r3 * d_out * es > kDecodeFoldBytes)
     return false;
   for (int64_t T : {16, 32, 64})   // one of each range of the rule
-    if (decode_fold_pays(T, rk, r3, r2, d_out, es)) return true;
+    if (decode_fold_pays(T, d_in, rk, r3, r2, d_out, es)) return true;
   return es == 2 && batch_out_tiles(kDecodeMaxT + 1, d_out) <= kBatchFoldTiles;
 }
 // floats of its scratch at FwdArgs::raw: z columns (T, r3), c (T, r1)

@@ -62,30 +62,37 @@ def test_other_batches(pkg):
         assert _form(pkg, T, d_in=768, d_out=768, r1=32, r2=512, flags=f.TMOE_FLAG_NO_FOLD) == 0
     shape = dict(d_in=256, d_out=10880, r1=8, r2=64, r3=64)
     assert _form(pkg, 192, **shape) == both and _form(pkg, 193, **shape) == 0
-    assert _form(pkg, 64, **shape) == f.TMOE_FORM_FOLDED and _form(pkg, 0, **shape) == 0
+    assert _form(pkg, 32, **shape) == f.TMOE_FORM_FOLDED and _form(pkg, 0, **shape) == 0
+    assert _form(pkg, 64, **shape) == 0
 
 
-# plans that are not folded otherwise, by rounds of 4096 columns: (r1, r3, r2, d_out, dtype) and
-# the T of 16, 17, 32, 33, 64 that run folded
+# plans that are not folded otherwise, by rounds of 4096 columns: (d_in, r1, r3, r2, d_out, dtype)
+# and the T of 16, 17, 32, 33, 64 that run folded
 BF, F32 = torch.bfloat16, torch.float32
-ALL, UP32, FROM33 = (16, 17, 32, 33, 64), (16, 17, 32), (33, 64)
+ALL, UP32, FROM33, MID, FROM17 = (16, 17, 32, 33, 64), (16, 17, 32), (33, 64), (17, 32), (17, 32, 33, 64)
 
 
-@pytest.mark.parametrize("r1,r3,r2,d_out,dtype,folded", [
-    (8, 256, 64, 4096, BF, ALL), (2, 256, 256, 4096, F32, ALL),        # one round
-    (8, 256, 512, 6144, BF, ALL), (8, 256, 256, 8192, BF, FROM33),     # two: W^T's extra bytes
-    (8, 256, 512, 8192, BF, FROM33), (8, 256, 1024, 8192, BF, ALL), (4, 256, 512, 8192, BF, ALL),
-    (2, 256, 256, 8192, BF, UP32), (2, 256, 256, 6144, BF, ALL),       # two: a short core
-    (2, 256, 256, 8192, F32, ALL), (2, 128, 256, 8192, BF, ALL),
-    (4, 256, 512, 9216, BF, UP32), (4, 256, 512, 12288, BF, UP32),     # three
-    (2, 256, 256, 9216, BF, ()), (4, 256, 64, 9216, BF, ()), (4, 128, 256, 12288, BF, ALL),
-    (16, 64, 256, 12288, BF, (17, 32, 33, 64)), (2, 256, 256, 9216, F32, ()),
-    (4, 256, 512, 12304, BF, ()), (2, 256, 256, 16384, BF, ()),        # four
+@pytest.mark.parametrize("d_in,r1,r3,r2,d_out,dtype,folded", [
+    (768, 8, 256, 64, 4096, BF, ALL), (128, 2, 256, 256, 4096, F32, ALL),        # one round
+    (768, 8, 256, 512, 6144, BF, ALL), (768, 8, 256, 256, 8192, BF, FROM33),     # two: W^T's extra bytes
+    (768, 8, 256, 512, 8192, BF, FROM33), (768, 8, 256, 1024, 8192, BF, ALL),
+    (768, 4, 256, 512, 8192, BF, ALL), (768, 16, 128, 512, 8192, BF, ALL),
+    (768, 2, 256, 256, 8192, BF, UP32), (768, 2, 256, 256, 6144, BF, ALL),       # two: a short core
+    (1024, 2, 256, 256, 8192, BF, ALL), (448, 2, 256, 256, 6144, BF, UP32),
+    (448, 4, 256, 256, 4112, BF, UP32), (448, 4, 256, 512, 8192, BF, ALL), (128, 2, 128, 256, 8192, BF, ALL),
+    (768, 2, 256, 256, 8192, F32, ALL), (448, 2, 256, 256, 8192, F32, UP32),
+    (448, 2, 256, 256, 6144, F32, ALL), (768, 1, 256, 64, 8192, F32, UP32),
+    (768, 4, 256, 512, 9216, BF, UP32), (768, 4, 256, 512, 12288, BF, UP32),     # three
+    (768, 4, 256, 256, 9216, BF, ()), (768, 4, 256, 512, 8208, F32, ()),
+    (768, 4, 128, 256, 12288, BF, ALL), (448, 4, 128, 256, 12288, BF, UP32),
+    (768, 4, 128, 64, 9216, BF, MID), (768, 8, 64, 64, 9216, BF, MID), (1024, 8, 64, 64, 9216, BF, FROM17),
+    (768, 16, 64, 256, 12288, BF, FROM17),
+    (768, 4, 256, 512, 12304, BF, ()), (768, 2, 256, 256, 16384, BF, ()),        # four
 ])
-def test_decode_forms(pkg, r1, r3, r2, d_out, dtype, folded):
+def test_decode_forms(pkg, d_in, r1, r3, r2, d_out, dtype, folded):
     f = pkg._lib
     for T in ALL:
-        got = _form(pkg, T, d_in=768, d_out=d_out, E=16, r1=r1, r3=r3, r2=r2, dtype=dtype)
+        got = _form(pkg, T, d_in=d_in, d_out=d_out, E=16, r1=r1, r3=r3, r2=r2, dtype=dtype)
         assert got == (f.TMOE_FORM_FOLDED if T in folded else 0), T
 
 

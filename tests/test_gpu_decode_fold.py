@@ -19,7 +19,7 @@ SHAPES = [
     (8, 2, 32, 256, 512, 768, 768), (8, 2, 32, 256, 512, 768, 4608),
     (8, 2, 4, 256, 512, 768, 4608), (16, 3, 32, 64, 64, 256, 1040),
     (16, 16, 3, 64, 64, 512, 272), (4, 1, 64, 128, 64, 1536, 128),
-    (8, 2, 8, 256, 256, 256, 8192), (16, 2, 4, 128, 256, 256, 12288),
+    (8, 2, 8, 256, 256, 256, 8192), (16, 2, 4, 128, 256, 512, 12288),
 ]
 
 
