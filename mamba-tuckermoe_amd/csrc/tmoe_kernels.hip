@@ -902,12 +902,13 @@ bool latent_pairs(const LatentArgs& l) {
   return 13 * (l.B + keys * (dev::kLatBM / 2)) * l.k <= 10 * l.B * l.E;
 }
 // The forward has no pass over H to skip, so that it also weighs its own two forms, in us
-// fitted to 326 measured pairs (E 2 to 16, k 1 and 2, ranks 128 and 256 x 128 to 2048, 64 to 65536
-// tokens; the dense fit within 10%, the grouped one within 17%, the slower form taken by more
-// than 3% in four cases): the dense one by its rounds of 256 x 256 tiles and its K, the grouped
-// one by its padded rows. dense : grouped at 16384 and 32768 tokens: E 2, k 1, 256 x 1024 31 : 34 and
-// 51 : 49, 128 x 512 19 : 24 and 23 : 31; E 3, k 2, 256 x 1024 40 : 44 and 66 : 72; E 4, k 2, 256 x 1024
-// 46 : 45 and 80 : 72, 128 x 512 25 : 26 and 29 : 38; E 8, k 2, 256 x 1024 71 : 47 and 130 : 75.
+// fitted to 890 measured pairs (E 2 to 6, k 1 and 2, ranks 128 and 256 x 128 to 2048, 300 to 65536
+// tokens; the dense fit within 3%, the grouped one within 6%, whence the 3% in its disfavour: the
+// slower form by more than 2.5% in none, the faster one left by more than 6% in ten): the dense
+// one by its rounds of 256 x 256 tiles and its K, the grouped one by its padded rows. dense : grouped
+// at 16384 and 32768 tokens: E 2, k 1, 256 x 1024 31 : 34 and 51 : 49, 128 x 512 19 : 24 and 23 : 31, 128 x
+// 2048 41 : 43; E 3, k 2, 256 x 1024 40 : 44 and 66 : 72; E 4, k 2, 256 x 1024 46 : 45 and 80 : 72, 128 x 512
+// 25 : 26 and 29 : 38; E 8, k 2, 256 x 1024 71 : 47 and 130 : 75.
 bool latent_pairs_forward(const LatentArgs& l) {
   if (!latent_pairs(l)) return false;
   const int64_t keys = l.k == 2 ? l.E * (l.E + 1) / 2 : l.E, ncu = cu_count();
@@ -915,14 +916,14 @@ bool latent_pairs_forward(const LatentArgs& l) {
   const double K = (double)(l.E * l.r3), out = (double)l.B * l.r2;
   // a round that leaves half of the compute units idle runs its tiles faster
   const double dense = 9 + 0.39e-6 * out +
-                       (2 * tiles <= ncu ? 2.7 + 0.0235 * K
-                                         : (double)cdiv(tiles, ncu) * (1.2 + 0.0266 * K));
+                       (2 * tiles <= ncu ? 2.8 + 0.025 * K
+                                         : (double)cdiv(tiles, ncu) * (1.8 + 0.029 * K));
   const double rows = (double)(l.B + keys * (dev::kLatBM / 2)), cols = (double)(l.k * l.r2);
   // an output past the last-level cache: its rows are stored in 128-byte pieces
-  const double spill = out * 2 > 134e6 ? 0.6e-6 * (out * 2 - 134e6) : 0;
-  const double grouped =
-      14.3 + rows * (0.18e-3 + cols * (0.24e-6 + 2.4e-9 * (double)l.r3)) + spill;
-  return grouped <= dense;
+  const double spill = out * 2 > 134e6 ? 0.24e-6 * (out * 2 - 134e6) : 0;
+  const double grouped = 15 + rows * (0.12e-3 + cols * (0.225e-6 + 2.43e-9 * (double)l.r3)) +
+                         0.3e-6 * out + spill;
+  return 1.03 * grouped <= dense;
 }
 // dG over each expert's own entries: below the dense form's B E rows. With many slots the sort
 // of the B k entries (64 work-groups) and their scaled rows outgrow what the narrower products

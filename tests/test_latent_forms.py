@@ -27,6 +27,9 @@ def _form(pkg, B, E, k, r3, r2, backward, dtype=torch.bfloat16):
     (2, 1, 256, 1024, 16384, 0, 1, 1), (2, 1, 128, 512, 16384, 0, 1, 1),
     (3, 2, 256, 1024, 16384, 0, 1, 1), (3, 2, 128, 512, 32768, 0, 1, 1),
     (4, 2, 128, 512, 32768, 0, 1, 1), (2, 1, 256, 2048, 65536, 0, 1, 1),
+    (2, 1, 128, 2048, 4572, 0, 1, 1), (2, 1, 256, 512, 21516, 0, 1, 1),
+    (3, 1, 128, 1024, 16384, 0, 1, 1), (3, 1, 128, 2048, 65536, 0, 1, 1),
+    (3, 1, 128, 2048, 50000, 1, 1, 1),
     (4, 2, 256, 1024, 8192, 1, 1, 1), (4, 1, 256, 1024, 32768, 1, 1, 1),
     (8, 2, 256, 1024, 16384, 1, 1, 1), (8, 2, 128, 512, 32768, 1, 1, 1),
 ])
