@@ -522,7 +522,8 @@ struct LatentDg {
 // DMA (dout's rows gathered); an MFMA fragment (8 entries of one column a lane) is two
 // transposed 64-bit reads. Within a K tile LDS row 4 (4 w + j) + s holds entry
 // 16 w + 4 s + j (the same for both operands), so that a lane's DMA rows are four
-// consecutive entries. Past the chunk's end xs is a row of zeros (dout's last row again).
+// consecutive entries. Past the chunk's end both are a row of zeros: dout's last row again would
+// give NaN where that row is not finite.
 __global__ __launch_bounds__(256, 2) void k_latent_dge(LatentDg q) {
   constexpr int kStage = 2 * 64 * 16;   // u32x4 slots: 64 rows x 16 chunks, twice
   __shared__ u32x4 smem[2 * kStage];
@@ -540,7 +541,8 @@ __global__ __launch_bounds__(256, 2) void k_latent_dge(LatentDg q) {
   const int64_t a_row = (int64_t)q.r3 * 2, b_row = (int64_t)q.r2 * 2;
   const char* abase = q.xs + d.x * a_row + tm * 256 + chunk * 16;
   const char* bbase = q.dout + tn * 256 + chunk * 16;
-  const int64_t zoff = q.zero + chunk * 16 - abase;   // entries past the end: a zero row of xs
+  // entries past the end: a zero row of either
+  const int64_t za = q.zero + chunk * 16 - abase, zb = q.zero + chunk * 16 - bbase;
   const int k0 = wave * 16 + sub * 4;   // this lane's first entry of a K tile
   const int nkt = (d.y + 63) / 64;
   int tok[4];
@@ -557,10 +559,11 @@ __global__ __launch_bounds__(256, 2) void k_latent_dge(LatentDg q) {
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
       const int k = kt * 64 + k0 + j;
-      const int64_t oa = k < d.y ? k * a_row : zoff;
+      const bool in = k < d.y;
+      const int64_t oa = in ? k * a_row : za, ob = in ? tok[j] * b_row : zb;
       __builtin_amdgcn_global_load_lds((gbl_cvptr)(abase + oa),
                                        (lds_vptr)(size_t)(s + (wave * 4 + j) * 1024), 16, 0, 0);
-      __builtin_amdgcn_global_load_lds((gbl_cvptr)(bbase + tok[j] * b_row),
+      __builtin_amdgcn_global_load_lds((gbl_cvptr)(bbase + ob),
                                        (lds_vptr)(size_t)(s + 16384 + (wave * 4 + j) * 1024), 16, 0,
                                        0);
     }

@@ -99,6 +99,25 @@ def test_grouped_is_deterministic(pkg, dev):
         assert torch.equal(a[n], b[n]), n
 
 
+@pytest.mark.parametrize("E,k,B", [(8, 6, 1), (8, 2, 63), (4, 2, 700), (16, 1, 300)])
+def test_infinite_dout_stays_infinite(pkg, dev, E, k, B):
+    """A column of dout that is infinite: positive x and p make dG infinite there for the experts
+    that were selected, and nothing NaN (the rows that fill a chunk's last K tile add zeros)."""
+    x, G, idx, p, dout = _inputs(B, E, k, 128, 256, 3, True)
+    x = x.abs() + 0.125
+    dout[:, 5] = float("inf")
+    f = pkg._lib
+    assert f.lib().tmoe_latent_form(B, E, k, 128, 256, f.TMOE_BF16, 1) & f.TMOE_LATENT_DG
+    Gs = G.to(dev).requires_grad_(True)
+    pkg.FusedLatentMoE.apply(x.to(dev), Gs, idx.to(dev), p.to(dev)).backward(dout.to(dev))
+    dG = Gs.grad.float().cpu()
+    used = torch.bincount(idx.flatten(), minlength=E) > 0
+    assert not torch.isnan(dG).any()
+    assert torch.isposinf(dG[used][:, :, 5]).all() and bool((dG[~used] == 0).all())
+    rest = torch.cat((dG[:, :, :5], dG[:, :, 6:]), 2)
+    assert torch.isfinite(rest).all()
+
+
 @pytest.mark.parametrize("E,k,r3,r2,counts", [
     (5, 4, 128, 128, (257, 257, 257, 257, 260)),        # every expert a full chunk and a rest
     (8, 2, 128, 128, (1, 1, 1, 1, 1, 1, 1, 1)),         # rests only
