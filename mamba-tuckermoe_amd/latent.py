@@ -83,7 +83,8 @@ class FusedLatentMoE(torch.autograd.Function):
         dt = _lib.dtype_code(x.dtype) | (_lib.TMOE_LATENT_P_F32 if p_f32 else 0)
         L = _lib.lib()
         dx = torch.empty_like(x)
-        dG = torch.empty_like(G)
+        # no token: no kernel runs, and nothing adds to dG
+        dG = torch.empty_like(G) if B else torch.zeros_like(G)
         dp = torch.empty(B, k, dtype=p.dtype, device=x.device)
         nws = L.tmoe_latent_workspace_bytes(B, E, r3, r2, dt, 1)
         ws = _ws(nws, x.device)

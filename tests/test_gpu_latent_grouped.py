@@ -118,6 +118,17 @@ def test_infinite_dout_stays_infinite(pkg, dev, E, k, B):
     assert torch.isfinite(rest).all()
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_no_tokens(pkg, dev, dtype):
+    x, idx, p = torch.zeros(0, 128), torch.zeros(0, 2, dtype=torch.int64), torch.zeros(0, 2)
+    torch.full((1 << 20,), 7.0, device=dev)            # memory that the gradient may be given
+    xs, Gs, ps = (t.to(dev, dtype).requires_grad_(True) for t in (x, torch.randn(8, 128, 256), p))
+    out = pkg.FusedLatentMoE.apply(xs, Gs, idx.to(dev), ps)
+    out.backward(torch.zeros_like(out))
+    assert out.shape == (0, 256) and xs.grad.shape == (0, 128) and ps.grad.shape == (0, 2)
+    assert bool((Gs.grad == 0).all())
+
+
 @pytest.mark.parametrize("E,k,r3,r2,counts", [
     (5, 4, 128, 128, (257, 257, 257, 257, 260)),        # every expert a full chunk and a rest
     (8, 2, 128, 128, (1, 1, 1, 1, 1, 1, 1, 1)),         # rests only
